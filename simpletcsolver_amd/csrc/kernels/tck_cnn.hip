@@ -10,8 +10,8 @@
  * Activations are channels-last BF16 rows act[v][C], v = x + NX (y + NY (z + NZ b)) for
  * sample b of a batch.  The convolution is an implicit GEMM on the matrix cores
  * (v_mfma_f32_16x16x32_bf16, FP32 accumulation) over activation tiles staged in LDS with
- * their halo; the weight gradient uses v_mfma_f32_16x16x16_bf16.  Weights are W[tap][co][ci]
- * BF16 with FP32 master copies; biases FP32.
+ * their halo; so is the weight gradient, on tiles transposed in LDS.  Weights are
+ * W[tap][co][ci] BF16 with FP32 master copies; biases FP32.
  *
  * Training: the backward data pass is the same convolution with the kernel flipped and its
  * channel roles exchanged (the adjoint of zero padding is zero padding, of periodic wrapping
@@ -22,7 +22,6 @@
 #include "tck_common.h"
 #include <stdint.h>
 
-typedef short cnn_s4 __attribute__((ext_vector_type(4)));
 typedef float cnn_f4 __attribute__((ext_vector_type(4)));
 
 /* FP32 -> BF16, round to nearest even (inputs here are finite) */
@@ -37,16 +36,6 @@ __device__ __forceinline__ float cnn_f32(unsigned short h){
 
 /* nb samples of nx x ny x nz cells, v = x + nx (y + ny (z + nz b)) */
 struct CnnGrid { int nx, ny, nz, nb; long long nv; };
-
-/* cell of a tap within sample b: x zero-padded (returns -1 outside), y and z periodic */
-__device__ __forceinline__ long long cnn_tap(const CnnGrid & G, int x, int y, int z, int b, int tap){
-  const int dx = tap % 3 - 1, dy = (tap / 3) % 3 - 1, dz = tap / 9 - 1;
-  const int xx = x + dx;
-  if(xx < 0 || xx >= G.nx) return -1;
-  int yy = y + dy; yy = yy < 0 ? yy + G.ny : (yy >= G.ny ? yy - G.ny : yy);
-  int zz = z + dz; zz = zz < 0 ? zz + G.nz : (zz >= G.nz ? zz - G.nz : zz);
-  return (long long)xx + (long long)G.nx * ((long long)yy + (long long)G.ny * ((long long)zz + (long long)G.nz * b));
-}
 
 /* ---------------------------------------------------------------------------------------
  * convolution: out[v][co] = bias[co] + sum_tap sum_ci W[tap][co][ci] in[v + tap][ci]
@@ -194,70 +183,174 @@ __global__ void __launch_bounds__(CNN_CONV_THREADS) tck_cnn_conv(const ConvArgs 
 /* ---------------------------------------------------------------------------------------
  * weight gradient on the matrix cores: for each tap a GEMM over cells,
  *   part[blk][tap][co][ci] = sum over the block's cells v of g[v][co] * in[v + tap][ci]
- * (FP32), then a fixed-order sum over blocks.  Block (blk, tap): 4 waves, each taking
- * 16-cell groups of the block's range in turn; lane l holds A = g^T row co = l % 16 over
- * cells 4 (l / 16) .. +3 of the group, B = the shifted inputs, column ci = l % 16 over the
- * same cells; the waves' accumulators are summed in LDS in wave order.
+ * (FP32), then a fixed-order sum over blocks.
+ *
+ * K of the product is the cells, while activations are channels-last, so a block transposes
+ * a tile of 16 x 4 x 4 cells into LDS rows of one channel along x: g without a halo, the inputs
+ * with a one-cell halo (periodic images in y and z, zeros past the walls; cells outside the
+ * grid have g = 0).  A lane then reads its eight K entries (consecutive x of one channel) as one
+ * 16-byte piece; the taps dx = -1 and +1 are the same piece shifted by one element, formed from
+ * its neighbour words in registers, so one read of the inputs serves the three taps of a
+ * (dy, dz) pair.  One wave per (dy, dz), nine per block, each holding the accumulators of its
+ * three taps; a block loops over a contiguous run of tiles with the next tile's loads in
+ * flight during the products.  An input row of a channel is 16 cells, the cell past them and,
+ * at the end of the row's 24 slots, the cell before the next row's; the channel pitches
+ * are 4 and 52 mod 64 words, so that the 16 lanes of a K group read distinct banks.
+ *
+ * Measured on a batch of 4 of 32 x 64 x 64 cells (29 GFLOP for 32 -> 32 channels): 50 us for
+ * 32 -> 32 (580 TFLOP/s), 39 us for 32 -> 16 and 30 us for 16 -> 32; gathering every tap's
+ * operands from memory as 2-byte loads took 675, 745 and 741 us.
  * ------------------------------------------------------------------------------------- */
 struct WgradArgs {
   CnnGrid G;
   const unsigned short * in;   /* [nv][CI] bf16 */
   const unsigned short * g;    /* [nv][CO] bf16 */
-  long long cells_per_block;   /* multiple of 64 */
   float * part;                /* [nblk][27][CO][CI] */
 };
 
-template <int CI, int CO>
-__global__ void __launch_bounds__(256) tck_cnn_wgrad(const WgradArgs A){
-  constexpr int NT = CO / 16, NS = CI / 16;
-  __shared__ float red[4][CO * CI];
-  const int lane = threadIdx.x % TCK_WAVE, wv = threadIdx.x / TCK_WAVE;
-  const int tap = blockIdx.y;
-  const long long v0 = (long long)blockIdx.x * A.cells_per_block;
-  const long long v1 = min(v0 + A.cells_per_block, A.G.nv);
-  cnn_f4 acc[NT][NS];
+#define CNN_WG_THREADS 576                    /* nine waves */
+#define CNN_WG_ROWS 36                        /* halo'd rows of a tile: 6 in y, 6 in z */
+#define CNN_WG_PITCH (8 + 24 * CNN_WG_ROWS)   /* elements per channel of the input tile */
+#define CNN_WG_GPITCH (256 + 8)               /* elements per channel of the gradient tile */
+#define CNN_WG_PAIRS (10 * CNN_WG_ROWS)       /* x pairs of the input tile */
+
+__host__ __device__ constexpr int cnn_wgrad_lds(int ci, int co){
+  return 2 * (ci * CNN_WG_PITCH + co * CNN_WG_GPITCH);
+}
+
+/* the same channel of two neighbouring cells, as one word */
+__device__ __forceinline__ uint32_t cnn_pair(uint32_t a, uint32_t b, int hi){
+  return hi ? (a >> 16) | (b & 0xffff0000u) : (a & 0xffffu) | (b << 16);
+}
+
+/* a and b: eight channels of two neighbouring cells -> the word at slot `at` of each of the
+ * eight channel rows */
+__device__ __forceinline__ void cnn_put_pair(uint32_t * at, int pitch_words, uint4 a, uint4 b){
+  const uint32_t aw[4] = {a.x, a.y, a.z, a.w}, bw[4] = {b.x, b.y, b.z, b.w};
   #pragma unroll
-  for(int t = 0; t < NT; t++)
-    #pragma unroll
-    for(int u = 0; u < NS; u++) acc[t][u] = cnn_f4{0.f, 0.f, 0.f, 0.f};
-  const int kq = 4 * (lane / 16), col = lane % 16;
-  for(long long c = v0 + 16 * wv; c < v1; c += 64){
-    cnn_s4 a[NT], b[NS];
-    #pragma unroll
-    for(int t = 0; t < NT; t++) a[t] = cnn_s4{0, 0, 0, 0};
-    #pragma unroll
-    for(int u = 0; u < NS; u++) b[u] = cnn_s4{0, 0, 0, 0};
-    #pragma unroll
-    for(int q = 0; q < 4; q++){
-      const long long v = c + kq + q;
-      if(v >= v1) break;
-      const int x = (int)(v % A.G.nx);
-      const long long r = v / A.G.nx;
-      const int y = (int)(r % A.G.ny);
-      const int z = (int)((r / A.G.ny) % A.G.nz);
-      const int bb = (int)(r / ((long long)A.G.ny * A.G.nz));
-      const long long src = cnn_tap(A.G, x, y, z, bb, tap);
-      if(src < 0) continue;
-      #pragma unroll
-      for(int t = 0; t < NT; t++) a[t][q] = (short)A.g[v * CO + 16 * t + col];
-      #pragma unroll
-      for(int u = 0; u < NS; u++) b[u][q] = (short)A.in[src * CI + 16 * u + col];
-    }
+  for(int q = 0; q < 8; q++) at[q * pitch_words] = cnn_pair(aw[q >> 1], bw[q >> 1], q & 1);
+}
+
+template <int CI, int CO>
+__global__ void __launch_bounds__(CNN_WG_THREADS) tck_cnn_wgrad(const WgradArgs A){
+  constexpr int NT = CO / 16, NS = CI / 16;
+  constexpr int NI = (CNN_WG_PAIRS * (CI / 8) + CNN_WG_THREADS - 1) / CNN_WG_THREADS;   /* input pieces per thread */
+  constexpr int NG = (128 * (CO / 8) + CNN_WG_THREADS - 1) / CNN_WG_THREADS;
+  extern __shared__ __align__(16) unsigned char cnn_smem[];
+  unsigned short * il = (unsigned short *)cnn_smem;     /* [CI][CNN_WG_PITCH] */
+  unsigned short * gl = il + CI * CNN_WG_PITCH;         /* [CO][CNN_WG_GPITCH] */
+  const CnnGrid & G = A.G;
+  const int lane = threadIdx.x % TCK_WAVE, wv = threadIdx.x / TCK_WAVE;
+  const int dy = wv % 3, dz = wv / 3;                   /* halo offsets 0..2 */
+  const int kg = lane / 16, cl = lane % 16;
+  const int ntx = (G.nx + 15) / 16, nty = (G.ny + 3) / 4, ntz = (G.nz + 3) / 4;
+  const int ntiles = ntx * nty * ntz * G.nb;
+  const int per = (ntiles + (int)gridDim.x - 1) / (int)gridDim.x;
+  const int t0 = blockIdx.x * per, t1 = min(t0 + per, ntiles);
+  cnn_f4 acc[3][NT][NS];
+  #pragma unroll
+  for(int d = 0; d < 3; d++)
     #pragma unroll
     for(int t = 0; t < NT; t++)
       #pragma unroll
-      for(int u = 0; u < NS; u++) acc[t][u] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a[t], b[u], acc[t][u], 0, 0, 0);
-  }
-  /* accumulator [t][u][q]: co = 16 t + kq + q, ci = 16 u + col */
-  #pragma unroll
-  for(int t = 0; t < NT; t++)
+      for(int u = 0; u < NS; u++) acc[d][t][u] = cnn_f4{0.f, 0.f, 0.f, 0.f};
+  const uint4 zero = {0u, 0u, 0u, 0u};
+  uint4 ia[NI], ib[NI], ga[NG], gb[NG];
+  /* a tile's pieces into registers: pairs of neighbouring cells, eight channels each */
+  auto fetch = [&](int tile){
+    const int tx = tile % ntx;
+    int r = tile / ntx;
+    const int ty = r % nty; r /= nty;
+    const int tz = r % ntz, b = r / ntz;
+    const int x0 = 16 * tx, y0 = 4 * ty, z0 = 4 * tz;
     #pragma unroll
-    for(int u = 0; u < NS; u++)
+    for(int q = 0; q < NI; q++){
+      const int e = threadIdx.x + q * CNN_WG_THREADS;
+      const int c = e % (CI / 8), pr = e / (CI / 8);
+      const int p = pr % 10, row = pr / 10;
+      ia[q] = zero; ib[q] = zero;
+      if(row < CNN_WG_ROWS){
+        const int y = cnn_wrap(y0 + row % 6 - 1, G.ny), z = cnn_wrap(z0 + row / 6 - 1, G.nz);
+        const int xa = x0 + 2 * p - 2;                  /* the pair's cells: xa, xa + 1 */
+        const unsigned short * src = A.in + (long long)G.nx * ((long long)y + (long long)G.ny * ((long long)z + (long long)G.nz * b)) * CI + 8 * c;
+        if(p > 0 && xa < G.nx) ia[q] = *(const uint4 *)(src + (long long)xa * CI);
+        if(p < 9 && xa + 1 >= 0 && xa + 1 < G.nx) ib[q] = *(const uint4 *)(src + (long long)(xa + 1) * CI);
+      }
+    }
+    #pragma unroll
+    for(int q = 0; q < NG; q++){
+      const int e = threadIdx.x + q * CNN_WG_THREADS;
+      const int c = e % (CO / 8), pr = e / (CO / 8);
+      const int x = x0 + 2 * (pr % 8), y = y0 + (pr / 8) % 4, z = z0 + pr / 32;
+      ga[q] = zero; gb[q] = zero;
+      if(pr < 128 && y < G.ny && z < G.nz){
+        const unsigned short * src = A.g + ((long long)x + (long long)G.nx * ((long long)y + (long long)G.ny * ((long long)z + (long long)G.nz * b))) * CO + 8 * c;
+        if(x < G.nx) ga[q] = *(const uint4 *)src;
+        if(x + 1 < G.nx) gb[q] = *(const uint4 *)(src + CO);
+      }
+    }
+  };
+  if(t0 < t1) fetch(t0);
+  for(int tile = t0; tile < t1; tile++){
+    __syncthreads();                                    /* the previous tile's reads are done */
+    #pragma unroll
+    for(int q = 0; q < NI; q++){
+      const int e = threadIdx.x + q * CNN_WG_THREADS;
+      const int c = e % (CI / 8), pr = e / (CI / 8);
+      const int p = pr % 10, row = pr / 10;
+      if(row < CNN_WG_ROWS)
+        cnn_put_pair((uint32_t *)il + (8 * c * CNN_WG_PITCH + 8 + 24 * row + 2 * p - 2) / 2, CNN_WG_PITCH / 2, ia[q], ib[q]);
+    }
+    #pragma unroll
+    for(int q = 0; q < NG; q++){
+      const int e = threadIdx.x + q * CNN_WG_THREADS;
+      const int c = e % (CO / 8), pr = e / (CO / 8);
+      if(pr < 128) cnn_put_pair((uint32_t *)gl + (8 * c * CNN_WG_GPITCH + 2 * pr) / 2, CNN_WG_GPITCH / 2, ga[q], gb[q]);
+    }
+    __syncthreads();
+    if(tile + 1 < t1) fetch(tile + 1);
+    /* 32 cells (two rows) per product: K entries 8 kg .. +7 are cells 8 (kg % 2) .. +7 of row
+     * kg / 2 of the two */
+    #pragma unroll 2
+    for(int s = 0; s < 8; s++){
+      const int ry = (2 * s + (kg >> 1)) % 4, rz = (2 * s) / 4;
+      const int at = 8 + 24 * (ry + dy + 6 * (rz + dz)) + 8 * (kg & 1);
+      cnn_b8 av[NT];
       #pragma unroll
-      for(int q = 0; q < 4; q++) red[wv][(16 * t + kq + q) * CI + 16 * u + col] = acc[t][u][q];
-  __syncthreads();
-  float * out = A.part + ((long long)blockIdx.x * 27 + tap) * (CO * CI);
-  for(int e = threadIdx.x; e < CO * CI; e += 256) out[e] = ((red[0][e] + red[1][e]) + red[2][e]) + red[3][e];
+      for(int t = 0; t < NT; t++) av[t] = *(const cnn_b8 *)(gl + (16 * t + cl) * CNN_WG_GPITCH + 32 * s + 8 * kg);
+      #pragma unroll
+      for(int u = 0; u < NS; u++){
+        const unsigned short * row = il + (16 * u + cl) * CNN_WG_PITCH + at;
+        const uint4 w = *(const uint4 *)row;
+        const uint32_t before = *(const uint32_t *)(row - 2), after = *(const uint32_t *)(row + 8);
+        uint4 m, n;                                     /* the cells one to the left and one to the right */
+        m.x = __builtin_amdgcn_alignbit(w.x, before, 16);
+        m.y = __builtin_amdgcn_alignbit(w.y, w.x, 16);
+        m.z = __builtin_amdgcn_alignbit(w.z, w.y, 16);
+        m.w = __builtin_amdgcn_alignbit(w.w, w.z, 16);
+        n.x = m.y; n.y = m.z; n.z = m.w;
+        n.w = __builtin_amdgcn_alignbit(after, w.w, 16);
+        const cnn_b8 bl = __builtin_bit_cast(cnn_b8, m), b0 = __builtin_bit_cast(cnn_b8, w), br = __builtin_bit_cast(cnn_b8, n);
+        #pragma unroll
+        for(int t = 0; t < NT; t++){
+          acc[0][t][u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[t], bl, acc[0][t][u], 0, 0, 0);
+          acc[1][t][u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[t], b0, acc[1][t][u], 0, 0, 0);
+          acc[2][t][u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[t], br, acc[2][t][u], 0, 0, 0);
+        }
+      }
+    }
+  }
+  /* accumulator [d][t][u][q]: tap d + 3 dy + 9 dz, co = 16 t + 4 kg + q, ci = 16 u + cl */
+  #pragma unroll
+  for(int d = 0; d < 3; d++){
+    float * out = A.part + ((long long)blockIdx.x * 27 + d + 3 * dy + 9 * dz) * (CO * CI);
+    #pragma unroll
+    for(int t = 0; t < NT; t++)
+      #pragma unroll
+      for(int u = 0; u < NS; u++)
+        #pragma unroll
+        for(int q = 0; q < 4; q++) out[(16 * t + 4 * kg + q) * CI + 16 * u + cl] = acc[d][t][u][q];
+  }
 }
 
 /* out[e] = sum_b part[b][e] (b in order) */
@@ -419,6 +512,19 @@ static int cnn_conv_launch(const ConvArgs & A, dim3 grd, int lds, hipStream_t st
   return 0;
 }
 
+template <int CI, int CO>
+static int cnn_wgrad_launch(const WgradArgs & A, int nblk, hipStream_t stream){
+  static int ready = 0;
+  constexpr int lds = cnn_wgrad_lds(CI, CO);
+  if(!ready){
+    const hipError_t e = hipFuncSetAttribute((const void *)tck_cnn_wgrad<CI, CO>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    if(e != hipSuccess) return (int)e;
+    ready = 1;
+  }
+  hipLaunchKernelGGL((tck_cnn_wgrad<CI, CO>), dim3((unsigned)nblk), dim3(CNN_WG_THREADS), lds, stream, A);
+  return 0;
+}
+
 static int g_cnn_ncu = 0;
 
 static int cnn_ncu(void){
@@ -463,12 +569,15 @@ int tck_cnn_launch_wgrad(int nx, int ny, int nz, int nb, const unsigned short * 
   WgradArgs A;
   A.G.nx = nx; A.G.ny = ny; A.G.nz = nz; A.G.nb = nb; A.G.nv = (long long)nx * ny * nz * nb;
   A.in = in; A.g = g; A.part = part;
-  A.cells_per_block = ((A.G.nv + nblk - 1) / nblk + 63) / 64 * 64;
-  const dim3 grd((unsigned)nblk, 27);
-  if(ci_n == 16 && co_n == 32) hipLaunchKernelGGL((tck_cnn_wgrad<16, 32>), grd, dim3(256), 0, stream, A);
-  else if(ci_n == 32 && co_n == 32) hipLaunchKernelGGL((tck_cnn_wgrad<32, 32>), grd, dim3(256), 0, stream, A);
-  else if(ci_n == 32 && co_n == 16) hipLaunchKernelGGL((tck_cnn_wgrad<32, 16>), grd, dim3(256), 0, stream, A);
+  const long long ntiles = (long long)((nx + 15) / 16) * ((ny + 3) / 4) * ((nz + 3) / 4) * nb;
+  if(ntiles > 0x7fffffffLL) return (int)hipErrorInvalidValue;
+  if(nblk > ntiles) nblk = (int)ntiles;
+  int rc;
+  if(ci_n == 16 && co_n == 32) rc = cnn_wgrad_launch<16, 32>(A, nblk, stream);
+  else if(ci_n == 32 && co_n == 32) rc = cnn_wgrad_launch<32, 32>(A, nblk, stream);
+  else if(ci_n == 32 && co_n == 16) rc = cnn_wgrad_launch<32, 16>(A, nblk, stream);
   else return (int)hipErrorInvalidValue;
+  if(rc) return rc;
   TCK_CHECK_LAUNCH();
   const int n = 27 * co_n * ci_n;
   hipLaunchKernelGGL(tck_cnn_reduce, dim3((n + 255) / 256), dim3(256), 0, stream, (const float *)part, nblk, n, out);
