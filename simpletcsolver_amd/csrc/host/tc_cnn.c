@@ -17,22 +17,24 @@
 #include "tc_internal.h"
 
 /* tck_cnn.hip */
+int tck_cnn_bgrad_blocks(int nx, int ny, int nz, int nb);
 int tck_cnn_launch_conv(int nx, int ny, int nz, int nb, const unsigned short * in, int ci,
-    const unsigned short * w, int co, const float * bias, int co_store, int relu,
-    unsigned short * out_bf, float * out_f, hipStream_t stream);
-int tck_cnn_launch_wgrad(int nx, int ny, int nz, int nb, const unsigned short * in, int ci_n,
-    const unsigned short * g, int co_n, float * part, int nblk, float * out, hipStream_t stream);
-int tck_cnn_launch_bgrad(long long nv, const float * g, int co_n, float * part, int nblk, float * out,
+    const unsigned short * w, int co, const float * bias, int co_store,
+    unsigned short * out_bf, float * out_f, const unsigned short * act, float * bpart, int * nblk,
     hipStream_t stream);
-int tck_cnn_launch_mse(const float * pred, const float * target, long long n, float scale,
-    float * grad, float * part, int nblk, hipStream_t stream);
-int tck_cnn_launch_relu_bwd(const float * gpost, const unsigned short * act, long long n,
-    unsigned short * gpre, float * gf, hipStream_t stream);
+int tck_cnn_launch_wgrad(int nx, int ny, int nz, int nb, const unsigned short * in, int ci_n,
+    const unsigned short * g, int co_n, float * part, int * nblk_io, hipStream_t stream);
+int tck_cnn_launch_reduce(int nseg, const float * const * part, const int * nblk, const int * n,
+    float * const * out, hipStream_t stream);
+int tck_cnn_launch_mse(const float * pred, const float * target, long long nv, float scale,
+    unsigned short * g, float * bpart, float * lpart, int nblk, hipStream_t stream);
 int tck_cnn_launch_to_bf16(const float * x, long long n, unsigned short * y, hipStream_t stream);
 int tck_cnn_launch_flip(const unsigned short * w, int co_n, int ci_n, int ci_p, int co_p,
     unsigned short * wt, hipStream_t stream);
-int tck_cnn_launch_adam(float * w, float * m, float * v, const float * g, int n, float lr,
-    float b1, float b2, float eps, float c1, float c2, unsigned short * wbf, hipStream_t stream);
+int tck_cnn_launch_adam(int nseg, float * const * w, float * const * m, float * const * v,
+    float * const * g, unsigned short * const * wbf, unsigned short * const * wt, const int * n,
+    const int * co, const int * ci, float lr, float b1, float b2, float eps, float c1, float c2,
+    hipStream_t stream);
 int tck_cnn_launch_gather(const tc_geom_t * g, const double * ux, const double * uy,
     const double * uz, const double * t, const double * xc, const float mean[5],
     const float inv_std[5], unsigned short * out, hipStream_t stream);
@@ -41,8 +43,9 @@ int tck_cnn_launch_scatter(const tc_geom_t * g, const float * pred, const float 
 
 #define CNN_C0 16      /* padded input channels */
 #define CNN_C 32       /* hidden channels */
-#define CNN_CO 16      /* padded output channels (4 used) */
-#define CNN_NBLK 256   /* blocks of the weight-gradient reductions */
+#define CNN_CO 16      /* padded output channels of the last layer's kernel */
+#define CNN_OUT 4      /* output channels stored */
+#define CNN_NBLK 256   /* most blocks of the weight gradients, and blocks of the loss */
 
 /* layer l: input channels ci, output channels co */
 static const int g_ci[3] = {CNN_C0, CNN_C, CNN_C};
@@ -65,16 +68,13 @@ struct tc_cnn_s {
   /* activations of one batch */
   unsigned short * x0;          /* [nv][16] */
   unsigned short * a1; unsigned short * a2;   /* [nv][32] */
-  float * out;                  /* [nv][16] */
-  float * target;               /* [nv][16] */
-  float * gout;                 /* d loss / d out */
-  unsigned short * g3;          /* BF16 of gout */
-  float * d2; float * d1;       /* d loss / d a2, d a1 (FP32) */
-  unsigned short * g2; unsigned short * g1;   /* through the ReLUs, BF16 */
-  float * g2f; float * g1f;
-  float * part;                 /* reduction scratch */
+  float * out;                  /* [nv][4] */
+  float * target;               /* [nv][4] */
+  unsigned short * g3;          /* d loss / d out, BF16, [nv][16] */
+  unsigned short * g2; unsigned short * g1;   /* d loss / d a2, d a1 through the ReLUs, BF16 */
+  float * pw[3]; float * pb[3]; /* per-block partial sums of the weight and bias gradients */
+  float * lpart;                /* and of the loss, [CNN_NBLK] */
   unsigned short * h_x;         /* host staging */
-  float * h_y;
 };
 
 static long long wsize(int l){ return 27LL * g_co[l] * g_ci[l]; }
@@ -107,15 +107,14 @@ int tc_cnn_destroy(tc_cnn_t * c){
   }
   if(c->stream) hipStreamSynchronize(c->stream);
   for(int l = 0; l < 3; l++){
-    void * p[] = {c->w[l], c->b[l], c->wbf[l], c->mw[l], c->vw[l], c->mb[l], c->vb[l], c->gw[l], c->gb[l], c->wt[l]};
+    void * p[] = {c->w[l], c->b[l], c->wbf[l], c->mw[l], c->vw[l], c->mb[l], c->vb[l], c->gw[l], c->gb[l], c->wt[l],
+      c->pw[l], c->pb[l]};
     for(size_t q = 0; q < sizeof(p) / sizeof(p[0]); q++) if(p[q]) hipFree(p[q]);
   }
-  void * a[] = {c->x0, c->a1, c->a2, c->out, c->target, c->gout, c->g3, c->d2, c->d1, c->g2, c->g1,
-    c->g2f, c->g1f, c->part};
+  void * a[] = {c->x0, c->a1, c->a2, c->out, c->target, c->g3, c->g2, c->g1, c->lpart};
   for(size_t q = 0; q < sizeof(a) / sizeof(a[0]); q++) if(a[q]) hipFree(a[q]);
   if(c->stream) hipStreamDestroy(c->stream);
   free(c->h_x);
-  free(c->h_y);
   free(c);
   return 0;
 }
@@ -153,16 +152,18 @@ int tc_cnn_create(int nx, int ny, int nz, int batch, unsigned long long seed, in
   if(!rc){
     rc |= cnn_alloc((void **)&c->x0, 2 * nv * CNN_C0);
     rc |= cnn_alloc((void **)&c->a1, 2 * nv * CNN_C) || cnn_alloc((void **)&c->a2, 2 * nv * CNN_C);
-    rc |= cnn_alloc((void **)&c->out, 4 * nv * CNN_CO) || cnn_alloc((void **)&c->target, 4 * nv * CNN_CO);
-    rc |= cnn_alloc((void **)&c->gout, 4 * nv * CNN_CO) || cnn_alloc((void **)&c->g3, 2 * nv * CNN_CO);
-    rc |= cnn_alloc((void **)&c->d2, 4 * nv * CNN_C) || cnn_alloc((void **)&c->d1, 4 * nv * CNN_C);
+    rc |= cnn_alloc((void **)&c->out, 4 * nv * CNN_OUT) || cnn_alloc((void **)&c->target, 4 * nv * CNN_OUT);
+    rc |= cnn_alloc((void **)&c->g3, 2 * nv * CNN_CO);
     rc |= cnn_alloc((void **)&c->g2, 2 * nv * CNN_C) || cnn_alloc((void **)&c->g1, 2 * nv * CNN_C);
-    rc |= cnn_alloc((void **)&c->g2f, 4 * nv * CNN_C) || cnn_alloc((void **)&c->g1f, 4 * nv * CNN_C);
-    rc |= cnn_alloc((void **)&c->part, 4 * (size_t)CNN_NBLK * 27 * CNN_C * CNN_C);
+    rc |= cnn_alloc((void **)&c->lpart, 4 * (size_t)CNN_NBLK);
+    for(int l = 0; l < 3; l++){
+      const size_t nbl = l == 2 ? CNN_NBLK : (size_t)tck_cnn_bgrad_blocks(nx, ny, nz, batch);
+      rc |= cnn_alloc((void **)&c->pw[l], 4 * (size_t)CNN_NBLK * (size_t)wsize(l)) ||
+            cnn_alloc((void **)&c->pb[l], 4 * nbl * (size_t)g_co[l]);
+    }
   }
   c->h_x = calloc(nv * CNN_C0, 2);
-  c->h_y = calloc(nv * CNN_CO, 4);
-  if(!c->h_x || !c->h_y) rc = tc_fail("host allocation failed");
+  if(!c->h_x) rc = tc_fail("host allocation failed");
   /* initial weights */
   unsigned long long st = seed * 0x9E3779B97F4A7C15ULL + 12345;
   for(int l = 0; l < 3 && !rc; l++){
@@ -196,6 +197,7 @@ int tc_cnn_set_layer(tc_cnn_t * c, int l, const float * w, const float * b){
   if(w){
     HIPOK(hipMemcpyAsync(c->w[l], w, 4 * (size_t)nw, hipMemcpyHostToDevice, c->stream));
     KOK(tck_cnn_launch_to_bf16(c->w[l], nw, c->wbf[l], c->stream));
+    KOK(tck_cnn_launch_flip(c->wbf[l], g_co[l], g_ci[l], g_ci[l], g_co[l], c->wt[l], c->stream));
   }
   if(b) HIPOK(hipMemcpyAsync(c->b[l], b, 4 * (size_t)g_co[l], hipMemcpyHostToDevice, c->stream));
   HIPOK(hipStreamSynchronize(c->stream));
@@ -224,44 +226,42 @@ static int upload_x(tc_cnn_t * c, const float * x){
   return 0;
 }
 
-static int forward(tc_cnn_t * c, const unsigned short * x0){
-  KOK(tck_cnn_launch_conv(c->nx, c->ny, c->nz, c->nb, x0, CNN_C0, c->wbf[0], CNN_C, c->b[0], CNN_C, 1, c->a1, NULL, c->stream));
-  KOK(tck_cnn_launch_conv(c->nx, c->ny, c->nz, c->nb, c->a1, CNN_C, c->wbf[1], CNN_C, c->b[1], CNN_C, 1, c->a2, NULL, c->stream));
-  KOK(tck_cnn_launch_conv(c->nx, c->ny, c->nz, c->nb, c->a2, CNN_C, c->wbf[2], CNN_CO, c->b[2], CNN_CO, 0, NULL, c->out, c->stream));
+static int forward(tc_cnn_t * c, int nb, hipStream_t stream){
+  KOK(tck_cnn_launch_conv(c->nx, c->ny, c->nz, nb, c->x0, CNN_C0, c->wbf[0], CNN_C, c->b[0], CNN_C, c->a1, NULL, NULL, NULL, NULL, stream));
+  KOK(tck_cnn_launch_conv(c->nx, c->ny, c->nz, nb, c->a1, CNN_C, c->wbf[1], CNN_C, c->b[1], CNN_C, c->a2, NULL, NULL, NULL, NULL, stream));
+  KOK(tck_cnn_launch_conv(c->nx, c->ny, c->nz, nb, c->a2, CNN_C, c->wbf[2], CNN_CO, c->b[2], CNN_OUT, NULL, c->out, NULL, NULL, NULL, stream));
   return 0;
 }
 
-/* loss and all gradients for the uploaded batch; targets [nb][nz][ny][nx][4] */
+/* loss and all gradients for the uploaded batch; targets [nb][nz][ny][nx][4].  The gradient
+ * with respect to a layer's output is rounded to BF16 once, as the operand of the layer below's
+ * products; its bias gradient sums the FP32 values. */
 static int backward(tc_cnn_t * c, const float * y, double * loss){
   const long long nv = c->nv;
-  for(long long v = 0; v < nv; v++){
-    for(int q = 0; q < CNN_CO; q++) c->h_y[v * CNN_CO + q] = q < 4 ? y[v * 4 + q] : 0.f;
+  HIPOK(hipMemcpyAsync(c->target, y, 4 * (size_t)nv * CNN_OUT, hipMemcpyHostToDevice, c->stream));
+  KOK(tck_cnn_launch_mse(c->out, c->target, nv, (float)(1.0 / (double)(nv * 4)), c->g3, c->pb[2], c->lpart, CNN_NBLK, c->stream));
+  const unsigned short * in[3] = {c->x0, c->a1, c->a2};
+  const unsigned short * g[3] = {c->g1, c->g2, c->g3};
+  unsigned short * gin[3] = {NULL, c->g1, c->g2};
+  const float * part[6];
+  float * out[6];
+  int nblk[6], n[6];
+  nblk[5] = CNN_NBLK;
+  for(int l = 2; l >= 0; l--){
+    part[l] = c->pw[l]; out[l] = c->gw[l]; n[l] = (int)wsize(l); nblk[l] = CNN_NBLK;
+    part[3 + l] = c->pb[l]; out[3 + l] = c->gb[l]; n[3 + l] = g_co[l];
+    KOK(tck_cnn_launch_wgrad(c->nx, c->ny, c->nz, c->nb, in[l], g_ci[l], g[l], g_co[l], c->pw[l], &nblk[l], c->stream));
+    if(l > 0)
+      KOK(tck_cnn_launch_conv(c->nx, c->ny, c->nz, c->nb, g[l], g_co[l], c->wt[l], CNN_C, NULL, CNN_C, gin[l], NULL,
+          in[l], c->pb[l - 1], &nblk[3 + l - 1], c->stream));
   }
-  HIPOK(hipMemcpyAsync(c->target, c->h_y, 4 * (size_t)nv * CNN_CO, hipMemcpyHostToDevice, c->stream));
-  const int nblk = 256;
-  KOK(tck_cnn_launch_mse(c->out, c->target, nv * CNN_CO, (float)(1.0 / (double)(nv * 4)), c->gout, c->part, nblk, c->stream));
-  float hp[256];
-  HIPOK(hipMemcpyAsync(hp, c->part, sizeof(hp), hipMemcpyDeviceToHost, c->stream));
-  /* layer 3 */
-  KOK(tck_cnn_launch_to_bf16(c->gout, nv * CNN_CO, c->g3, c->stream));
-  KOK(tck_cnn_launch_wgrad(c->nx, c->ny, c->nz, c->nb, c->a2, CNN_C, c->g3, CNN_CO, c->part, CNN_NBLK, c->gw[2], c->stream));
-  KOK(tck_cnn_launch_bgrad(nv, c->gout, CNN_CO, c->part, CNN_NBLK, c->gb[2], c->stream));
-  KOK(tck_cnn_launch_flip(c->wbf[2], CNN_CO, CNN_C, CNN_C, CNN_CO, c->wt[2], c->stream));
-  KOK(tck_cnn_launch_conv(c->nx, c->ny, c->nz, c->nb, c->g3, CNN_CO, c->wt[2], CNN_C, NULL, CNN_C, 0, NULL, c->d2, c->stream));
-  /* layer 2 */
-  KOK(tck_cnn_launch_relu_bwd(c->d2, c->a2, nv * CNN_C, c->g2, c->g2f, c->stream));
-  KOK(tck_cnn_launch_wgrad(c->nx, c->ny, c->nz, c->nb, c->a1, CNN_C, c->g2, CNN_C, c->part, CNN_NBLK, c->gw[1], c->stream));
-  KOK(tck_cnn_launch_bgrad(nv, c->g2f, CNN_C, c->part, CNN_NBLK, c->gb[1], c->stream));
-  KOK(tck_cnn_launch_flip(c->wbf[1], CNN_C, CNN_C, CNN_C, CNN_C, c->wt[1], c->stream));
-  KOK(tck_cnn_launch_conv(c->nx, c->ny, c->nz, c->nb, c->g2, CNN_C, c->wt[1], CNN_C, NULL, CNN_C, 0, NULL, c->d1, c->stream));
-  /* layer 1 */
-  KOK(tck_cnn_launch_relu_bwd(c->d1, c->a1, nv * CNN_C, c->g1, c->g1f, c->stream));
-  KOK(tck_cnn_launch_wgrad(c->nx, c->ny, c->nz, c->nb, c->x0, CNN_C0, c->g1, CNN_C, c->part, CNN_NBLK, c->gw[0], c->stream));
-  KOK(tck_cnn_launch_bgrad(nv, c->g1f, CNN_C, c->part, CNN_NBLK, c->gb[0], c->stream));
+  KOK(tck_cnn_launch_reduce(6, part, nblk, n, out, c->stream));
+  float hp[CNN_NBLK];
+  HIPOK(hipMemcpyAsync(hp, c->lpart, sizeof(hp), hipMemcpyDeviceToHost, c->stream));
   HIPOK(hipStreamSynchronize(c->stream));
   if(loss){
     double s = 0.;
-    for(int q = 0; q < nblk; q++) s += hp[q];
+    for(int q = 0; q < CNN_NBLK; q++) s += hp[q];
     *loss = s / (double)(nv * 4);
   }
   return 0;
@@ -269,17 +269,15 @@ static int backward(tc_cnn_t * c, const float * y, double * loss){
 
 int tc_cnn_predict(tc_cnn_t * c, const float * x, float * y){
   HIPOK(hipSetDevice(c->device));
-  if(upload_x(c, x) || forward(c, c->x0)) return 1;
-  float * h = c->h_y;
-  HIPOK(hipMemcpyAsync(h, c->out, 4 * (size_t)c->nv * CNN_CO, hipMemcpyDeviceToHost, c->stream));
+  if(upload_x(c, x) || forward(c, c->nb, c->stream)) return 1;
+  HIPOK(hipMemcpyAsync(y, c->out, 4 * (size_t)c->nv * CNN_OUT, hipMemcpyDeviceToHost, c->stream));
   HIPOK(hipStreamSynchronize(c->stream));
-  for(long long v = 0; v < c->nv; v++) for(int q = 0; q < 4; q++) y[v * 4 + q] = h[v * CNN_CO + q];
   return 0;
 }
 
 int tc_cnn_gradients(tc_cnn_t * c, const float * x, const float * y, double * loss){
   HIPOK(hipSetDevice(c->device));
-  if(upload_x(c, x) || forward(c, c->x0)) return 1;
+  if(upload_x(c, x) || forward(c, c->nb, c->stream)) return 1;
   return backward(c, y, loss);
 }
 
@@ -288,10 +286,16 @@ int tc_cnn_train_step(tc_cnn_t * c, const float * x, const float * y, float lr, 
   const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
   c->step += 1;
   const float c1 = (float)(1.0 - pow(b1, (double)c->step)), c2 = (float)(1.0 - pow(b2, (double)c->step));
+  float * w[6], * m[6], * v[6], * g[6];
+  unsigned short * wbf[6], * wt[6];
+  int n[6], co[6], ci[6];
   for(int l = 0; l < 3; l++){
-    KOK(tck_cnn_launch_adam(c->w[l], c->mw[l], c->vw[l], c->gw[l], (int)wsize(l), lr, b1, b2, eps, c1, c2, c->wbf[l], c->stream));
-    KOK(tck_cnn_launch_adam(c->b[l], c->mb[l], c->vb[l], c->gb[l], g_co[l], lr, b1, b2, eps, c1, c2, NULL, c->stream));
+    w[l] = c->w[l]; m[l] = c->mw[l]; v[l] = c->vw[l]; g[l] = c->gw[l]; wbf[l] = c->wbf[l]; wt[l] = c->wt[l];
+    w[3 + l] = c->b[l]; m[3 + l] = c->mb[l]; v[3 + l] = c->vb[l]; g[3 + l] = c->gb[l]; wbf[3 + l] = NULL; wt[3 + l] = NULL;
+    n[l] = (int)wsize(l); n[3 + l] = g_co[l];
+    co[l] = co[3 + l] = g_co[l]; ci[l] = ci[3 + l] = g_ci[l];
   }
+  KOK(tck_cnn_launch_adam(6, w, m, v, g, wbf, wt, n, co, ci, lr, b1, b2, eps, c1, c2, c->stream));
   HIPOK(hipStreamSynchronize(c->stream));
   return 0;
 }
@@ -341,9 +345,7 @@ int tc_closure_eval(tc_solver_t * s){
   if(!c) return 0;
   KOK(tck_cnn_launch_gather(&s->g, tc_field_ptr(s, 0), tc_field_ptr(s, 1), tc_field_ptr(s, 2),
       s->p.scalar ? tc_field_ptr(s, 3) : NULL, s->d_cnn_xc, s->cnn_mean, s->cnn_inv_std, c->x0, s->stream));
-  KOK(tck_cnn_launch_conv(c->nx, c->ny, c->nz, 1, c->x0, CNN_C0, c->wbf[0], CNN_C, c->b[0], CNN_C, 1, c->a1, NULL, s->stream));
-  KOK(tck_cnn_launch_conv(c->nx, c->ny, c->nz, 1, c->a1, CNN_C, c->wbf[1], CNN_C, c->b[1], CNN_C, 1, c->a2, NULL, s->stream));
-  KOK(tck_cnn_launch_conv(c->nx, c->ny, c->nz, 1, c->a2, CNN_C, c->wbf[2], CNN_CO, c->b[2], CNN_CO, 0, NULL, c->out, s->stream));
+  if(forward(c, 1, s->stream)) return 1;
   KOK(tck_cnn_launch_scatter(&s->g, c->out, s->cnn_scale, (float *)s->d_corr[0], (float *)s->d_corr[1],
       (float *)s->d_corr[2], s->p.scalar ? (float *)s->d_corr[3] : NULL, s->stream));
   return 0;

@@ -40,14 +40,14 @@ struct CnnGrid { int nx, ny, nz, nb; long long nv; };
 /* ---------------------------------------------------------------------------------------
  * convolution: out[v][co] = bias[co] + sum_tap sum_ci W[tap][co][ci] in[v + tap][ci]
  *   CI input channels (16 or 32), CO output channels (16 or 32) of which the first co_store
- *   are written; relu: out = max(0, .) stored BF16 (next layer's input), otherwise FP32.
+ *   are written, as the launch's mode says.
  *
- * Implicit GEMM on v_mfma_f32_16x16x32_bf16: A = 16 cells of an x row by 32 K entries, B = 32
- * K entries by 16 output channels.  K is the 32 input channels of one tap (CI = 32), or the
+ * Implicit GEMM on v_mfma_f32_16x16x32_bf16: A = 16 output channels by 32 K entries, B = 32 K
+ * entries by 16 cells of an x row.  K is the 32 input channels of one tap (CI = 32), or the
  * 16 input channels of two taps (CI = 16, the 27th tap paired with zeros).  Lane l holds the
  * eight K entries 8 (l / 16) .. +7 of A row l % 16 and of B column l % 16 (the same K order on
- * both sides, which is all the product needs); the accumulator holds rows (cells)
- * 4 (l / 16) .. +3 of column l % 16.
+ * both sides, which is all the product needs); the accumulator holds four consecutive
+ * channels 4 (l / 16) .. +3 of cell l % 16, which go out as one 8- or 16-byte store.
  *
  * A block stages the kernel once (rows of CI BF16 padded by 16 bytes, so that the 16 lanes
  * reading one K group hit distinct banks) and loops over tiles of 16 x CNN_TY x CNN_TZ cells
@@ -60,11 +60,18 @@ struct ConvArgs {
   const unsigned short * in;     /* [nv][CI] bf16 */
   const unsigned short * w;      /* [27][CO][CI] bf16 */
   const float * bias;            /* [CO] or null */
-  unsigned short * out_bf;       /* [nv][co_store] bf16 (relu) */
-  float * out_f;                 /* [nv][co_store] fp32 (no relu) */
-  int co_store;
-  int relu;
+  unsigned short * out_bf;       /* [nv][co_store] bf16 (CNN_RELU, CNN_RELU_BWD) */
+  float * out_f;                 /* [nv][co_store] fp32 (CNN_PLAIN) */
+  const unsigned short * act;    /* CNN_RELU_BWD: [nv][co_store] bf16, the layer's stored activations */
+  float * bpart;                 /* CNN_RELU_BWD: [blocks][CO], sums of the gradient over a block's cells */
+  int co_store;                  /* a multiple of 4 */
+  int mode;
 };
+
+/* what becomes of an output value: stored FP32; max(0, .) stored BF16; or, in the backward data
+ * pass, the gradient through the layer's ReLU (kept where its stored activation is positive),
+ * stored BF16 for the next products, with the FP32 values summed for the bias gradient */
+enum { CNN_PLAIN = 0, CNN_RELU = 1, CNN_RELU_BWD = 2 };
 
 #define CNN_CONV_THREADS 512
 #define CNN_TY 4
@@ -108,6 +115,9 @@ __global__ void __launch_bounds__(CNN_CONV_THREADS) tck_cnn_conv(const ConvArgs 
   /* CI = 16: K group kg reads tap 2 s + (kg >> 1), channels 8 (kg & 1) .. +7 */
   const int ktap = CI == 32 ? 0 : (kg >> 1);
   const int kbyte = CI == 32 ? 16 * kg : 16 * (kg & 1);
+  cnn_f4 bsum[NT];
+  #pragma unroll
+  for(int t = 0; t < NT; t++) bsum[t] = cnn_f4{0.f, 0.f, 0.f, 0.f};
   for(long long tile = blockIdx.x; tile < ntiles; tile += gridDim.x){
     const int tx = (int)(tile % ntx);
     long long r = tile / ntx;
@@ -152,31 +162,58 @@ __global__ void __launch_bounds__(CNN_CONV_THREADS) tck_cnn_conv(const ConvArgs 
         const int c = (cl + dx) + CNN_HX * ((ry + dy) + (CNN_TY + 2) * (rz + dz));
         const cnn_b8 av = *(const cnn_b8 *)(al + c * RS + kbyte);
         #pragma unroll
-        for(int t = 0; t < NT; t++) acc[q][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, bw[t], acc[q][t], 0, 0, 0);
+        for(int t = 0; t < NT; t++) acc[q][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bw[t], av, acc[q][t], 0, 0, 0);
       }
     }
-    /* accumulator: cells 4 kg .. +3 of the row, output channel 16 t + cl */
+    /* accumulator: channels 16 t + 4 kg .. +3 of cell x0 + cl of the row */
     #pragma unroll
     for(int q = 0; q < CNN_RPW; q++){
       const int row = wv * CNN_RPW + q;
-      const int y = y0 + row % CNN_TY, z = z0 + row / CNN_TY;
-      if(y >= G.ny || z >= G.nz) continue;
+      const int x = x0 + cl, y = y0 + row % CNN_TY, z = z0 + row / CNN_TY;
+      if(x >= G.nx || y >= G.ny || z >= G.nz) continue;
+      const long long v = (long long)x + (long long)G.nx * ((long long)y + (long long)G.ny * ((long long)z + (long long)G.nz * b));
       #pragma unroll
       for(int t = 0; t < NT; t++){
-        const int co = 16 * t + cl;
+        const int co = 16 * t + 4 * kg;
         if(co >= A.co_store) continue;
-        const float bv = A.bias ? A.bias[co] : 0.f;
-        #pragma unroll
-        for(int u = 0; u < 4; u++){
-          const int xc = x0 + 4 * kg + u;
-          if(xc >= G.nx) continue;
-          const long long v = (long long)xc + (long long)G.nx * ((long long)y + (long long)G.ny * ((long long)z + (long long)G.nz * b));
-          const float val = acc[q][t][u] + bv;
-          if(A.relu) A.out_bf[v * A.co_store + co] = cnn_bf16(val > 0.f ? val : 0.f);
-          else A.out_f[v * A.co_store + co] = val;
+        cnn_f4 val = acc[q][t];
+        if(A.bias) val += *(const cnn_f4 *)(A.bias + co);
+        if(A.mode == CNN_PLAIN){
+          *(cnn_f4 *)(A.out_f + v * A.co_store + co) = val;
+          continue;
         }
+        if(A.mode == CNN_RELU){
+          #pragma unroll
+          for(int u = 0; u < 4; u++) val[u] = val[u] > 0.f ? val[u] : 0.f;
+        }else{
+          const ushort4 a = *(const ushort4 *)(A.act + v * A.co_store + co);
+          val[0] = cnn_f32(a.x) > 0.f ? val[0] : 0.f;
+          val[1] = cnn_f32(a.y) > 0.f ? val[1] : 0.f;
+          val[2] = cnn_f32(a.z) > 0.f ? val[2] : 0.f;
+          val[3] = cnn_f32(a.w) > 0.f ? val[3] : 0.f;
+          bsum[t] += val;
+        }
+        *(ushort4 *)(A.out_bf + v * A.co_store + co) = make_ushort4(cnn_bf16(val[0]), cnn_bf16(val[1]), cnn_bf16(val[2]), cnn_bf16(val[3]));
       }
     }
+  }
+  if(A.mode != CNN_RELU_BWD) return;
+  /* the block's sums: over the 16 cells of a wave's lanes, then over the waves in order */
+  __syncthreads();
+  float * red = (float *)al;                      /* [waves][CO] */
+  #pragma unroll
+  for(int t = 0; t < NT; t++)
+    #pragma unroll
+    for(int u = 0; u < 4; u++){
+      float v = bsum[t][u];
+      for(int off = 8; off > 0; off >>= 1) v += __shfl_xor(v, off, TCK_WAVE);
+      if(cl == 0) red[wv * CO + 16 * t + 4 * kg + u] = v;
+    }
+  __syncthreads();
+  if((int)threadIdx.x < CO){
+    float v = 0.f;
+    for(int w = 0; w < CNN_CONV_THREADS / TCK_WAVE; w++) v += red[w * CO + threadIdx.x];
+    A.bpart[(long long)blockIdx.x * CO + threadIdx.x] = v;
   }
 }
 
@@ -353,58 +390,83 @@ __global__ void __launch_bounds__(CNN_WG_THREADS) tck_cnn_wgrad(const WgradArgs 
   }
 }
 
-/* out[e] = sum_b part[b][e] (b in order) */
-__global__ void tck_cnn_reduce(const float * part, int nblk, int n, float * out){
-  const int e = blockIdx.x * blockDim.x + threadIdx.x;
-  if(e >= n) return;
-  float s = 0.f;
-  for(int b = 0; b < nblk; b++) s += part[(long long)b * n + e];
-  out[e] = s;
-}
+/* The fixed-order sums of the per-block partial results of all layers in one launch:
+ * out[e] = sum_b part[b][e].  A block takes 64 entries of one segment; its four waves sum a
+ * quarter of the partials each, in order, eight loads at a time, and the quarters are added
+ * in order. */
+#define CNN_NSEG 6
+struct ReduceArgs {
+  const float * part[CNN_NSEG];
+  float * out[CNN_NSEG];
+  int n[CNN_NSEG], nblk[CNN_NSEG];
+  int first[CNN_NSEG + 1];     /* first block of each segment */
+};
 
-/* bias gradient: db[co] partial sums of g over cells (fp32 from the un-rounded gradient) */
-__global__ void tck_cnn_bgrad(const float * g, long long nv, int co_n, long long cells_per_block, float * part){
-  const long long v0 = (long long)blockIdx.x * cells_per_block;
-  const long long v1 = min(v0 + cells_per_block, nv);
-  for(int co = threadIdx.x; co < co_n; co += blockDim.x){
-    float s = 0.f;
-    for(long long v = v0; v < v1; v++) s += g[v * co_n + co];
-    part[(long long)blockIdx.x * co_n + co] = s;
+__global__ void __launch_bounds__(256) tck_cnn_reduce(const ReduceArgs A){
+  __shared__ float red[4][64];
+  int sg = 0;
+  while(sg + 1 < CNN_NSEG && (int)blockIdx.x >= A.first[sg + 1]) sg++;
+  const int lane = threadIdx.x % 64, w = threadIdx.x / 64;
+  const int n = A.n[sg], nblk = A.nblk[sg];
+  const int e = ((int)blockIdx.x - A.first[sg]) * 64 + lane;
+  const int q = (nblk + 3) / 4;
+  const int b1 = min((w + 1) * q, nblk);
+  int b = w * q;
+  float s = 0.f;
+  if(e < n){
+    const float * p = A.part[sg] + e;
+    for(; b + 8 <= b1; b += 8){
+      float v[8];
+      #pragma unroll
+      for(int u = 0; u < 8; u++) v[u] = p[(long long)(b + u) * n];
+      #pragma unroll
+      for(int u = 0; u < 8; u++) s += v[u];
+    }
+    for(; b < b1; b++) s += p[(long long)b * n];
   }
+  red[w][lane] = s;
+  __syncthreads();
+  if(w == 0 && e < n) A.out[sg][e] = ((red[0][lane] + red[1][lane]) + red[2][lane]) + red[3][lane];
 }
 
 /* ---------------------------------------------------------------------------------------
  * elementwise pieces
  * ------------------------------------------------------------------------------------- */
-/* loss = mean over cells and channels of (pred - target)^2; grad = d loss / d pred.
- * part[blk] = partial sum of squares */
-__global__ void __launch_bounds__(256) tck_cnn_mse(const float * pred, const float * target, long long n,
-    float scale, float * grad, float * part){
-  __shared__ float red[256];
-  float s = 0.f;
-  for(long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x; e < n; e += (long long)gridDim.x * blockDim.x){
-    const float d = pred[e] - target[e];
-    grad[e] = 2.f * d * scale;
-    s += d * d;
+/* loss = mean over cells and the four channels of (pred - target)^2, and its gradient: one
+ * cell per thread and iteration.  g: the gradient as BF16 rows of 16 channels (4 used, the
+ * others zero), the operand of the backward products; bpart, lpart: per-block sums of the FP32
+ * gradient (16 entries) and of the squares */
+__global__ void __launch_bounds__(256) tck_cnn_mse(const float4 * pred, const float4 * target, long long nv,
+    float scale, unsigned short * g, float * bpart, float * lpart){
+  __shared__ float red[256][5];
+  float s[5] = {0.f, 0.f, 0.f, 0.f, 0.f};
+  for(long long v = (long long)blockIdx.x * blockDim.x + threadIdx.x; v < nv; v += (long long)gridDim.x * blockDim.x){
+    const float4 p = pred[v], t = target[v];
+    const float d[4] = {p.x - t.x, p.y - t.y, p.z - t.z, p.w - t.w};
+    uint32_t h[4];
+    #pragma unroll
+    for(int c = 0; c < 4; c++){
+      const float gr = 2.f * d[c] * scale;
+      h[c] = cnn_bf16(gr);
+      s[c] += gr;
+      s[4] += d[c] * d[c];
+    }
+    uint4 * row = (uint4 *)(g + v * 16);
+    row[0] = make_uint4(h[0] | (h[1] << 16), h[2] | (h[3] << 16), 0u, 0u);
+    row[1] = make_uint4(0u, 0u, 0u, 0u);
   }
-  red[threadIdx.x] = s;
+  #pragma unroll
+  for(int c = 0; c < 5; c++) red[threadIdx.x][c] = s[c];
   __syncthreads();
   for(int h = 128; h > 0; h >>= 1){
-    if((int)threadIdx.x < h) red[threadIdx.x] += red[threadIdx.x + h];
+    if((int)threadIdx.x < h){
+      #pragma unroll
+      for(int c = 0; c < 5; c++) red[threadIdx.x][c] += red[threadIdx.x + h][c];
+    }
     __syncthreads();
   }
-  if(threadIdx.x == 0) part[blockIdx.x] = red[0];
-}
-
-/* gradient through ReLU: g_pre = g_post where the stored activation is positive, as BF16
- * (the operand of the next products); gf: the same in FP32 for the bias gradient */
-__global__ void tck_cnn_relu_bwd(const float * gpost, const unsigned short * act, long long n,
-    unsigned short * gpre, float * gf){
-  for(long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x; e < n; e += (long long)gridDim.x * blockDim.x){
-    const float v = cnn_f32(act[e]) > 0.f ? gpost[e] : 0.f;
-    gpre[e] = cnn_bf16(v);
-    if(gf) gf[e] = v;
-  }
+  if(threadIdx.x < 16) bpart[blockIdx.x * 16 + threadIdx.x] = threadIdx.x < 4 ? red[0][threadIdx.x] : 0.f;
+  if(threadIdx.x == 16) lpart[blockIdx.x] = red[0][4];
 }
 
 /* FP32 -> BF16 copy */
@@ -427,19 +489,38 @@ __global__ void tck_cnn_flip(const unsigned short * w, int co_n, int ci_n, int c
   wt[e] = v;
 }
 
-/* Adam on FP32 masters, BF16 copies re-rounded */
-__global__ void tck_cnn_adam(float * w, float * m, float * v, const float * g, int n, float lr,
-    float b1, float b2, float eps, float c1, float c2, unsigned short * wbf){
+/* Adam on the FP32 masters of all layers in one launch (one segment per blockIdx.y); weights
+ * are re-rounded to their BF16 copies, the plain one and the flipped one of the backward data
+ * pass (tck_cnn_flip) */
+struct AdamArgs {
+  float * w[CNN_NSEG]; float * m[CNN_NSEG]; float * v[CNN_NSEG];
+  const float * g[CNN_NSEG];
+  unsigned short * wbf[CNN_NSEG]; unsigned short * wt[CNN_NSEG];   /* or null */
+  int n[CNN_NSEG], co[CNN_NSEG], ci[CNN_NSEG];
+  float lr, b1, b2, eps, c1, c2;
+};
+
+__global__ void __launch_bounds__(256) tck_cnn_adam(const AdamArgs A){
+  const int sg = blockIdx.y;
   const int e = blockIdx.x * blockDim.x + threadIdx.x;
-  if(e >= n) return;
-  const float gg = g[e];
-  const float mm = b1 * m[e] + (1.f - b1) * gg;
-  const float vv = b2 * v[e] + (1.f - b2) * gg * gg;
-  m[e] = mm;
-  v[e] = vv;
-  const float upd = lr * (mm / c1) / (sqrtf(vv / c2) + eps);
-  w[e] -= upd;
-  if(wbf) wbf[e] = cnn_bf16(w[e]);
+  if(e >= A.n[sg]) return;
+  const float gg = A.g[sg][e];
+  const float mm = A.b1 * A.m[sg][e] + (1.f - A.b1) * gg;
+  const float vv = A.b2 * A.v[sg][e] + (1.f - A.b2) * gg * gg;
+  A.m[sg][e] = mm;
+  A.v[sg][e] = vv;
+  const float upd = A.lr * (mm / A.c1) / (sqrtf(vv / A.c2) + A.eps);
+  const float w = A.w[sg][e] - upd;
+  A.w[sg][e] = w;
+  if(A.wbf[sg]){
+    const unsigned short h = cnn_bf16(w);
+    A.wbf[sg][e] = h;
+    if(A.wt[sg]){
+      const int ci = A.ci[sg], co = A.co[sg];
+      const int ic = e % ci, oc = (e / ci) % co, tap = e / (ci * co);
+      A.wt[sg][((26 - tap) * ci + ic) * co + oc] = h;
+    }
+  }
 }
 
 /* ---------------------------------------------------------------------------------------
@@ -476,7 +557,7 @@ __global__ void tck_cnn_gather(const GatherArgs A){
 
 struct ScatterArgs {
   tc_geom_t g;
-  const float * pred;       /* [nv][16] network output, channels 0..3 used */
+  const float * pred;       /* [nv][4] network output */
   float scale[4];           /* output de-normalisation */
   float * cx; float * cy; float * cz; float * ct;   /* corrections, field layout */
 };
@@ -490,11 +571,11 @@ __global__ void tck_cnn_scatter(const ScatterArgs A){
   if(i > A.g.nx) return;
   const long long o = tck_idx(A.g, i, j, k);
   const long long v = (long long)(i - 1) + (long long)A.g.nx * ((long long)(j - 1) + (long long)A.g.ny * (k - 1));
-  const float * p = A.pred + v * 16;
+  const float * p = A.pred + v * 4;
   A.cy[o] = A.scale[1] * p[1];
   A.cz[o] = A.scale[2] * p[2];
   if(A.ct) A.ct[o] = A.scale[3] * p[3];
-  if(i >= 2) A.cx[o] = A.scale[0] * (0.5f * A.pred[(v - 1) * 16] + 0.5f * p[0]);
+  if(i >= 2) A.cx[o] = A.scale[0] * (0.5f * A.pred[(v - 1) * 4] + 0.5f * p[0]);
   else A.cx[o] = 0.f;
 }
 
@@ -536,28 +617,45 @@ static int cnn_ncu(void){
   return g_cnn_ncu;
 }
 
+/* blocks of a convolution: persistent, as many as the LDS holds per CU (the kernel and a
+ * halo'd tile) */
+static int cnn_conv_blocks(int nx, int ny, int nz, int nb, int ci, int co){
+  const long long ntiles = (long long)((nx + 15) / 16) * ((ny + CNN_TY - 1) / CNN_TY) * ((nz + CNN_TZ - 1) / CNN_TZ) * nb;
+  long long per_cu = (160LL * 1024) / cnn_conv_lds(ci, co);
+  per_cu = per_cu < 1 ? 1 : (per_cu > 4 ? 4 : per_cu);
+  const long long cap = per_cu * cnn_ncu();
+  return (int)(ntiles < cap ? ntiles : cap);
+}
+
 extern "C" {
 
+/* the most blocks a backward convolution has (entries of its bias partial sums: 32 each) */
+int tck_cnn_bgrad_blocks(int nx, int ny, int nz, int nb){
+  const int a = cnn_conv_blocks(nx, ny, nz, nb, 16, 32), b = cnn_conv_blocks(nx, ny, nz, nb, 32, 32);
+  return a > b ? a : b;
+}
+
+/* out_bf set and act null: CNN_RELU; act set: CNN_RELU_BWD, *nblk the blocks of its partial
+ * sums; else CNN_PLAIN into out_f */
 int tck_cnn_launch_conv(int nx, int ny, int nz, int nb, const unsigned short * in, int ci,
-    const unsigned short * w, int co, const float * bias, int co_store, int relu,
-    unsigned short * out_bf, float * out_f, hipStream_t stream){
+    const unsigned short * w, int co, const float * bias, int co_store,
+    unsigned short * out_bf, float * out_f, const unsigned short * act, float * bpart, int * nblk,
+    hipStream_t stream){
   ConvArgs A;
   A.G.nx = nx; A.G.ny = ny; A.G.nz = nz; A.G.nb = nb; A.G.nv = (long long)nx * ny * nz * nb;
   A.in = in; A.w = w; A.bias = bias; A.out_bf = out_bf; A.out_f = out_f;
-  A.co_store = co_store; A.relu = relu;
-  /* persistent blocks, as many as the LDS holds per CU (the kernel and a halo'd tile) */
-  const long long ntiles = (long long)((nx + 15) / 16) * ((ny + CNN_TY - 1) / CNN_TY) * ((nz + CNN_TZ - 1) / CNN_TZ) * nb;
+  A.act = act; A.bpart = bpart;
+  A.co_store = co_store;
+  A.mode = act ? CNN_RELU_BWD : (out_bf ? CNN_RELU : CNN_PLAIN);
+  if(co_store % 4 != 0 || co_store > co) return (int)hipErrorInvalidValue;
   const int lds = cnn_conv_lds(ci, co);
-  long long per_cu = (160LL * 1024) / lds;
-  per_cu = per_cu < 1 ? 1 : (per_cu > 4 ? 4 : per_cu);
-  long long nblk = ntiles;
-  if(nblk > per_cu * cnn_ncu()) nblk = per_cu * cnn_ncu();
-  const dim3 grd((unsigned)nblk);
+  const int blocks = cnn_conv_blocks(nx, ny, nz, nb, ci, co);
+  if(nblk) *nblk = blocks;
+  const dim3 grd((unsigned)blocks);
   int rc;
   if(ci == 16 && co == 32) rc = cnn_conv_launch<16, 32>(A, grd, lds, stream);
   else if(ci == 32 && co == 32) rc = cnn_conv_launch<32, 32>(A, grd, lds, stream);
   else if(ci == 32 && co == 16) rc = cnn_conv_launch<32, 16>(A, grd, lds, stream);
-  else if(ci == 16 && co == 16) rc = cnn_conv_launch<16, 16>(A, grd, lds, stream);
   else return (int)hipErrorInvalidValue;
   if(rc) return rc;
   TCK_CHECK_LAUNCH();
@@ -565,7 +663,8 @@ int tck_cnn_launch_conv(int nx, int ny, int nz, int nb, const unsigned short * i
 }
 
 int tck_cnn_launch_wgrad(int nx, int ny, int nz, int nb, const unsigned short * in, int ci_n,
-    const unsigned short * g, int co_n, float * part, int nblk, float * out, hipStream_t stream){
+    const unsigned short * g, int co_n, float * part, int * nblk_io, hipStream_t stream){
+  int nblk = *nblk_io;
   WgradArgs A;
   A.G.nx = nx; A.G.ny = ny; A.G.nz = nz; A.G.nb = nb; A.G.nv = (long long)nx * ny * nz * nb;
   A.in = in; A.g = g; A.part = part;
@@ -578,32 +677,33 @@ int tck_cnn_launch_wgrad(int nx, int ny, int nz, int nb, const unsigned short * 
   else if(ci_n == 32 && co_n == 16) rc = cnn_wgrad_launch<32, 16>(A, nblk, stream);
   else return (int)hipErrorInvalidValue;
   if(rc) return rc;
-  TCK_CHECK_LAUNCH();
-  const int n = 27 * co_n * ci_n;
-  hipLaunchKernelGGL(tck_cnn_reduce, dim3((n + 255) / 256), dim3(256), 0, stream, (const float *)part, nblk, n, out);
+  *nblk_io = nblk;
   TCK_CHECK_LAUNCH();
   return 0;
 }
 
-int tck_cnn_launch_bgrad(long long nv, const float * g, int co_n, float * part, int nblk, float * out,
-    hipStream_t stream){
-  hipLaunchKernelGGL(tck_cnn_bgrad, dim3(nblk), dim3(64), 0, stream, g, nv, co_n, (nv + nblk - 1) / nblk, part);
-  TCK_CHECK_LAUNCH();
-  hipLaunchKernelGGL(tck_cnn_reduce, dim3((co_n + 255) / 256), dim3(256), 0, stream, (const float *)part, nblk, co_n, out);
+/* nseg sums of per-block partials, in one launch */
+int tck_cnn_launch_reduce(int nseg, const float * const * part, const int * nblk, const int * n,
+    float * const * out, hipStream_t stream){
+  if(nseg < 1 || nseg > CNN_NSEG) return (int)hipErrorInvalidValue;
+  ReduceArgs A;
+  int first = 0;
+  for(int q = 0; q < CNN_NSEG; q++){
+    const int m = q < nseg ? q : nseg - 1;
+    A.part[q] = part[m]; A.out[q] = out[m]; A.n[q] = n[m]; A.nblk[q] = nblk[m];
+    A.first[q] = first;
+    if(q < nseg) first += (n[q] + 63) / 64;
+  }
+  A.first[CNN_NSEG] = first;
+  hipLaunchKernelGGL(tck_cnn_reduce, dim3((unsigned)first), dim3(256), 0, stream, A);
   TCK_CHECK_LAUNCH();
   return 0;
 }
 
-int tck_cnn_launch_mse(const float * pred, const float * target, long long n, float scale,
-    float * grad, float * part, int nblk, hipStream_t stream){
-  hipLaunchKernelGGL(tck_cnn_mse, dim3(nblk), dim3(256), 0, stream, pred, target, n, scale, grad, part);
-  TCK_CHECK_LAUNCH();
-  return 0;
-}
-
-int tck_cnn_launch_relu_bwd(const float * gpost, const unsigned short * act, long long n,
-    unsigned short * gpre, float * gf, hipStream_t stream){
-  hipLaunchKernelGGL(tck_cnn_relu_bwd, dim3(2048), dim3(256), 0, stream, gpost, act, n, gpre, gf);
+int tck_cnn_launch_mse(const float * pred, const float * target, long long nv, float scale,
+    unsigned short * g, float * bpart, float * lpart, int nblk, hipStream_t stream){
+  hipLaunchKernelGGL(tck_cnn_mse, dim3(nblk), dim3(256), 0, stream, (const float4 *)pred, (const float4 *)target,
+      nv, scale, g, bpart, lpart);
   TCK_CHECK_LAUNCH();
   return 0;
 }
@@ -622,10 +722,20 @@ int tck_cnn_launch_flip(const unsigned short * w, int co_n, int ci_n, int ci_p, 
   return 0;
 }
 
-int tck_cnn_launch_adam(float * w, float * m, float * v, const float * g, int n, float lr,
-    float b1, float b2, float eps, float c1, float c2, unsigned short * wbf, hipStream_t stream){
-  hipLaunchKernelGGL(tck_cnn_adam, dim3((n + 255) / 256), dim3(256), 0, stream, w, m, v, g, n, lr,
-      b1, b2, eps, c1, c2, wbf);
+int tck_cnn_launch_adam(int nseg, float * const * w, float * const * m, float * const * v,
+    float * const * g, unsigned short * const * wbf, unsigned short * const * wt, const int * n,
+    const int * co, const int * ci, float lr, float b1, float b2, float eps, float c1, float c2,
+    hipStream_t stream){
+  if(nseg < 1 || nseg > CNN_NSEG) return (int)hipErrorInvalidValue;
+  AdamArgs A;
+  int nmax = 0;
+  for(int q = 0; q < nseg; q++){
+    A.w[q] = w[q]; A.m[q] = m[q]; A.v[q] = v[q]; A.g[q] = g[q]; A.wbf[q] = wbf[q]; A.wt[q] = wt[q];
+    A.n[q] = n[q]; A.co[q] = co[q]; A.ci[q] = ci[q];
+    if(n[q] > nmax) nmax = n[q];
+  }
+  A.lr = lr; A.b1 = b1; A.b2 = b2; A.eps = eps; A.c1 = c1; A.c2 = c2;
+  hipLaunchKernelGGL(tck_cnn_adam, dim3((nmax + 255) / 256, nseg), dim3(256), 0, stream, A);
   TCK_CHECK_LAUNCH();
   return 0;
 }
