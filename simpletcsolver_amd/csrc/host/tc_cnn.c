@@ -3,7 +3,7 @@
  *
  * A tc_cnn_t holds the network (FP32 master weights, BF16 copies, Adam moments) and the
  * activation buffers of one batch.  Training data arrive from the host as FP32 channels-last
- * arrays (the caller normalises them); the library pads the inputs to 16 channels and rounds
+ * arrays (the caller normalises them); the device pads the inputs to 16 channels and rounds
  * them to BF16.  tc_closure_attach couples a trained network to a solver: at the start of
  * every step the solver evaluates the network on its current fields and the predictor adds
  * the resulting corrections to the explicit right-hand sides of ux, uy, uz and T.
@@ -28,6 +28,7 @@ int tck_cnn_launch_reduce(int nseg, const float * const * part, const int * nblk
     float * const * out, hipStream_t stream);
 int tck_cnn_launch_mse(const float * pred, const float * target, long long nv, float scale,
     unsigned short * g, float * bpart, float * lpart, int nblk, hipStream_t stream);
+int tck_cnn_launch_pack(const float * x, long long nv, unsigned short * out, hipStream_t stream);
 int tck_cnn_launch_to_bf16(const float * x, long long n, unsigned short * y, hipStream_t stream);
 int tck_cnn_launch_flip(const unsigned short * w, int co_n, int ci_n, int ci_p, int co_p,
     unsigned short * wt, hipStream_t stream);
@@ -42,6 +43,7 @@ int tck_cnn_launch_scatter(const tc_geom_t * g, const float * pred, const float 
     float * cx, float * cy, float * cz, float * ct, hipStream_t stream);
 
 #define CNN_C0 16      /* padded input channels */
+#define CNN_IN 5       /* input channels in use */
 #define CNN_C 32       /* hidden channels */
 #define CNN_CO 16      /* padded output channels of the last layer's kernel */
 #define CNN_OUT 4      /* output channels stored */
@@ -66,6 +68,7 @@ struct tc_cnn_s {
   unsigned short * wt[3];       /* flipped kernels of the backward data pass */
   long long step;
   /* activations of one batch */
+  float * xin;                  /* [nv][5], the caller's inputs */
   unsigned short * x0;          /* [nv][16] */
   unsigned short * a1; unsigned short * a2;   /* [nv][32] */
   float * out;                  /* [nv][4] */
@@ -74,7 +77,6 @@ struct tc_cnn_s {
   unsigned short * g2; unsigned short * g1;   /* d loss / d a2, d a1 through the ReLUs, BF16 */
   float * pw[3]; float * pb[3]; /* per-block partial sums of the weight and bias gradients */
   float * lpart;                /* and of the loss, [CNN_NBLK] */
-  unsigned short * h_x;         /* host staging */
 };
 
 static long long wsize(int l){ return 27LL * g_co[l] * g_ci[l]; }
@@ -83,14 +85,6 @@ static int cnn_alloc(void ** p, size_t bytes){
   if(hipMalloc(p, bytes ? bytes : 8) != hipSuccess) return tc_fail("tc_cnn: hipMalloc of %zu bytes failed", bytes);
   if(hipMemset(*p, 0, bytes ? bytes : 8) != hipSuccess) return tc_fail("tc_cnn: hipMemset failed");
   return 0;
-}
-
-/* host FP32 -> BF16 (round to nearest even) */
-static unsigned short bf16(float x){
-  unsigned int u;
-  memcpy(&u, &x, 4);
-  u += 0x7fffu + ((u >> 16) & 1u);
-  return (unsigned short)(u >> 16);
 }
 
 int tc_cnn_destroy(tc_cnn_t * c){
@@ -111,10 +105,9 @@ int tc_cnn_destroy(tc_cnn_t * c){
       c->pw[l], c->pb[l]};
     for(size_t q = 0; q < sizeof(p) / sizeof(p[0]); q++) if(p[q]) hipFree(p[q]);
   }
-  void * a[] = {c->x0, c->a1, c->a2, c->out, c->target, c->g3, c->g2, c->g1, c->lpart};
+  void * a[] = {c->xin, c->x0, c->a1, c->a2, c->out, c->target, c->g3, c->g2, c->g1, c->lpart};
   for(size_t q = 0; q < sizeof(a) / sizeof(a[0]); q++) if(a[q]) hipFree(a[q]);
   if(c->stream) hipStreamDestroy(c->stream);
-  free(c->h_x);
   free(c);
   return 0;
 }
@@ -150,7 +143,7 @@ int tc_cnn_create(int nx, int ny, int nz, int batch, unsigned long long seed, in
   }
   const size_t nv = (size_t)c->nv;
   if(!rc){
-    rc |= cnn_alloc((void **)&c->x0, 2 * nv * CNN_C0);
+    rc |= cnn_alloc((void **)&c->xin, 4 * nv * CNN_IN) || cnn_alloc((void **)&c->x0, 2 * nv * CNN_C0);
     rc |= cnn_alloc((void **)&c->a1, 2 * nv * CNN_C) || cnn_alloc((void **)&c->a2, 2 * nv * CNN_C);
     rc |= cnn_alloc((void **)&c->out, 4 * nv * CNN_OUT) || cnn_alloc((void **)&c->target, 4 * nv * CNN_OUT);
     rc |= cnn_alloc((void **)&c->g3, 2 * nv * CNN_CO);
@@ -162,8 +155,6 @@ int tc_cnn_create(int nx, int ny, int nz, int batch, unsigned long long seed, in
             cnn_alloc((void **)&c->pb[l], 4 * nbl * (size_t)g_co[l]);
     }
   }
-  c->h_x = calloc(nv * CNN_C0, 2);
-  if(!c->h_x) rc = tc_fail("host allocation failed");
   /* initial weights */
   unsigned long long st = seed * 0x9E3779B97F4A7C15ULL + 12345;
   for(int l = 0; l < 3 && !rc; l++){
@@ -218,11 +209,8 @@ int tc_cnn_get_layer(tc_cnn_t * c, int l, float * w, float * b, float * gw, floa
 
 /* inputs [nb][nz][ny][nx][5] FP32 (normalised) -> BF16 [nv][16] on the device */
 static int upload_x(tc_cnn_t * c, const float * x){
-  const long long nv = c->nv;
-  for(long long v = 0; v < nv; v++){
-    for(int q = 0; q < CNN_C0; q++) c->h_x[v * CNN_C0 + q] = q < 5 ? bf16(x[v * 5 + q]) : 0;
-  }
-  HIPOK(hipMemcpyAsync(c->x0, c->h_x, 2 * (size_t)nv * CNN_C0, hipMemcpyHostToDevice, c->stream));
+  HIPOK(hipMemcpyAsync(c->xin, x, 4 * (size_t)c->nv * CNN_IN, hipMemcpyHostToDevice, c->stream));
+  KOK(tck_cnn_launch_pack(c->xin, c->nv, c->x0, c->stream));
   return 0;
 }
 

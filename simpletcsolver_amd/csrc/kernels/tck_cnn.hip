@@ -469,6 +469,21 @@ __global__ void __launch_bounds__(256) tck_cnn_mse(const float4 * pred, const fl
   if(threadIdx.x == 16) lpart[blockIdx.x] = red[0][4];
 }
 
+/* network inputs as the caller gives them, [nv][5] FP32, to the BF16 rows of 16 channels the
+ * first convolution reads (channels 5..15 zero).  One cell per thread: the rows are formed
+ * here rather than on the host, which took 5.5 ms for a million cells against 20 us, and 20
+ * bytes per cell cross PCIe instead of 32 */
+__global__ void __launch_bounds__(256) tck_cnn_pack(const float * x, long long nv, unsigned short * out){
+  for(long long v = (long long)blockIdx.x * blockDim.x + threadIdx.x; v < nv; v += (long long)gridDim.x * blockDim.x){
+    uint32_t h[5];
+    #pragma unroll
+    for(int q = 0; q < 5; q++) h[q] = cnn_bf16(x[v * 5 + q]);
+    uint4 * row = (uint4 *)(out + v * 16);
+    row[0] = make_uint4(h[0] | (h[1] << 16), h[2] | (h[3] << 16), h[4], 0u);
+    row[1] = make_uint4(0u, 0u, 0u, 0u);
+  }
+}
+
 /* FP32 -> BF16 copy */
 __global__ void tck_cnn_to_bf16(const float * x, long long n, unsigned short * y){
   for(long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x; e < n; e += (long long)gridDim.x * blockDim.x)
@@ -704,6 +719,13 @@ int tck_cnn_launch_mse(const float * pred, const float * target, long long nv, f
     unsigned short * g, float * bpart, float * lpart, int nblk, hipStream_t stream){
   hipLaunchKernelGGL(tck_cnn_mse, dim3(nblk), dim3(256), 0, stream, (const float4 *)pred, (const float4 *)target,
       nv, scale, g, bpart, lpart);
+  TCK_CHECK_LAUNCH();
+  return 0;
+}
+
+int tck_cnn_launch_pack(const float * x, long long nv, unsigned short * out, hipStream_t stream){
+  const long long nb = (nv + 255) / 256;
+  hipLaunchKernelGGL(tck_cnn_pack, dim3((unsigned)(nb < 4096 ? nb : 4096)), dim3(256), 0, stream, x, nv, out);
   TCK_CHECK_LAUNCH();
   return 0;
 }
