@@ -50,10 +50,20 @@ struct CnnGrid { int nx, ny, nz, nb; long long nv; };
  * channels 4 (l / 16) .. +3 of cell l % 16, which go out as one 8- or 16-byte store.
  *
  * A block stages the kernel once (rows of CI BF16 padded by 16 bytes, so that the 16 lanes
- * reading one K group hit distinct banks) and loops over tiles of 16 x CNN_TY x CNN_TZ cells
- * of one sample: each tile's activations with a one-cell halo (zero outside the walls in x,
- * periodic images in y and z) are staged in LDS with the same padded rows, and every tap of
- * every cell is then read from LDS.  Each wave takes CNN_RPW rows of the tile.
+ * reading one K group hit distinct banks) and loops over a run of tiles of 16 x CNN_TY x CNN_TZ
+ * cells of one sample: each tile's activations with a one-cell halo (zero outside the walls in
+ * x, periodic images in y and z) are staged in LDS with the same padded rows, the next tile's
+ * on their way into registers during the products.  A wave takes the CNN_TY rows of one z; the
+ * 18 input pieces (six rows, three x shifts) that a plane of taps needs are read once and
+ * used by all rows and taps they reach, so that the plane's 72 products of a 32 -> 32 layer
+ * read 36 pieces from LDS instead of 72.  The taps are added in the order of their index
+ * whatever the tile, so the result does not depend on the tiling.
+ *
+ * Measured on a million cells (64 x 128 x 128): 88 us for 32 -> 32 channels (660 TFLOP/s), 56
+ * us for 32 -> 16 and 63 us for 16 -> 32; reading each tap's operands from LDS again for every
+ * row, with the halo images found by runtime division, took 149, 111 and 73 us.  LDS reads
+ * and, on small grids, the staging bound it: 18, 11 and 14 us at 32 x 64 x 64, where each CU
+ * has one tile (23, 18 and 14 us before).
  * ------------------------------------------------------------------------------------- */
 struct ConvArgs {
   CnnGrid G;
@@ -73,12 +83,13 @@ struct ConvArgs {
  * stored BF16 for the next products, with the FP32 values summed for the bias gradient */
 enum { CNN_PLAIN = 0, CNN_RELU = 1, CNN_RELU_BWD = 2 };
 
-#define CNN_CONV_THREADS 512
 #define CNN_TY 4
-#define CNN_TZ 4
+/* depth of a tile, one wave per z: a block of 155 KB (32 input channels) or 93 KB (16) per CU.
+ * For 16 input channels two blocks of depth 4 per CU were no faster (66 against 63 us for a
+ * million cells) and slower where each CU has one tile (17.0 against 13.6 us at 32 x 64 x 64) */
+#define CNN_TZ 8
 #define CNN_HX 18                             /* halo'd tile: 16 + 2 cells in x */
 #define CNN_HCELLS (CNN_HX * (CNN_TY + 2) * (CNN_TZ + 2))
-#define CNN_RPW ((CNN_TY * CNN_TZ) / (CNN_CONV_THREADS / TCK_WAVE))   /* rows per wave */
 
 typedef __bf16 cnn_b8 __attribute__((ext_vector_type(8)));
 
@@ -87,89 +98,166 @@ __host__ __device__ constexpr int cnn_conv_lds(int ci, int co){
   return (27 * co + CNN_HCELLS) * (2 * ci + 16);
 }
 
+/* periodic image of a position at most one cell below the grid or some cells above it (the
+ * halo and the unused rows of a tile); only grids thinner than a tile need the division */
 __device__ __forceinline__ int cnn_wrap(int a, int n){
-  a %= n;
-  return a < 0 ? a + n : a;
+  if(a < 0) return a + n;
+  if(a >= n){
+    a -= n;
+    if(a >= n) a %= n;
+  }
+  return a;
 }
 
 template <int CI, int CO>
-__global__ void __launch_bounds__(CNN_CONV_THREADS) tck_cnn_conv(const ConvArgs A){
+__global__ void __launch_bounds__(CNN_TZ * TCK_WAVE) tck_cnn_conv(const ConvArgs A){
+  constexpr int TZ = CNN_TZ, NTH = TZ * TCK_WAVE, HC = CNN_HCELLS;
   constexpr int RS = 2 * CI + 16;                 /* padded row: bytes per cell or per co */
   constexpr int NT = CO / 16;                     /* 16-channel output blocks */
-  constexpr int NK = CI == 32 ? 27 : 14;          /* MFMA steps over the taps */
+  constexpr int PC = CI / 8;                      /* 16-byte pieces per row */
+  constexpr int NP = (HC * PC + NTH - 1) / NTH;   /* tile pieces per thread */
+  constexpr int NW = (27 * CO * PC + NTH - 1) / NTH;      /* kernel pieces per thread */
   extern __shared__ __align__(16) unsigned char cnn_smem[];
   unsigned char * wl = cnn_smem;                  /* [27][CO] rows */
   unsigned char * al = cnn_smem + 27 * CO * RS;   /* [HZ][HY][HX] rows */
-  /* the kernel: 16-byte pieces, CI / 8 per row */
-  for(int e = threadIdx.x; e < 27 * CO * (CI / 8); e += CNN_CONV_THREADS){
-    const int row = e / (CI / 8), pc = e % (CI / 8);
-    *(uint4 *)(wl + row * RS + 16 * pc) = *(const uint4 *)(A.w + (long long)row * CI + 8 * pc);
-  }
   const int lane = threadIdx.x % TCK_WAVE;
-  const int wv = threadIdx.x / TCK_WAVE;
+  const int wv = threadIdx.x / TCK_WAVE;          /* z within the tile */
   const int kg = lane / 16;                       /* this lane's K group */
-  const int cl = lane % 16;                       /* A row (cell in x) / B column (channel) */
+  const int cl = lane % 16;                       /* A row (channel) / B column (cell in x) */
   const CnnGrid & G = A.G;
-  const int ntx = (G.nx + 15) / 16, nty = (G.ny + CNN_TY - 1) / CNN_TY, ntz = (G.nz + CNN_TZ - 1) / CNN_TZ;
-  const long long ntiles = (long long)ntx * nty * ntz * G.nb;
-  /* CI = 16: K group kg reads tap 2 s + (kg >> 1), channels 8 (kg & 1) .. +7 */
-  const int ktap = CI == 32 ? 0 : (kg >> 1);
-  const int kbyte = CI == 32 ? 16 * kg : 16 * (kg & 1);
+  const int ntx = (G.nx + 15) / 16, nty = (G.ny + CNN_TY - 1) / CNN_TY, ntz = (G.nz + TZ - 1) / TZ;
+  const int ntiles = ntx * nty * ntz * G.nb;
+  /* a contiguous run of tiles per block, neighbouring runs on the same XCD */
+  const int per = (ntiles + (int)gridDim.x - 1) / (int)gridDim.x;
+  int run = blockIdx.x;
+  if(gridDim.x % TCK_NXCD == 0) run = (run % TCK_NXCD) * ((int)gridDim.x / TCK_NXCD) + run / TCK_NXCD;
+  const int t0 = run * per, t1 = min(t0 + per, ntiles);
+  uint4 pre[NP];
+  auto fetch = [&](int tile){
+    int r = tile / ntx;
+    const int x0 = 16 * (tile % ntx), y0 = CNN_TY * (r % nty);
+    r /= nty;
+    const int z0 = TZ * (r % ntz), b = r / ntz;
+    #pragma unroll
+    for(int q = 0; q < NP; q++){
+      const int e = threadIdx.x + q * NTH;
+      const int c = e / PC, pc = e % PC;
+      const int hx = c % CNN_HX, hy = (c / CNN_HX) % (CNN_TY + 2), hz = c / (CNN_HX * (CNN_TY + 2));
+      const int xx = x0 + hx - 1;
+      pre[q] = uint4{0u, 0u, 0u, 0u};
+      if(c < HC && xx >= 0 && xx < G.nx){
+        const int yy = cnn_wrap(y0 + hy - 1, G.ny), zz = cnn_wrap(z0 + hz - 1, G.nz);
+        const long long src = (long long)xx + (long long)G.nx * ((long long)yy + (long long)G.ny * ((long long)zz + (long long)G.nz * b));
+        pre[q] = *(const uint4 *)(A.in + src * CI + 8 * pc);
+      }
+    }
+  };
+  if(t0 < t1) fetch(t0);
+  {
+    uint4 wp[NW];
+    #pragma unroll
+    for(int q = 0; q < NW; q++){
+      const int e = threadIdx.x + q * NTH;
+      if(e < 27 * CO * PC) wp[q] = *(const uint4 *)(A.w + 8LL * e);
+    }
+    #pragma unroll
+    for(int q = 0; q < NW; q++){
+      const int e = threadIdx.x + q * NTH;
+      if(e < 27 * CO * PC) *(uint4 *)(wl + (e / PC) * RS + 16 * (e % PC)) = wp[q];
+    }
+  }
   cnn_f4 bsum[NT];
   #pragma unroll
   for(int t = 0; t < NT; t++) bsum[t] = cnn_f4{0.f, 0.f, 0.f, 0.f};
-  for(long long tile = blockIdx.x; tile < ntiles; tile += gridDim.x){
-    const int tx = (int)(tile % ntx);
-    long long r = tile / ntx;
-    const int ty = (int)(r % nty); r /= nty;
-    const int tz = (int)(r % ntz);
-    const int b = (int)(r / ntz);
-    const int x0 = 16 * tx, y0 = CNN_TY * ty, z0 = CNN_TZ * tz;
+  for(int tile = t0; tile < t1; tile++){
+    int r = tile / ntx;
+    const int x0 = 16 * (tile % ntx), y0 = CNN_TY * (r % nty);
+    r /= nty;
+    const int z0 = TZ * (r % ntz), b = r / ntz;
     __syncthreads();                              /* the previous tile's reads are done */
-    for(int e = threadIdx.x; e < CNN_HCELLS * (CI / 8); e += CNN_CONV_THREADS){
-      const int c = e / (CI / 8), pc = e % (CI / 8);
-      const int hx = c % CNN_HX, hy = (c / CNN_HX) % (CNN_TY + 2), hz = c / (CNN_HX * (CNN_TY + 2));
-      const int xx = x0 + hx - 1;
-      uint4 v = {0u, 0u, 0u, 0u};
-      if(xx >= 0 && xx < G.nx){
-        const int yy = cnn_wrap(y0 + hy - 1, G.ny), zz = cnn_wrap(z0 + hz - 1, G.nz);
-        const long long src = (long long)xx + (long long)G.nx * ((long long)yy + (long long)G.ny * ((long long)zz + (long long)G.nz * b));
-        v = *(const uint4 *)(A.in + src * CI + 8 * pc);
-      }
-      *(uint4 *)(al + c * RS + 16 * pc) = v;
+    #pragma unroll
+    for(int q = 0; q < NP; q++){
+      const int e = threadIdx.x + q * NTH;
+      if(e < HC * PC) *(uint4 *)(al + (e / PC) * RS + 16 * (e % PC)) = pre[q];
     }
     __syncthreads();
-    cnn_f4 acc[CNN_RPW][NT];
+    if(tile + 1 < t1) fetch(tile + 1);
+    /* the stored activations of the wave's cells, in flight during the products */
+    ushort4 act[CNN_TY][NT];
+    if(A.mode == CNN_RELU_BWD){
+      #pragma unroll
+      for(int q = 0; q < CNN_TY; q++){
+        const int x = x0 + cl, y = y0 + q, z = z0 + wv;
+        const bool in = x < G.nx && y < G.ny && z < G.nz;
+        const long long v = in ? (long long)x + (long long)G.nx * ((long long)y + (long long)G.ny * ((long long)z + (long long)G.nz * b)) : 0;
+        #pragma unroll
+        for(int t = 0; t < NT; t++){
+          const int co = 16 * t + 4 * kg;
+          act[q][t] = *(const ushort4 *)(A.act + v * A.co_store + (co < A.co_store ? co : 0));
+        }
+      }
+    }
+    cnn_f4 acc[CNN_TY][NT];
     #pragma unroll
-    for(int q = 0; q < CNN_RPW; q++)
+    for(int q = 0; q < CNN_TY; q++)
       #pragma unroll
       for(int t = 0; t < NT; t++) acc[q][t] = cnn_f4{0.f, 0.f, 0.f, 0.f};
-    for(int s = 0; s < NK; s++){
-      const int tap = CI == 32 ? s : 2 * s + ktap;
-      const bool live = tap < 27;
-      const int tp = live ? tap : 26;
-      const int dx = tp % 3, dy = (tp / 3) % 3, dz = tp / 9;   /* halo offsets 0..2 */
-      cnn_b8 bw[NT];
-      #pragma unroll
-      for(int t = 0; t < NT; t++){
-        bw[t] = *(const cnn_b8 *)(wl + (tp * CO + 16 * t + cl) * RS + kbyte);
-        if(!live) bw[t] = cnn_b8{};
-      }
-      #pragma unroll
-      for(int q = 0; q < CNN_RPW; q++){
-        const int row = wv * CNN_RPW + q;
-        const int ry = row % CNN_TY, rz = row / CNN_TY;
-        const int c = (cl + dx) + CNN_HX * ((ry + dy) + (CNN_TY + 2) * (rz + dz));
-        const cnn_b8 av = *(const cnn_b8 *)(al + c * RS + kbyte);
+    if constexpr (CI == 32){
+      #pragma unroll 1
+      for(int dz = 0; dz < 3; dz++){
+        const unsigned char * ap = al + (cl + CNN_HX * ((CNN_TY + 2) * (wv + dz))) * RS + 16 * kg;
+        const unsigned char * wp = wl + (9 * dz * CO + cl) * RS + 16 * kg;
+        cnn_b8 av[CNN_TY + 2][3];
         #pragma unroll
-        for(int t = 0; t < NT; t++) acc[q][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bw[t], av, acc[q][t], 0, 0, 0);
+        for(int hy = 0; hy < CNN_TY + 2; hy++)
+          #pragma unroll
+          for(int dx = 0; dx < 3; dx++) av[hy][dx] = *(const cnn_b8 *)(ap + (dx + CNN_HX * hy) * RS);
+        #pragma unroll
+        for(int tp = 0; tp < 9; tp++){
+          cnn_b8 bw[NT];
+          #pragma unroll
+          for(int t = 0; t < NT; t++) bw[t] = *(const cnn_b8 *)(wp + (tp * CO + 16 * t) * RS);
+          #pragma unroll
+          for(int q = 0; q < CNN_TY; q++)
+            #pragma unroll
+            for(int t = 0; t < NT; t++)
+              acc[q][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bw[t], av[q + tp / 3][tp % 3], acc[q][t], 0, 0, 0);
+        }
+      }
+    }else{
+      /* K group kg reads tap 2 s + (kg >> 1), channels 8 (kg & 1) .. +7: fully unrolled, so that
+       * a step's input offset is one select between two constants */
+      const int odd = kg >> 1;
+      const unsigned char * ap = al + (cl + CNN_HX * ((CNN_TY + 2) * wv)) * RS + 16 * (kg & 1);
+      const unsigned char * wp = wl + (odd * CO + cl) * RS + 16 * (kg & 1);
+      #pragma unroll
+      for(int s = 0; s < 14; s++){
+        constexpr int HP = CNN_HX * (CNN_TY + 2);
+        const int ta = 2 * s, tb = 2 * s + 1 < 27 ? 2 * s + 1 : 26;
+        const int oa = (ta % 3 + CNN_HX * ((ta / 3) % 3) + HP * (ta / 9)) * RS;
+        const int ob = (tb % 3 + CNN_HX * ((tb / 3) % 3) + HP * (tb / 9)) * RS;
+        const unsigned char * as = ap + (odd ? ob : oa);
+        cnn_b8 bw[NT];
+        #pragma unroll
+        for(int t = 0; t < NT; t++){
+          /* the last step's odd half has no tap: zeros (its read stays on tap 26) */
+          if(s == 13){
+            bw[t] = *(const cnn_b8 *)(wl + (26 * CO + cl + 16 * t) * RS + 16 * (kg & 1));
+            if(odd) bw[t] = cnn_b8{};
+          }else bw[t] = *(const cnn_b8 *)(wp + (ta * CO + 16 * t) * RS);
+        }
+        #pragma unroll
+        for(int q = 0; q < CNN_TY; q++){
+          const cnn_b8 av = *(const cnn_b8 *)(as + CNN_HX * q * RS);
+          #pragma unroll
+          for(int t = 0; t < NT; t++) acc[q][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bw[t], av, acc[q][t], 0, 0, 0);
+        }
       }
     }
     /* accumulator: channels 16 t + 4 kg .. +3 of cell x0 + cl of the row */
     #pragma unroll
-    for(int q = 0; q < CNN_RPW; q++){
-      const int row = wv * CNN_RPW + q;
-      const int x = x0 + cl, y = y0 + row % CNN_TY, z = z0 + row / CNN_TY;
+    for(int q = 0; q < CNN_TY; q++){
+      const int x = x0 + cl, y = y0 + q, z = z0 + wv;
       if(x >= G.nx || y >= G.ny || z >= G.nz) continue;
       const long long v = (long long)x + (long long)G.nx * ((long long)y + (long long)G.ny * ((long long)z + (long long)G.nz * b));
       #pragma unroll
@@ -186,7 +274,7 @@ __global__ void __launch_bounds__(CNN_CONV_THREADS) tck_cnn_conv(const ConvArgs 
           #pragma unroll
           for(int u = 0; u < 4; u++) val[u] = val[u] > 0.f ? val[u] : 0.f;
         }else{
-          const ushort4 a = *(const ushort4 *)(A.act + v * A.co_store + co);
+          const ushort4 a = act[q][t];
           val[0] = cnn_f32(a.x) > 0.f ? val[0] : 0.f;
           val[1] = cnn_f32(a.y) > 0.f ? val[1] : 0.f;
           val[2] = cnn_f32(a.z) > 0.f ? val[2] : 0.f;
@@ -212,7 +300,7 @@ __global__ void __launch_bounds__(CNN_CONV_THREADS) tck_cnn_conv(const ConvArgs 
   __syncthreads();
   if((int)threadIdx.x < CO){
     float v = 0.f;
-    for(int w = 0; w < CNN_CONV_THREADS / TCK_WAVE; w++) v += red[w * CO + threadIdx.x];
+    for(int w = 0; w < TZ; w++) v += red[w * CO + threadIdx.x];
     A.bpart[(long long)blockIdx.x * CO + threadIdx.x] = v;
   }
 }
@@ -604,7 +692,7 @@ static int cnn_conv_launch(const ConvArgs & A, dim3 grd, int lds, hipStream_t st
     if(e != hipSuccess) return (int)e;
     ready = 1;
   }
-  hipLaunchKernelGGL((tck_cnn_conv<CI, CO>), grd, dim3(CNN_CONV_THREADS), lds, stream, A);
+  hipLaunchKernelGGL((tck_cnn_conv<CI, CO>), grd, dim3(CNN_TZ * TCK_WAVE), lds, stream, A);
   return 0;
 }
 
@@ -632,10 +720,14 @@ static int cnn_ncu(void){
   return g_cnn_ncu;
 }
 
+static long long cnn_conv_tiles(int nx, int ny, int nz, int nb){
+  return (long long)((nx + 15) / 16) * ((ny + CNN_TY - 1) / CNN_TY) * ((nz + CNN_TZ - 1) / CNN_TZ) * nb;
+}
+
 /* blocks of a convolution: persistent, as many as the LDS holds per CU (the kernel and a
  * halo'd tile) */
 static int cnn_conv_blocks(int nx, int ny, int nz, int nb, int ci, int co){
-  const long long ntiles = (long long)((nx + 15) / 16) * ((ny + CNN_TY - 1) / CNN_TY) * ((nz + CNN_TZ - 1) / CNN_TZ) * nb;
+  const long long ntiles = cnn_conv_tiles(nx, ny, nz, nb);
   long long per_cu = (160LL * 1024) / cnn_conv_lds(ci, co);
   per_cu = per_cu < 1 ? 1 : (per_cu > 4 ? 4 : per_cu);
   const long long cap = per_cu * cnn_ncu();
@@ -662,7 +754,7 @@ int tck_cnn_launch_conv(int nx, int ny, int nz, int nb, const unsigned short * i
   A.act = act; A.bpart = bpart;
   A.co_store = co_store;
   A.mode = act ? CNN_RELU_BWD : (out_bf ? CNN_RELU : CNN_PLAIN);
-  if(co_store % 4 != 0 || co_store > co) return (int)hipErrorInvalidValue;
+  if(co_store % 4 != 0 || co_store > co || cnn_conv_tiles(nx, ny, nz, nb) > 0x7fffffffLL) return (int)hipErrorInvalidValue;
   const int lds = cnn_conv_lds(ci, co);
   const int blocks = cnn_conv_blocks(nx, ny, nz, nb, ci, co);
   if(nblk) *nblk = blocks;
