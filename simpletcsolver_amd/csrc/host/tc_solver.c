@@ -338,28 +338,50 @@ static int setup_linesolve(tc_solver_t * s){
   return 0;
 }
 
-/* launch shapes of the cell kernels (planes per block kb, rows per block ty): 32 x 4 for both
- * the predictor and the correction, shortened until the grid has at least four blocks
- * per CU, so that small grids fill the device (tc_autotune refines them).  The predictor
- * stages the fields' planes in LDS whenever its tiles have 4 rows. */
+/* launch shapes of the cell kernels (planes per block kb, rows per block ty; tc_autotune refines
+ * them).
+ *
+ * The predictor (window form, 32 x 8 tiles, three blocks per CU): a block costs its prologue
+ * (two planes and the coefficient rows) and its planes, and what a choice of kb costs beyond that
+ * is the last, partly empty round of blocks.  kb is the cheapest by a model of both, measured
+ * on nine grids from 64 x 64 x 64 to 512 x 1024 x 1024: a full round of blocks takes
+ * 4.5 + 5.85 kb us, a round with r blocks per CU 4.5 + (2.0 + 1.28 r) kb; it reproduces the
+ * times to 5-15 % and their order where they differ by more than 5 %.  Against the former rule
+ * (kb halved from 32 until the grid has four 64 x 4 tiles per CU, 4 rows or fewer): 64 x 8 x 32
+ * 16.9 -> 9.6 us (the direct form before), 64 x 64 x 64 19.4 -> 17.4, 96 x 192 x 192 136 -> 114,
+ * 150 x 140 x 180 146 -> 136, 97 x 150 x 105 83 -> 75; above some 10^7 cells kb = 24 or 32 either
+ * way.
+ *
+ * The correction (64 x 4 tiles, no prologue to speak of): kb halved from 16 until there are 14
+ * blocks per CU, which hides its load latency best: 150 x 140 x 180 72 -> 66 us, 97 x 150 x 105
+ * 39 -> 34, 256 x 512 x 512 1050 -> 1019, 512 x 1024 x 1024 8.12 -> 8.08 ms. */
 static void default_shapes(tc_solver_t * s){
   int ncu = 0;
   if(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, s->p.device) != hipSuccess || ncu <= 0) ncu = 256;
-  const long long want = 4LL * ncu;
-  const long long nbx = (s->p.nx + 63) / 64;
-  const int start[2][2] = {{32, 4}, {32, 4}};
-  const int which[2] = {TC_TUNE_PREDICT, TC_TUNE_CORRECT};
-  for(int q = 0; q < 2; q++){
-    int kb = start[q][0], ty = start[q][1];
-    for(;;){
-      const long long nb = nbx * ((s->p.ny + ty - 1) / ty) * ((s->p.nz + kb - 1) / kb);
-      if(nb >= want) break;
-      if(kb > 1) kb /= 2;
-      else if(ty > 1) ty /= 2;
-      else break;
+  const int nx = s->p.nx, ny = s->p.ny, nz = s->p.nz;
+  {
+    static const int kbs[10] = {32, 24, 16, 12, 8, 6, 4, 3, 2, 1};
+    const long long tiles = (long long)((nx + 31) / 32) * ((ny + 7) / 8), slots = 3LL * ncu;
+    double best = INFINITY;
+    for(int q = 0; q < 10; q++){
+      const int kb = kbs[q];
+      if(kb > nz) continue;
+      const long long nb = tiles * ((nz + kb - 1) / kb);
+      const long long rem = nb % slots, r = (rem + ncu - 1) / ncu;
+      const double t = (double)(nb / slots) * (4.5 + 5.85 * kb) + (rem ? 4.5 + (2.0 + 1.28 * (double)r) * kb : 0.);
+      if(t < best){
+        best = t;
+        s->tune[TC_TUNE_PREDICT][0] = kb;
+      }
     }
-    s->tune[which[q]][0] = kb;
-    s->tune[which[q]][1] = ty;
+    s->tune[TC_TUNE_PREDICT][1] = 4;
+  }
+  {
+    const long long tiles = (long long)((nx + 63) / 64) * ((ny + 3) / 4);
+    int kb = 16;
+    while(kb > 1 && (kb > nz || tiles * ((nz + kb - 1) / kb) < 14LL * ncu)) kb /= 2;
+    s->tune[TC_TUNE_CORRECT][0] = kb;
+    s->tune[TC_TUNE_CORRECT][1] = 4;
   }
   s->predict_window = 1;
   s->fft_exact = 7;
