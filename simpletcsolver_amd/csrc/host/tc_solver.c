@@ -758,12 +758,13 @@ static int launch_dt(tc_solver_t * s){
 }
 
 /* stale-tensor diagnostics of the reference's logging: gradients at the start of the last
- * predict (injection.c:49-51, dissipation.c:36-229) */
+ * predict (injection.c:49-51, dissipation.c:36-229); the scalar terms read the current T, so
+ * they are left out here */
 static int snapshot_diag(tc_solver_t * s){
   PROF(TC_S_DIAG, tck_launch_diag_walls(&s->g, &s->coef, tc_field_ptr(s, TC_FUX), tc_field_ptr(s, TC_FUY),
-      tc_field_ptr(s, TC_FT), s->p.scalar, s->d_part, s->d_diag + 8, s->stream));
+      tc_field_ptr(s, TC_FT), 0, s->d_part, s->d_diag + 8, s->stream));
   PROF(TC_S_DIAG, tck_launch_diag_cells(&s->g, &s->coef, tc_field_ptr(s, TC_FUX), tc_field_ptr(s, TC_FUY),
-      tc_field_ptr(s, TC_FUZ), tc_field_ptr(s, TC_FT), s->p.scalar, s->d_part, s->d_diag, s->stream));
+      tc_field_ptr(s, TC_FUZ), tc_field_ptr(s, TC_FT), 0, s->d_part, s->d_diag, s->stream));
   HIPOK(hipMemcpyAsync(s->h_diag_snap, s->d_diag, sizeof(double) * 10, hipMemcpyDeviceToHost, s->stream));
   s->diag_pending = 1;
   return 0;
@@ -1124,12 +1125,12 @@ int tc_total_energy(tc_solver_t * s, double out[4]){
 
 /* values of the reference's logging: the velocity terms come from the tensors left by the
  * last predict (snapshot), the scalar terms read the current T (injection.c:75-87,
- * dissipation.c:243-318) */
-static int logging_values(tc_solver_t * s, double vals[10]){
+ * dissipation.c:243-318); walls: the injection's terms (vals 8 and 9), else the dissipation's */
+static int logging_values(tc_solver_t * s, int walls, double vals[10]){
   HIPOK(hipSetDevice(s->p.device));
-  KOK(tck_launch_diag_walls(&s->g, &s->coef, tc_field_ptr(s, TC_FUX), tc_field_ptr(s, TC_FUY),
+  if(walls) KOK(tck_launch_diag_walls(&s->g, &s->coef, tc_field_ptr(s, TC_FUX), tc_field_ptr(s, TC_FUY),
       tc_field_ptr(s, TC_FT), s->p.scalar, s->d_part, s->d_diag + 8, s->stream));
-  KOK(tck_launch_diag_cells(&s->g, &s->coef, tc_field_ptr(s, TC_FUX), tc_field_ptr(s, TC_FUY),
+  else KOK(tck_launch_diag_cells(&s->g, &s->coef, tc_field_ptr(s, TC_FUX), tc_field_ptr(s, TC_FUY),
       tc_field_ptr(s, TC_FUZ), tc_field_ptr(s, TC_FT), s->p.scalar, s->d_part, s->d_diag, s->stream));
   HIPOK(hipMemcpyAsync(vals, s->d_diag, sizeof(double) * 10, hipMemcpyDeviceToHost, s->stream));
   HIPOK(hipStreamSynchronize(s->stream));
@@ -1142,7 +1143,7 @@ static int logging_values(tc_solver_t * s, double vals[10]){
 
 int tc_injection(tc_solver_t * s, double out[2]){
   double v[10];
-  if(logging_values(s, v)) return 1;
+  if(logging_values(s, 1, v)) return 1;
   out[0] = s->nu * v[8];
   out[1] = s->kappa * v[9];
   return 0;
@@ -1150,7 +1151,7 @@ int tc_injection(tc_solver_t * s, double out[2]){
 
 int tc_dissipation(tc_solver_t * s, double out[2]){
   double v[10];
-  if(logging_values(s, v)) return 1;
+  if(logging_values(s, 0, v)) return 1;
   out[0] = s->nu * v[1];
   out[1] = s->kappa * v[2];
   return 0;
