@@ -396,17 +396,108 @@ __device__ __forceinline__ void wave_sync(){
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+/* The x systems of a field are the same for every line, so what a solve does to the factors
+ * alone is done once per block: the products a_i = - r_i l_i of the rows, and the products of a
+ * that each step of the two scans multiplies by (the composition's slopes), which leaves only
+ * the offsets to be exchanged and combined per line. */
+struct XSlopes {
+  double fwd[6], bwd[6];
+  __device__ __forceinline__ double f(int k) const { return fwd[k]; }
+  __device__ __forceinline__ double g(int k) const { return bwd[k]; }
+};
+/* the same, read from LDS where they are used ([12][64], this lane's column) */
+struct XSlopesLds {
+  const double * at;
+  __device__ __forceinline__ double f(int k) const { return at[k * TCK_WAVE]; }
+  __device__ __forceinline__ double g(int k) const { return at[(6 + k) * TCK_WAVE]; }
+};
+
+template <int SEG>
+__device__ __forceinline__ XSlopes xsolve_slopes(const double * rr, const double * ll, const double * vv, int n){
+  XSlopes S;
+  const int lane = threadIdx.x % TCK_WAVE;
+  const int row0 = lane * SEG;
+  double a = 1.;
+  #pragma unroll
+  for(int e = 0; e < SEG; e++) if(row0 + e < n) a = row0 + e == 0 ? 0. : (- rr[e] * ll[e]) * a;
+  #pragma unroll
+  for(int k = 0; k < 6; k++){
+    S.fwd[k] = a;
+    const double ap = __shfl_up(a, 1 << k, TCK_WAVE);
+    if(lane >= (1 << k)) a = a * ap;
+  }
+  a = 1.;
+  #pragma unroll
+  for(int e = SEG - 1; e >= 0; e--) if(row0 + e < n) a = row0 + e == n - 1 ? 0. : (- vv[e]) * a;
+  #pragma unroll
+  for(int k = 0; k < 6; k++){
+    S.bwd[k] = a;
+    const double ap = __shfl_down(a, 1 << k, TCK_WAVE);
+    if(lane + (1 << k) < TCK_WAVE) a = a * ap;
+  }
+  return S;
+}
+
+/* wave_tdm on one real line with the slopes given: the same operations on q, so the same bits.
+ * Rows past n are left alone and pass values through. */
+template <int SEG, typename SL>
+__device__ __forceinline__ void xsolve_line(double * q, const double * rr, const double * ll, const double * vv,
+    const SL & S, int n){
+  const int lane = threadIdx.x % TCK_WAVE;
+  const int row0 = lane * SEG;
+  const double q0 = lane == 0 ? q[0] / rr[0] : 0.;   /* row 0 */
+  double b = 0.;
+  #pragma unroll
+  for(int e = 0; e < SEG; e++) if(row0 + e < n){
+    if(e == 0) b = lane == 0 ? q0 : (- rr[e] * ll[e]) * b + rr[e] * q[e];
+    else b = (- rr[e] * ll[e]) * b + rr[e] * q[e];
+  }
+  #pragma unroll
+  for(int k = 0; k < 6; k++){
+    const double bp = __shfl_up(b, 1 << k, TCK_WAVE);
+    if(lane >= (1 << k)) b = S.f(k) * bp + b;
+  }
+  double in = __shfl_up(b, 1, TCK_WAVE);
+  if(lane == 0) in = 0.;
+  #pragma unroll
+  for(int e = 0; e < SEG; e++) if(row0 + e < n){
+    if(e == 0) q[e] = lane == 0 ? q0 : rr[e] * (q[e] - ll[e] * in);
+    else q[e] = rr[e] * (q[e] - ll[e] * in);
+    in = q[e];
+  }
+  b = 0.;
+  #pragma unroll
+  for(int e = SEG - 1; e >= 0; e--) if(row0 + e < n) b = row0 + e == n - 1 ? q[e] : (- vv[e]) * b + q[e];
+  #pragma unroll
+  for(int k = 0; k < 6; k++){
+    const double bp = __shfl_down(b, 1 << k, TCK_WAVE);
+    if(lane + (1 << k) < TCK_WAVE) b = S.g(k) * bp + b;
+  }
+  in = __shfl_down(b, 1, TCK_WAVE);
+  if(lane == TCK_WAVE - 1) in = 0.;
+  #pragma unroll
+  for(int e = SEG - 1; e >= 0; e--) if(row0 + e < n){
+    if(row0 + e != n - 1) q[e] -= vv[e] * in;
+    in = q[e];
+  }
+}
+
 /* Four waves per block, one x line per wave per iteration; blocks loop over groups of four
  * lines.  The factor rows (the same for every line) are staged once per block in LDS, in the
- * lanes' segment order, and read where the recurrences use them: held in registers for the
- * whole loop they would cost 3 SEG doubles per lane and occupancy.  Lines are staged through
- * a wave-private LDS area: global loads and stores are contiguous across the wave (lane t
- * touches elements t, t+64, ...), each lane solves its contiguous segment. */
+ * lanes' segment order; lines of up to 256 rows hold them and the slopes in registers from there,
+ * longer ones read both where they are used (3 SEG + 12 doubles per lane would cost occupancy).
+ * Lines are staged through a wave-private LDS area: global loads and stores are contiguous
+ * across the wave (lane t touches elements t, t+64, ...), each lane solves its contiguous
+ * segment.  What bounds it is the LDS: 26 exchanges and
+ * 16 reads and writes of 8 bytes per line of 256 (52 and 44 with the slopes formed per line and
+ * the factors read from LDS), 8 B per cell in FP32.  Measured: the x solves of 256 x 512 x 512 in
+ * mixed precision 2.64 -> 1.74 ms per step, of 128 x 192 x 256 in FP64 (with the field update)
+ * 0.416 -> 0.354, of 256 x 512 x 512 3.80 -> 3.71 (5.2 TB/s). */
 template <int SEG, typename D, bool U>
 __device__ __forceinline__ void xsolve_body(const XSolveArgs & A, D * __restrict__ dd,
     double * uout, const double * __restrict__ ucur, const double * __restrict__ rt,
     const double * __restrict__ vt, const double * __restrict__ lt, const int i0, const int n,
-    double * sm, double (*tab)[TCK_WAVE * (SEG + 1)]){
+    double * sm, double (*tab)[TCK_WAVE * (SEG + 1)], double * slt){
   const tc_geom_t & g = A.g;
   const int w = threadIdx.x / TCK_WAVE;
   const int lane = threadIdx.x % TCK_WAVE;
@@ -417,6 +508,26 @@ __device__ __forceinline__ void xsolve_body(const XSolveArgs & A, D * __restrict
     tab[2][stage_pos<SEG>(idx)] = vt[row];
   }
   __syncthreads();
+  constexpr bool REG = SEG <= 4;
+  constexpr int NREG = REG ? SEG : 1;
+  double rreg[NREG], lreg[NREG], vreg[NREG];
+  if constexpr (REG){
+    #pragma unroll
+    for(int e = 0; e < SEG; e++){
+      rreg[e] = tab[0][lane * (SEG + 1) + e];
+      lreg[e] = tab[1][lane * (SEG + 1) + e];
+      vreg[e] = tab[2][lane * (SEG + 1) + e];
+    }
+  }
+  XSlopes slopes;
+  if constexpr (REG || !U) slopes = xsolve_slopes<SEG>(&tab[0][lane * (SEG + 1)], &tab[1][lane * (SEG + 1)], &tab[2][lane * (SEG + 1)], n);
+  if constexpr (!REG && !U){
+    if(w == 0){
+      #pragma unroll
+      for(int k = 0; k < 6; k++){ slt[k * TCK_WAVE + lane] = slopes.fwd[k]; slt[(6 + k) * TCK_WAVE + lane] = slopes.bwd[k]; }
+    }
+    __syncthreads();
+  }
   const long long nlines = (long long)g.ny * g.nz;
   const int wpb = TCK_BLOCK / TCK_WAVE;
   const long long stride = (long long)gridDim.x * wpb;
@@ -464,15 +575,24 @@ __device__ __forceinline__ void xsolve_body(const XSolveArgs & A, D * __restrict
     XS_FETCH(line + stride);
     const long long base = tck_idx(g, i0, j, k);
     wave_sync();
-    /* the table offset is opaque to the compiler, so the reads stay inside the loop */
-    int toff = lane * (SEG + 1);
-    asm volatile("" : "+v"(toff));
-    double q[SEG][1];
+    double q[SEG];
     #pragma unroll
-    for(int e = 0; e < SEG; e++) q[e][0] = sm[lane * (SEG + 1) + e];
-    wave_tdm<SEG, 1>(q, &tab[0][toff], &tab[1][toff], &tab[2][toff], n);
+    for(int e = 0; e < SEG; e++) q[e] = sm[lane * (SEG + 1) + e];
+    if constexpr (REG) xsolve_line<SEG>(q, rreg, lreg, vreg, slopes, n);
+    else if constexpr (U){
+      /* beside the old field's values there are no registers to spare for the slopes' reads:
+       * formed again per line (1.5 % faster here) */
+      int toff = lane * (SEG + 1);
+      asm volatile("" : "+v"(toff));
+      wave_tdm<SEG, 1>((double (*)[1])q, &tab[0][toff], &tab[1][toff], &tab[2][toff], n);
+    }else{
+      /* the table offsets are opaque to the compiler, so the reads stay inside the loop */
+      int toff = lane * (SEG + 1), soff = lane;
+      asm volatile("" : "+v"(toff), "+v"(soff));
+      xsolve_line<SEG>(q, &tab[0][toff], &tab[1][toff], &tab[2][toff], XSlopesLds{slt + soff}, n);
+    }
     #pragma unroll
-    for(int e = 0; e < SEG; e++) sm[lane * (SEG + 1) + e] = q[e][0];
+    for(int e = 0; e < SEG; e++) sm[lane * (SEG + 1) + e] = q[e];
     wave_sync();
     if constexpr (U){
       const __amdgpu_buffer_rsrc_t ro = tck_rsrc_u(uout + base, live ? nbu : 0u);
@@ -502,9 +622,10 @@ template <int SEG, typename D, bool U>
 __global__ void __launch_bounds__(TCK_BLOCK) __attribute__((amdgpu_waves_per_eu(SEG <= 8 ? 4 : 1))) tck_xsolve(const XSolveArgs A){
   __shared__ double xs_sm[TCK_BLOCK / TCK_WAVE][TCK_WAVE * (SEG + 1)];
   __shared__ double xs_tab[3][TCK_WAVE * (SEG + 1)];
+  __shared__ double xs_slopes[SEG <= 4 || U ? 1 : 12 * TCK_WAVE];
   const int f = blockIdx.y;
   xsolve_body<SEG, D, U>(A, (D *)A.d[f], A.uout[f], A.ucur[f], A.r[f], A.v[f], A.l[f], A.i0[f], A.n[f],
-      xs_sm[threadIdx.x / TCK_WAVE], xs_tab);
+      xs_sm[threadIdx.x / TCK_WAVE], xs_tab, xs_slopes);
 }
 
 /* periodic lines in y (solve_in_y, :39-70) or z (solve_in_z, :72-103).  A block holds TI
