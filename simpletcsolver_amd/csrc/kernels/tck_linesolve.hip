@@ -682,19 +682,35 @@ __device__ __forceinline__ void ps_rows(Q * out, const double * __restrict__ t, 
   }
 }
 
+/* bytes of n elements of sz bytes, for a buffer resource's size */
+__device__ __forceinline__ unsigned ps_bytes(long long n, int sz){
+  const long long b = n * sz;
+  return b <= 0 ? 0u : (b < 0xFFFFFFFFLL ? (unsigned)b : 0xFFFFFFFFu);
+}
+
 /* plain store (as a halo image's) at byte offset vo + so of resource r */
 __device__ __forceinline__ void ps_bsti(__amdgpu_buffer_rsrc_t r, unsigned vo, unsigned so, double v){
   __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(tck_u2v, v), r, vo, so, 0);
 }
 
+/* rows per segment: FP64 lines are cut into full segments (the last one shorter), so that all
+ * but the first and last can take the lean form; the mixed step's are cut evenly */
+template <typename D, int MAXM>
+__device__ __forceinline__ int ps_seg(int m, int S){
+  return sizeof(D) == 8 ? MAXM : (m + S - 1) / S;
+}
+
 /* body with restrict-qualified pointers: loads of the old field and the tables may be
  * scheduled ahead of the stores to the increment array.
- * Two forms of the same operations, chosen per wave: the general one tests every row (row 0,
- * row m-1, rows past the segment's count) and forms 64-bit addresses per row; the lean one,
- * taken when every lane of the wave holds a full segment (MAXM rows) of interior rows, has no
- * row tests and reaches the rows through buffer resources based at the wave's first lane, with
- * a 32-bit offset per lane and a uniform one per row (the launcher checks that the offsets of
- * a wave stay below 2^31).  The arithmetic of a row is the same in both. */
+ * Two forms of the same operations, chosen per wave.  The lean one, taken when every lane of
+ * the wave holds a full segment (MAXM rows) of interior rows at or past the convergence row,
+ * has no row tests, constant factors, and one buffer resource based at the wave's first lane
+ * with a 32-bit offset per lane and a uniform one per row.  The other handles everything else
+ * in groups of PS_PRE rows: what a group needs (table rows below jc, the pivot of row m-1, rows
+ * past a segment's end) is decided for the wave, so that most groups run the lean form's
+ * instructions; its rows are reached the same way, through a resource based at the group's
+ * first row and bounded by the array's end (a lane's rows past its segment may lie past it:
+ * they read as 0 and are not used).  The arithmetic of a row is the same in both. */
 template <typename D, int MAXM, bool LEAN>
 __device__ __forceinline__ void psolve_body(const PSolveArgs & A, D * __restrict__ d, double * uout,
     const double * __restrict__ ucur, const double * __restrict__ rt, const double * __restrict__ vt,
@@ -711,7 +727,7 @@ __device__ __forceinline__ void psolve_body(const PSolveArgs & A, D * __restrict
   const bool valid = i >= ib0 && i < ib0 + isz;
   const int n = A.dir == 1 ? g.ny : g.nz;
   const int m = n - 1;
-  const int seg = (m + S - 1) / S;
+  const int seg = ps_seg<D, MAXM>(m, S);
   const int row0 = sg * seg;
   int cnt = m - row0;
   cnt = cnt < 0 ? 0 : (cnt > seg ? seg : cnt);
@@ -725,7 +741,6 @@ __device__ __forceinline__ void psolve_body(const PSolveArgs & A, D * __restrict
   const long long ts = A.tstride;
   const double * r = rt + col;
   const double * v = vt + col;
-  const double * q1 = q1t + col;
   typedef D Q;   /* arithmetic type: the increment's own */
   const Q den = Q(meta[col]);
   const Q tl = Q(meta[ts + col]);
@@ -745,6 +760,22 @@ __device__ __forceinline__ void psolve_body(const PSolveArgs & A, D * __restrict
   const unsigned sel = (unsigned)step;
   unsigned vtab = (unsigned)((col + ts * row0) * 8);
   const unsigned stab = (unsigned)(ts * 8);
+  /* the most rows any lane of the wave has (the first lane's: segments are in lane order), and
+   * whether any lane has rows below the convergence row */
+  const int cu = __builtin_amdgcn_readfirstlane(cnt);
+  const bool low = __builtin_amdgcn_ballot_w64(row0 < jc) != 0;
+  /* resource of array p (elements of sz bytes) from the wave's first lane's row e0 to its end */
+  #define PS_GRP(p, e0, sz) tck_rsrc_u((p) + (w0 + step * (e0)), ps_bytes(g.n3 - (w0 + step * (e0)), (int)(sz)))
+  /* do all lanes have the PS_PRE rows from e0; does any hold row m-1 among them */
+  #define PS_FULL(e0) (__builtin_amdgcn_ballot_w64(cnt < (e0) + PS_PRE) == 0)
+  /* factor rows of a group */
+  #define PS_ROWS(t, tab, e0, cval, lval) \
+    if(low && __builtin_amdgcn_ballot_w64(row0 + (e0) < jc) != 0) ps_rows(t, tab, ts, row0, e0, jc, m, cval, lval); \
+    else if(__builtin_amdgcn_ballot_w64(row0 + (e0) <= m - 1 && row0 + (e0) + PS_PRE > m - 1) != 0){ \
+      _Pragma("unroll") for(int e = 0; e < PS_PRE; e++) t[e] = row0 + (e0) + e == m - 1 ? (lval) : (cval); \
+    }else{ \
+      _Pragma("unroll") for(int e = 0; e < PS_PRE; e++) t[e] = (cval); \
+    }
   Q q[MAXM];
   if constexpr(LEAN){
     const __amdgpu_buffer_rsrc_t rd = tck_rsrc_u(d + w0, 0xFFFFFFFFu);
@@ -753,12 +784,21 @@ __device__ __forceinline__ void psolve_body(const PSolveArgs & A, D * __restrict
       q[e] = Q(tck_bldn<D>(rd, vel * (unsigned)sizeof(D), (unsigned)e * sel * (unsigned)sizeof(D)));
   }else{
     #pragma unroll
-    for(int e = 0; e < MAXM; e++) q[e] = (valid && e < cnt) ? Q(tck_ld(&d[base + step * (row0 + e)])) : Q(0.);
+    for(int e0 = 0; e0 < MAXM; e0 += PS_PRE){
+      if(e0 < cu){
+        const __amdgpu_buffer_rsrc_t rd = PS_GRP(d, e0, sizeof(D));
+        #pragma unroll
+        for(int e = 0; e < PS_PRE; e++) q[e0 + e] = Q(tck_bldn<D>(rd, vel * (unsigned)sizeof(D), (unsigned)e * sel * (unsigned)sizeof(D)));
+      }else{
+        #pragma unroll
+        for(int e = 0; e < PS_PRE; e++) q[e0 + e] = Q(0.);
+      }
+    }
   }
   if(valid && sg == S - 1) smX[2 * TI + ti] = Q(d[base + step * m]);
   Q t[PS_PRE];
   /* forward: q0 = q0 / c0, q_i = r_i (q_i - l q_{i-1}) */
-  Q a = Q(1.), b = Q(0.);
+  Q a = Q(1.), b = Q(0.), q0d = Q(0.);   /* q0d: row 0's result */
   if constexpr(LEAN){
     /* rows from jc on: the factors are the constants */
     #pragma unroll
@@ -771,20 +811,22 @@ __device__ __forceinline__ void psolve_body(const PSolveArgs & A, D * __restrict
   }else{
     #pragma unroll
     for(int e0 = 0; e0 < MAXM; e0 += PS_PRE){
-      if(e0 < cnt){
-        ps_rows(t, r, ts, row0, e0, jc, m, rc, rlast);
-        #pragma unroll
-        for(int e = 0; e < PS_PRE; e++){
-          if(e0 + e < cnt){
-            const int row = row0 + e0 + e;
-            if(row == 0){ a = Q(0.); b = q[e0 + e] / t[e]; }
-            else {
-              const Q ai = - t[e] * tl;
-              b = ai * b + t[e] * q[e0 + e];
-              a = ai * a;
-            }
-          }
+      if(e0 < cu){
+        PS_ROWS(t, r, e0, rc, rlast);
+        if(e0 == 0 && row0 == 0) q0d = q[0] / t[0];
+        #define PS_STEP(e) { \
+          const Q ai = - t[e] * tl; \
+          b = ai * b + t[e] * q[e0 + e]; \
+          a = ai * a; \
+          if(e0 + e == 0 && row0 == 0){ a = Q(0.); b = q0d; } }
+        if(PS_FULL(e0)){
+          #pragma unroll
+          for(int e = 0; e < PS_PRE; e++) PS_STEP(e)
+        }else{
+          #pragma unroll
+          for(int e = 0; e < PS_PRE; e++) if(e0 + e < cnt) PS_STEP(e)
         }
+        #undef PS_STEP
       }
     }
   }
@@ -815,20 +857,23 @@ __device__ __forceinline__ void psolve_body(const PSolveArgs & A, D * __restrict
   }else{
     #pragma unroll
     for(int e0 = 0; e0 < MAXM; e0 += PS_PRE){
-      if(e0 < cnt){
-        ps_rows(t, r, ts, row0, e0, jc, m, rc, rlast);
-        #pragma unroll
-        for(int e = 0; e < PS_PRE; e++){
-          if(e0 + e < cnt){
-            const int row = row0 + e0 + e;
-            if(row == 0) q[e0 + e] = q[e0 + e] / t[e];
-            else q[e0 + e] = t[e] * (q[e0 + e] - tl * in);
-            in = q[e0 + e];
-            if(row == m - 1) smX[TI + ti] = q[e0 + e];
-          }
+      if(e0 < cu){
+        PS_ROWS(t, r, e0, rc, rlast);
+        #define PS_STEP(e) { \
+          q[e0 + e] = t[e] * (q[e0 + e] - tl * in); \
+          if(e0 + e == 0 && row0 == 0) q[0] = q0d; \
+          in = q[e0 + e]; }
+        if(PS_FULL(e0)){
+          #pragma unroll
+          for(int e = 0; e < PS_PRE; e++) PS_STEP(e)
+        }else{
+          #pragma unroll
+          for(int e = 0; e < PS_PRE; e++) if(e0 + e < cnt) PS_STEP(e)
         }
+        #undef PS_STEP
       }
     }
+    if(cnt > 0 && row0 + cnt == m) smX[TI + ti] = in;   /* q0[n-2] */
   }
   __syncthreads();
   /* backward: q_i -= v_i q_{i+1}, q0[n-2] kept */
@@ -843,22 +888,23 @@ __device__ __forceinline__ void psolve_body(const PSolveArgs & A, D * __restrict
       a = ai * a;
     }
   }else{
+    /* the factor of row m-1 is 0, which keeps q0[n-2] */
     #pragma unroll
     for(int e0 = MAXM - PS_PRE; e0 >= 0; e0 -= PS_PRE){
-      if(e0 < cnt){
-        ps_rows(t, v, ts, row0, e0, jc, m, vc, Q(0.));
-        #pragma unroll
-        for(int e = PS_PRE - 1; e >= 0; e--){
-          if(e0 + e < cnt){
-            const int row = row0 + e0 + e;
-            if(row == m - 1){ a = Q(0.); b = q[e0 + e]; }
-            else {
-              const Q ai = - t[e];
-              b = ai * b + q[e0 + e];
-              a = ai * a;
-            }
-          }
+      if(e0 < cu){
+        PS_ROWS(t, v, e0, vc, Q(0.));
+        #define PS_STEP(e) { \
+          const Q ai = - t[e]; \
+          b = ai * b + q[e0 + e]; \
+          a = ai * a; }
+        if(PS_FULL(e0)){
+          #pragma unroll
+          for(int e = PS_PRE - 1; e >= 0; e--) PS_STEP(e)
+        }else{
+          #pragma unroll
+          for(int e = PS_PRE - 1; e >= 0; e--) if(e0 + e < cnt) PS_STEP(e)
         }
+        #undef PS_STEP
       }
     }
   }
@@ -887,16 +933,19 @@ __device__ __forceinline__ void psolve_body(const PSolveArgs & A, D * __restrict
   }else{
     #pragma unroll
     for(int e0 = MAXM - PS_PRE; e0 >= 0; e0 -= PS_PRE){
-      if(e0 < cnt){
-        ps_rows(t, v, ts, row0, e0, jc, m, vc, Q(0.));
-        #pragma unroll
-        for(int e = PS_PRE - 1; e >= 0; e--){
-          if(e0 + e < cnt){
-            const int row = row0 + e0 + e;
-            if(row != m - 1) q[e0 + e] -= t[e] * in;
-            in = q[e0 + e];
-          }
+      if(e0 < cu){
+        PS_ROWS(t, v, e0, vc, Q(0.));
+        #define PS_STEP(e) { \
+          q[e0 + e] -= t[e] * in; \
+          in = q[e0 + e]; }
+        if(PS_FULL(e0)){
+          #pragma unroll
+          for(int e = PS_PRE - 1; e >= 0; e--) PS_STEP(e)
+        }else{
+          #pragma unroll
+          for(int e = PS_PRE - 1; e >= 0; e--) if(e0 + e < cnt) PS_STEP(e)
         }
+        #undef PS_STEP
       }
     }
   }
@@ -906,22 +955,22 @@ __device__ __forceinline__ void psolve_body(const PSolveArgs & A, D * __restrict
   const Q num = smX[2 * TI + ti] - tu * smX[ti] - tl * smX[TI + ti];
   const Q xl = fabs(double(den)) < DBL_EPSILON ? Q(0.) : num / den;
   if(!valid) return;
+  /* where the halo images of the other index's boundary lie (a uniform offset, 0: none) */
+  long long dimg = 0;
+  if(A.dir == 1){
+    if(other == 1) dimg = (long long)g.nz * g.plane;
+    else if(other == g.nz) dimg = -(long long)g.nz * g.plane;
+  }else{
+    if(other == 1) dimg = (long long)g.ny * g.px;
+    else if(other == g.ny) dimg = -(long long)g.ny * g.px;
+  }
   if constexpr(LEAN){
-    /* interior rows only: no row m, and the halo images are those of the other index (a
-     * uniform offset, when it is at a wall of the period) */
+    /* interior rows only: no row m, and the halo images are those of the other index */
     const __amdgpu_buffer_rsrc_t rq = tck_rsrc_u(q1t, 0xFFFFFFFFu);
     unsigned vd = vel * (unsigned)sizeof(D);
     const unsigned sd = sel * (unsigned)sizeof(D);
     unsigned vu = vel * 8u;
     const unsigned su = sel * 8u;
-    long long dimg = 0;
-    if(A.dir == 1){
-      if(other == 1) dimg = (long long)g.nz * g.plane;
-      else if(other == g.nz) dimg = -(long long)g.nz * g.plane;
-    }else{
-      if(other == 1) dimg = (long long)g.ny * g.px;
-      else if(other == g.ny) dimg = -(long long)g.ny * g.px;
-    }
     const __amdgpu_buffer_rsrc_t rd = tck_rsrc_u(d + w0, 0xFFFFFFFFu);
     const __amdgpu_buffer_rsrc_t rc2 = tck_rsrc_u(ucur ? ucur + w0 : q1t, 0xFFFFFFFFu);
     const __amdgpu_buffer_rsrc_t ro = tck_rsrc_u(uout ? uout + w0 : q1t, 0xFFFFFFFFu);
@@ -986,91 +1035,83 @@ __device__ __forceinline__ void psolve_body(const PSolveArgs & A, D * __restrict
     }
     return;
   }
-  if constexpr(sizeof(Q) == 8){
-    /* FP64: every load of the pass (q1, the old field) before the first store, the results
-     * formed in place in q; then the stores.  A load issued after a store could be waited for
-     * only together with the store. */
-    double ulast = 0.;
-    if(sg == S - 1 && ucur) ulast = ucur[base + step * m];
-    #pragma unroll
-    for(int e0 = 0; e0 < MAXM; e0 += PS_PRE){
-      if(e0 < cnt){
-        Q qq[PS_PRE];
-        double uu[PS_PRE];
+  /* q1 and the old field, PS_PRE rows at a time.  FP64: every load of the pass before the first
+   * store, the results formed in place in q (a load issued after a store could be waited for only
+   * together with the store); the mixed step, whose results are wider than q, stores each group */
+  const __amdgpu_buffer_rsrc_t rq = tck_rsrc_u(q1t, (unsigned)((long long)n * ts * 8));
+  const unsigned vd = vel * (unsigned)sizeof(D), vu = vel * 8u;
+  const unsigned sd = sel * (unsigned)sizeof(D), su = sel * 8u;
+  double ulast = 0.;
+  if(sg == S - 1 && ucur) ulast = ucur[base + step * m];
+  #define PS_OUT(e0, val) { \
+    if(ucur){ \
+      const __amdgpu_buffer_rsrc_t ro = PS_GRP(uout, e0, 8); \
+      _Pragma("unroll") for(int e = 0; e < PS_PRE; e++) if(e0 + e < cnt) tck_bstn<double>(ro, vu, (unsigned)e * su, val); \
+      if(dimg != 0){ \
+        const __amdgpu_buffer_rsrc_t ri = tck_rsrc_u(uout + (w0 + step * (e0) + dimg), ps_bytes(g.n3 - (w0 + step * (e0) + dimg), 8)); \
+        _Pragma("unroll") for(int e = 0; e < PS_PRE; e++) if(e0 + e < cnt) ps_bsti(ri, vu, (unsigned)e * su, val); \
+      } \
+    }else{ \
+      const __amdgpu_buffer_rsrc_t rd = PS_GRP(d, e0, sizeof(D)); \
+      _Pragma("unroll") for(int e = 0; e < PS_PRE; e++) if(e0 + e < cnt) tck_bstn<D>(rd, vd, (unsigned)e * sd, D(val)); \
+    } }
+  double img0 = 0.;   /* row 0's result, for its image past the line's end */
+  #pragma unroll
+  for(int e0 = 0; e0 < MAXM; e0 += PS_PRE){
+    if(e0 < cu){
+      Q qq[PS_PRE];
+      double uu[PS_PRE];
+      #pragma unroll
+      for(int e = 0; e < PS_PRE; e++) qq[e] = Q(tck_bld<double>(rq, vtab, (unsigned)(e0 + e) * stab));
+      if(ucur){
+        const __amdgpu_buffer_rsrc_t rc2 = PS_GRP(ucur, e0, 8);
         #pragma unroll
-        for(int e = 0; e < PS_PRE; e++){
-          const int row = row0 + e0 + e < m ? row0 + e0 + e : m - 1;
-          qq[e] = Q(q1[ts * row]);
-          uu[e] = ucur ? ucur[base + step * row] : 0.;
-        }
+        for(int e = 0; e < PS_PRE; e++) uu[e] = tck_bldn<double>(rc2, vu, (unsigned)e * su);
+      }
+      if constexpr(sizeof(Q) == 8){
         #pragma unroll
         for(int e = 0; e < PS_PRE; e++){
           const Q x = q[e0 + e] + xl * qq[e];
           q[e0 + e] = ucur ? Q(uu[e] + double(x)) : x;
         }
-      }
-    }
-    #pragma unroll
-    for(int e = 0; e < MAXM; e++){
-      if(e < cnt){
-        const int row = row0 + e;
-        if(ucur){
-          const int jj = A.dir == 1 ? 1 + row : other;
-          const int kk = A.dir == 1 ? other : 1 + row;
-          tck_store_halo(uout, g, i, jj, kk, double(q[e]), false);
-        }else{
-          tck_st(&d[base + step * row], D(q[e]));
-        }
-      }
-    }
-    if(sg == S - 1){
-      if(ucur){
-        const int jj = A.dir == 1 ? n : other;
-        const int kk = A.dir == 1 ? other : n;
-        tck_store_halo(uout, g, i, jj, kk, ulast + double(xl), false);
+        if(e0 == 0) img0 = double(q[0]);
       }else{
-        tck_st(&d[base + step * m], D(xl));
-      }
-    }
-    return;
-  }
-  /* q1 and the old field, PS_PRE rows at a time */
-  #pragma unroll
-  for(int e0 = 0; e0 < MAXM; e0 += PS_PRE){
-    if(e0 < cnt){
-      Q qq[PS_PRE];
-      double uu[PS_PRE];
-      #pragma unroll
-      for(int e = 0; e < PS_PRE; e++){
-        const int row = row0 + e0 + e < m ? row0 + e0 + e : m - 1;
-        qq[e] = Q(q1[ts * row]);
-        uu[e] = ucur ? ucur[base + step * row] : 0.;
-      }
-      #pragma unroll
-      for(int e = 0; e < PS_PRE; e++){
-        if(e0 + e < cnt){
-          const int row = row0 + e0 + e;
+        double y[PS_PRE];
+        #pragma unroll
+        for(int e = 0; e < PS_PRE; e++){
           const Q x = q[e0 + e] + xl * qq[e];
-          if(ucur){
-            const int jj = A.dir == 1 ? 1 + row : other;
-            const int kk = A.dir == 1 ? other : 1 + row;
-            tck_store_halo(uout, g, i, jj, kk, uu[e] + double(x), false);
-          }else{
-            tck_st(&d[base + step * row], D(x));
-          }
+          y[e] = ucur ? uu[e] + double(x) : double(x);
         }
+        if(e0 == 0) img0 = y[0];
+        PS_OUT(e0, y[e])
       }
     }
+  }
+  if constexpr(sizeof(Q) == 8){
+    #pragma unroll
+    for(int e0 = 0; e0 < MAXM; e0 += PS_PRE) if(e0 < cu) PS_OUT(e0, double(q[e0 + e]))
+  }
+  if(ucur && row0 == 0 && cnt > 0){
+    uout[base + step * n] = img0;
+    if(dimg != 0) uout[base + step * n + dimg] = img0;
   }
   if(sg == S - 1){
     if(ucur){
-      const int jj = A.dir == 1 ? n : other;
-      const int kk = A.dir == 1 ? other : n;
-      tck_store_halo(uout, g, i, jj, kk, ucur[base + step * m] + double(xl), false);
+      const double y = ulast + double(xl);
+      tck_st(&uout[base + step * m], y);
+      uout[base - step] = y;
+      if(dimg != 0){
+        uout[base + step * m + dimg] = y;
+        uout[base - step + dimg] = y;
+      }
     }else{
       tck_st(&d[base + step * m], D(xl));
     }
   }
+  #undef PS_OUT
+  #undef PS_GRP
+  #undef PS_FULL
+  #undef PS_ROWS
 }
 
 template <typename D, int MAXM>
@@ -1081,7 +1122,7 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) t
    * past the convergence row jc (constant factors; a uniform branch: each form passes the
    * same three barriers) */
   const int m = (A.dir == 1 ? A.g.ny : A.g.nz) - 1;
-  const int seg = (m + A.nsg - 1) / A.nsg;
+  const int seg = ps_seg<D, MAXM>(m, A.nsg);
   const int row0 = (int)threadIdx.y * seg;
   const int i = 1 + blockIdx.x * A.nti + threadIdx.x;
   const int ib0 = A.i0[f], ihi = A.isz[f] > 0 ? ib0 + A.isz[f] - 1 : ib0;
@@ -1349,9 +1390,12 @@ int tck_launch_psolve(const tc_geom_t * g, int dir, int nf, void * const * d, do
   /* the lean form's byte offsets: within a wave (its lanes span at most 64 / TI + 2 segments
    * and TI columns) plus a segment's rows, and the table rows, all below 2^31 */
   const long long step = dir == 1 ? (long long)g->px : g->plane;
-  const long long seg = (m + S - 1) / S;
+  const long long seg = mixed ? (m + S - 1) / S : maxm;
   const long long wspan = ((long long)(64 / TI + 2) * seg + maxm) * step + 64;
   const long long tspan = ((long long)(tcol ? tstride : 1) * (m + 1) + g->px) * 8;
+  /* the other form's: from the first lane's row of a group to the last lane's (grids past this
+   * would not fit in memory) */
+  if(((63 / TI) * seg + PS_PRE) * step * 8 >= (1LL << 32) || tspan >= (1LL << 32)) return (int)hipErrorInvalidValue;
   A.lean = (lean & 2) | ((lean & 1) && wspan * 8 < (1LL << 31) && tspan < (1LL << 31) ? 1 : 0);
   if(mixed) hipLaunchKernelGGL((tck_psolve<float, 2 * PS_MAXM>), grd, dim3(TI, S), lds, stream, A);
   else hipLaunchKernelGGL((tck_psolve<double, PS_MAXM>), grd, dim3(TI, S), lds, stream, A);
