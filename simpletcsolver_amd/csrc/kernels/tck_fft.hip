@@ -30,8 +30,6 @@
 #define FFT_MAXST 16
 #define FFT_EPT 16   /* complex elements per thread per pass */
 #define FFT_MAXTHREADS 1024
-#define FFT_G 4      /* one-tile transforms: divergence elements whose loads are issued together */
-#define FFT_GZ 8     /* one-tile transforms: spectrum elements whose loads are issued together */
 
 /* complex pair of the transform's arithmetic type T (double, or float in the mixed step) */
 template <typename T> struct cvec;
@@ -281,6 +279,157 @@ __device__ void lds_fft(typename cvec<T>::type * buf, int ld, int nb, const FftP
   }
 }
 
+/* The first and last passes with the tile's memory accesses in them.  The inputs of a first
+ * pass's butterfly jj are the elements jj + r M / R, and the outputs of a last pass's the same,
+ * so a thread loads its butterflies' inputs straight into registers and stores the last
+ * pass's results from there: a transform of n passes crosses LDS n - 1 times instead of n + 1.
+ * Butterflies are numbered with the line fastest, so that a row access covers consecutive
+ * lines.  The first pass's twiddle factors are all 1 and are left out; otherwise the operations
+ * are fft_stage's. */
+template <int R, typename T, int EPT, typename LD>
+__device__ __forceinline__ void fft_load_pass(typename cvec<T>::type (*v)[R], int M, int lg, int nbf, T s, int nt, LD load){
+  constexpr int BPT = (EPT + R - 1) / R;
+  const int per = M / R, nb1 = (1 << lg) - 1;
+  #pragma unroll
+  for(int q = 0; q < BPT; q++){
+    const int bf = (int)threadIdx.x + q * nt;
+    #pragma unroll
+    for(int r = 0; r < R; r++) v[q][r] = load(bf & nb1, (bf >> lg) + r * per, bf < nbf);
+  }
+  #pragma unroll
+  for(int q = 0; q < BPT; q++) dftr<R, T>::run(v[q], s);
+}
+
+template <int R, typename T, int EPT, typename LD>
+__device__ __forceinline__ void fft_first_r(typename cvec<T>::type * buf, int M, int ld, int lg, T s, int nt, LD load){
+  constexpr int BPT = (EPT + R - 1) / R;
+  const int nbf = (M / R) << lg, nb1 = (1 << lg) - 1;
+  typename cvec<T>::type v[BPT][R];
+  fft_load_pass<R, T, EPT>(v, M, lg, nbf, s, nt, load);
+  #pragma unroll
+  for(int q = 0; q < BPT; q++){
+    const int bf = (int)threadIdx.x + q * nt;
+    if(bf < nbf){
+      typename cvec<T>::type * dst = buf + (bf & nb1) * ld;
+      const int d0 = (bf >> lg) * R;
+      #pragma unroll
+      for(int r = 0; r < R; r++) dst[fpad(d0 + r)] = v[q][r];
+    }
+  }
+}
+
+template <typename T, int EPT, bool W, typename LD>
+__device__ __forceinline__ void fft_first(typename cvec<T>::type * buf, int ld, int lg, const FftPlan & P, T s, LD load){
+  const int R = P.rad[0];
+  if(R == 8) fft_first_r<8, T, EPT>(buf, P.M, ld, lg, s, P.nt, load);
+  else if(R == 4) fft_first_r<4, T, EPT>(buf, P.M, ld, lg, s, P.nt, load);
+  else if(R == 2) fft_first_r<2, T, EPT>(buf, P.M, ld, lg, s, P.nt, load);
+  else if(W && R == 5) fft_first_r<5, T, EPT>(buf, P.M, ld, lg, s, P.nt, load);
+  else if(W && R == 7) fft_first_r<7, T, EPT>(buf, P.M, ld, lg, s, P.nt, load);
+  else fft_first_r<3, T, EPT>(buf, P.M, ld, lg, s, P.nt, load);
+  fft_pass_barrier();
+}
+
+/* passes st0 .. st1 - 1 in LDS */
+template <typename T, int EPT, bool W>
+__device__ __forceinline__ void fft_mid(typename cvec<T>::type * buf, int ld, int nb, const FftPlan & P,
+    const typename cvec<T>::type * __restrict__ tw, T s, int st0, int st1){
+  int Ns = 1;
+  for(int st = 0; st < st0; st++) Ns *= P.rad[st];
+  for(int st = st0; st < st1; st++){
+    const int R = P.rad[st];
+    const unsigned mp = P.mper[st], mn = P.mns[st];
+    if(R == 8) fft_stage<8, T, EPT>(buf, P.M, ld, nb, Ns, tw, s, mp, mn, P.nt);
+    else if(R == 4) fft_stage<4, T, EPT>(buf, P.M, ld, nb, Ns, tw, s, mp, mn, P.nt);
+    else if(R == 3) fft_stage<3, T, EPT>(buf, P.M, ld, nb, Ns, tw, s, mp, mn, P.nt);
+    else if(W && R == 5) fft_stage<5, T, EPT>(buf, P.M, ld, nb, Ns, tw, s, mp, mn, P.nt);
+    else if(W && R == 7) fft_stage<7, T, EPT>(buf, P.M, ld, nb, Ns, tw, s, mp, mn, P.nt);
+    else if(R == 2) fft_stage<2, T, EPT>(buf, P.M, ld, nb, Ns, tw, s, mp, mn, P.nt);
+    Ns *= R;
+  }
+}
+
+template <int R, typename T, int EPT, typename ST>
+__device__ __forceinline__ void fft_last_r(const typename cvec<T>::type * buf, int M, int ld, int lg,
+    const typename cvec<T>::type * __restrict__ tw, T s, int nt, ST store){
+  typedef typename cvec<T>::type V;
+  constexpr int BPT = (EPT + R - 1) / R;
+  const int per = M / R, nbf = per << lg, nb1 = (1 << lg) - 1;
+  V v[BPT][R];
+  #pragma unroll
+  for(int q = 0; q < BPT; q++){
+    const int bf = (int)threadIdx.x + q * nt;
+    if(bf < nbf){
+      const int jj = bf >> lg;
+      const V * src = buf + (bf & nb1) * ld;
+      #pragma unroll
+      for(int r = 0; r < R; r++){
+        V x = src[fpad(jj + r * per)];
+        if(r > 0){
+          V w = tw[jj * r];
+          if(s > T(0.)) w.y = - w.y;
+          x = cmul(x, w);
+        }
+        v[q][r] = x;
+      }
+      dftr<R, T>::run(v[q], s);
+    }
+  }
+  #pragma unroll
+  for(int q = 0; q < BPT; q++){
+    const int bf = (int)threadIdx.x + q * nt;
+    #pragma unroll
+    for(int r = 0; r < R; r++) store(bf & nb1, (bf >> lg) + r * per, v[q][r], bf < nbf);
+  }
+}
+
+template <typename T, int EPT, bool W, typename ST>
+__device__ __forceinline__ void fft_last(const typename cvec<T>::type * buf, int ld, int lg, const FftPlan & P,
+    const typename cvec<T>::type * __restrict__ tw, T s, ST store){
+  const int R = P.rad[P.nst - 1];
+  if(R == 8) fft_last_r<8, T, EPT>(buf, P.M, ld, lg, tw, s, P.nt, store);
+  else if(R == 4) fft_last_r<4, T, EPT>(buf, P.M, ld, lg, tw, s, P.nt, store);
+  else if(R == 2) fft_last_r<2, T, EPT>(buf, P.M, ld, lg, tw, s, P.nt, store);
+  else if(W && R == 5) fft_last_r<5, T, EPT>(buf, P.M, ld, lg, tw, s, P.nt, store);
+  else if(W && R == 7) fft_last_r<7, T, EPT>(buf, P.M, ld, lg, tw, s, P.nt, store);
+  else fft_last_r<3, T, EPT>(buf, P.M, ld, lg, tw, s, P.nt, store);
+}
+
+/* a transform of one pass (lengths 2, 3, 4, 5, 7 and 8): no LDS at all */
+template <int R, typename T, int EPT, typename LD, typename ST>
+__device__ __forceinline__ void fft_only_r(int M, int lg, T s, int nt, LD load, ST store){
+  constexpr int BPT = (EPT + R - 1) / R;
+  const int per = M / R, nbf = per << lg, nb1 = (1 << lg) - 1;
+  typename cvec<T>::type v[BPT][R];
+  fft_load_pass<R, T, EPT>(v, M, lg, nbf, s, nt, load);
+  #pragma unroll
+  for(int q = 0; q < BPT; q++){
+    const int bf = (int)threadIdx.x + q * nt;
+    #pragma unroll
+    for(int r = 0; r < R; r++) store(bf & nb1, (bf >> lg) + r * per, v[q][r], bf < nbf);
+  }
+}
+
+/* the whole transform of a tile of 1 << lg lines: load(t, n, ok) gives element n of line t (ok
+ * false: any value, from a valid address), store(t, n, v, ok) takes it (ok false: nothing) */
+template <typename T, int EPT, bool W, typename LD, typename ST>
+__device__ __forceinline__ void fft_tile_run(typename cvec<T>::type * buf, int ld, int lg, const FftPlan & P,
+    const typename cvec<T>::type * __restrict__ tw, T s, LD load, ST store){
+  if(P.nst == 1){
+    const int R = P.rad[0];
+    if(R == 8) fft_only_r<8, T, EPT>(P.M, lg, s, P.nt, load, store);
+    else if(R == 4) fft_only_r<4, T, EPT>(P.M, lg, s, P.nt, load, store);
+    else if(R == 2) fft_only_r<2, T, EPT>(P.M, lg, s, P.nt, load, store);
+    else if(W && R == 5) fft_only_r<5, T, EPT>(P.M, lg, s, P.nt, load, store);
+    else if(W && R == 7) fft_only_r<7, T, EPT>(P.M, lg, s, P.nt, load, store);
+    else fft_only_r<3, T, EPT>(P.M, lg, s, P.nt, load, store);
+    return;
+  }
+  fft_first<T, EPT, W>(buf, ld, lg, P, s, load);
+  fft_mid<T, EPT, W>(buf, ld, 1 << lg, P, tw, s, 1, P.nst - 1);
+  fft_last<T, EPT, W>(buf, ld, lg, P, tw, s, store);
+}
+
 __constant__ double c_fft_rka[3] = {32. / 60., 25. / 60., 45. / 60.};
 __constant__ double c_fft_rkb[3] = { 0. / 60., -17. / 60., -25. / 60.};
 
@@ -308,13 +457,75 @@ struct YFwdArgs {
 
 /* the divergence is formed in FP64 (assign_input :404-423) and rounded to the transform
  * type T only when it enters the transform */
-template <typename T, bool W>
-__global__ void __launch_bounds__(FFT_MAXTHREADS) tck_div_yfft(const YFwdArgs A){
+/* the first pass of a tile: packed element n of a line is the divergence at rows 2 n + 1 and
+ * 2 n + 2, whose common face is read once; GD elements' loads are issued together (out-of-field
+ * elements read cell (1, 1) of the plane and are put as 0, so that no load is conditional) */
+template <int R, typename T, int EPT, int GD>
+__device__ __forceinline__ void div_first_r(typename cvec<T>::type * buf, const YFwdArgs & A, int i0, int k, double prefactor){
+  typedef typename cvec<T>::type V;
+  constexpr int BPT = (EPT + R - 1) / R;
+  const tc_geom_t & g = A.g;
+  const tc_coef_t & c = A.c;
+  const int lg = fft_lg(A.ti), nt = A.P.nt;
+  const int per = A.P.M / R, nbf = per << lg;
+  const long long sy = g.px, sz = g.plane;
+  V v[BPT][R];
+  #pragma unroll
+  for(int q = 0; q < BPT; q++){
+    const int bf = (int)threadIdx.x + q * nt;
+    const int i = i0 + (bf & (A.ti - 1)), jj = bf >> lg;
+    const bool ok = bf < nbf && i <= g.nx;
+    const int ii = ok ? i : 1;
+    #pragma unroll
+    for(int r0 = 0; r0 < R; r0 += GD){
+      /* one batch of loads at a time: more would not fit in registers beside v */
+      asm volatile("" ::: "memory");
+      double P[GD][11];
+      #pragma unroll
+      for(int u = 0; u < GD; u++) if(r0 + u < R){
+        const long long o = tck_idx(g, ii, ok ? 2 * (jj + (r0 + u) * per) + 1 : 1, k);
+        P[u][0] = A.ux[o]; P[u][1] = A.ux[o + 1]; P[u][2] = A.ux[o + sy]; P[u][3] = A.ux[o + sy + 1];
+        P[u][4] = A.uy[o]; P[u][5] = A.uy[o + sy]; P[u][6] = A.uy[o + 2 * sy];
+        P[u][7] = A.uz[o]; P[u][8] = A.uz[o + sz]; P[u][9] = A.uz[o + sy]; P[u][10] = A.uz[o + sy + sz];
+      }
+      #pragma unroll
+      for(int u = 0; u < GD; u++) if(r0 + u < R){
+        const double d0 = c.ijdxc[ii] * (
+            - c.jhxf[ii] * P[u][0] + c.jhxf[ii + 1] * P[u][1]
+            - c.jhyc[ii] * P[u][4] + c.jhyc[ii] * P[u][5]
+            - c.jhzc[ii] * P[u][7] + c.jhzc[ii] * P[u][8]);
+        const double d1 = c.ijdxc[ii] * (
+            - c.jhxf[ii] * P[u][2] + c.jhxf[ii + 1] * P[u][3]
+            - c.jhyc[ii] * P[u][5] + c.jhyc[ii] * P[u][6]
+            - c.jhzc[ii] * P[u][9] + c.jhzc[ii] * P[u][10]);
+        v[q][r0 + u] = mk2<T>(ok ? T(prefactor * d0) : T(0.), ok ? T(prefactor * d1) : T(0.));
+        asm volatile("" : "+v"(v[q][r0 + u].x), "+v"(v[q][r0 + u].y));
+      }
+    }
+  }
+  #pragma unroll
+  for(int q = 0; q < BPT; q++){
+    dftr<R, T>::run(v[q], T(-1.));
+    const int bf = (int)threadIdx.x + q * nt;
+    if(bf < nbf){
+      V * dst = buf + (bf & (A.ti - 1)) * A.ld;
+      const int d0 = (bf >> lg) * R;
+      #pragma unroll
+      for(int r = 0; r < R; r++) dst[fpad(d0 + r)] = v[q][r];
+    }
+  }
+}
+
+/* NTMAX, the block size the kernel is compiled for, sets how many elements' loads are issued at a
+ * time beside the pass's registers: 1024 two (four in FP32), 512 three (at four waves per SIMD),
+ * 256 all eight, for launches of so few waves that their latency is what counts */
+template <typename T, int EPT, bool W, int NTMAX>
+__global__ void __launch_bounds__(NTMAX) tck_div_yfft(const YFwdArgs A){
+  constexpr int GD = NTMAX == 256 ? 8 : (sizeof(T) == 4 ? 4 : (NTMAX == 512 ? 3 : 2));
   typedef typename cvec<T>::type V;
   extern __shared__ __align__(16) unsigned char fft_smem[];
   V * sm = (V *)fft_smem;
   const tc_geom_t & g = A.g;
-  const tc_coef_t & c = A.c;
   const int ti = A.ti;
   const int M = A.P.M;
   const int ntx = (g.nx + ti - 1) / ti;
@@ -325,43 +536,17 @@ __global__ void __launch_bounds__(FFT_MAXTHREADS) tck_div_yfft(const YFwdArgs A)
   const double gamma = c_fft_rka[A.rkstep] + c_fft_rkb[A.rkstep];
   const double norm = 1. * g.ny * g.nz;
   const double prefactor = 1. / (gamma * dt) / norm;
-  const long long sy = g.px;
-  const long long sz = g.plane;
   const V * twM = (const V *)A.twM;
   const V * twN = (const V *)A.twN;
-  /* divergence packed as z_m = x_2m + i x_2m+1; the velocities of FFT_G elements are loaded
-   * together (out-of-field elements read cell (1, 1) of the plane and are put as 0, so that no
-   * load is conditional) */
-  const int nel = ti * g.ny;
-  for(int e0 = threadIdx.x; e0 < nel; e0 += FFT_G * A.P.nt){
-    double P[FFT_G][6];
-    #pragma unroll
-    for(int u = 0; u < FFT_G; u++){
-      const int e = e0 + u * A.P.nt;
-      const int t = (e & (ti - 1)), j0 = (e >> fft_lg(ti)), i = i0 + t;
-      const bool ok = e < nel && i <= g.nx;
-      const long long o = tck_idx(g, ok ? i : 1, ok ? j0 + 1 : 1, k);
-      P[u][0] = A.ux[o]; P[u][1] = A.ux[o + 1]; P[u][2] = A.uy[o]; P[u][3] = A.uy[o + sy];
-      P[u][4] = A.uz[o]; P[u][5] = A.uz[o + sz];
-    }
-    #pragma unroll
-    for(int u = 0; u < FFT_G; u++){
-      const int e = e0 + u * A.P.nt;
-      if(e >= nel) break;
-      const int t = (e & (ti - 1)), j0 = (e >> fft_lg(ti)), i = i0 + t;
-      double val = 0.;
-      if(i <= g.nx){
-        const double div = c.ijdxc[i] * (
-            - c.jhxf[i] * P[u][0] + c.jhxf[i + 1] * P[u][1]
-            - c.jhyc[i] * P[u][2] + c.jhyc[i] * P[u][3]
-            - c.jhzc[i] * P[u][4] + c.jhzc[i] * P[u][5]);
-        val = prefactor * div;
-      }
-      ((T *)(sm + t * A.ld))[2 * fpad(j0 >> 1) + (j0 & 1)] = T(val);
-    }
-  }
-  __syncthreads();
-  lds_fft<T, FFT_EPT, W>(sm, A.ld, ti, A.P, twM, T(-1.));
+  const int R = A.P.rad[0];
+  if(R == 8) div_first_r<8, T, EPT, GD>(sm, A, i0, k, prefactor);
+  else if(R == 4) div_first_r<4, T, EPT, GD>(sm, A, i0, k, prefactor);
+  else if(R == 2) div_first_r<2, T, EPT, GD>(sm, A, i0, k, prefactor);
+  else if(W && R == 5) div_first_r<5, T, EPT, GD>(sm, A, i0, k, prefactor);
+  else if(W && R == 7) div_first_r<7, T, EPT, GD>(sm, A, i0, k, prefactor);
+  else div_first_r<3, T, EPT, GD>(sm, A, i0, k, prefactor);
+  fft_pass_barrier();
+  fft_mid<T, EPT, W>(sm, A.ld, ti, A.P, twM, T(-1.), 1, A.P.nst);
   /* split: X_k = (Z_k + conj Z_{M-k}) / 2 - i W^k (Z_k - conj Z_{M-k}) / 2, k = 0..M */
   V * S = (V *)A.S;
   for(int e = threadIdx.x; e < ti * (M + 1); e += A.P.nt){
@@ -579,45 +764,22 @@ struct ZArgs {
 };
 
 /* one block per tile of tz consecutive i at one ky */
-template <typename T, bool W>
+template <typename T, int EPT, bool W>
 __global__ void __launch_bounds__(FFT_MAXTHREADS) tck_zfft(const ZArgs A){
   typedef typename cvec<T>::type V;
   extern __shared__ __align__(16) unsigned char fft_smem[];
   V * sm = (V *)fft_smem;
   const int tz = A.tz;
-  const int nz = A.nz;
   const int ntx = (A.nx + tz - 1) / tz;
   const long long tile = fft_tile_of((long long)ntx * A.nky);
   const int i0 = (int)(tile % ntx) * tz;
   const int ky = (int)(tile / ntx);
   const long long kstride = (long long)A.nx * A.nky;
-  V * base = (V *)A.S + (long long)A.nx * ky;
-  /* FFT_GZ elements loaded together; out-of-range ones read element 0 and are put as 0 */
-  const int nel = tz * nz;
-  for(int e0 = threadIdx.x; e0 < nel; e0 += FFT_GZ * A.P.nt){
-    V v[FFT_GZ];
-    #pragma unroll
-    for(int u = 0; u < FFT_GZ; u++){
-      const int e = e0 + u * A.P.nt;
-      const int t = (e & (tz - 1)), kz = (e >> fft_lg(tz)), ii = i0 + t;
-      v[u] = tck_ld((e < nel && ii < A.nx) ? &base[ii + kstride * kz] : (const V *)A.S);
-    }
-    #pragma unroll
-    for(int u = 0; u < FFT_GZ; u++){
-      const int e = e0 + u * A.P.nt;
-      if(e >= nel) break;
-      const int t = (e & (tz - 1)), kz = (e >> fft_lg(tz));
-      sm[t * A.ld + fpad(kz)] = i0 + t < A.nx ? v[u] : mk2<T>(T(0.), T(0.));
-    }
-  }
-  __syncthreads();
-  lds_fft<T, FFT_EPT, W>(sm, A.ld, tz, A.P, (const V *)A.tw, T(A.sign));
-  for(int e = threadIdx.x; e < tz * nz; e += A.P.nt){
-    const int t = (e & (tz - 1));
-    const int kz = (e >> fft_lg(tz));
-    const int ii = i0 + t;
-    if(ii < A.nx) tck_st(&base[ii + kstride * kz], sm[t * A.ld + fpad(kz)]);
-  }
+  V * base = (V *)A.S + (long long)A.nx * ky + i0;
+  const int nl = A.nx - i0;   /* lines of this tile inside the spectrum */
+  fft_tile_run<T, EPT, W>(sm, A.ld, fft_lg(tz), A.P, (const V *)A.tw, T(A.sign),
+      [&](int t, int kz, bool ok){ return tck_ld(ok && t < nl ? &base[t + kstride * kz] : (const V *)A.S); },
+      [&](int t, int kz, V v, bool ok){ if(ok && t < nl) tck_st(&base[t + kstride * kz], v); });
 }
 
 /* Persistent form: each block loops over tiles and issues the loads of the first PF of its
@@ -788,81 +950,82 @@ __device__ __forceinline__ V c2r_pre(V xk, V xmk, V w){
   return r;
 }
 
-template <typename T, bool W>
+template <typename T, int EPT, bool W>
 __global__ void __launch_bounds__(FFT_MAXTHREADS) tck_yifft_psi(const YInvArgs A){
   typedef typename cvec<T>::type V;
   extern __shared__ __align__(16) unsigned char fft_smem[];
   V * sm = (V *)fft_smem;
   const tc_geom_t & g = A.g;
-  const int ti = A.ti;
+  const int ti = A.ti, lg = fft_lg(ti);
   const int M = A.P.M;
   const int ntx = (g.nx + ti - 1) / ti;
   const long long tile = fft_tile_of((long long)ntx * g.nz);
   const int i0 = 1 + (int)(tile % ntx) * ti;
   const int k = 1 + (int)(tile / ntx);
-  const long long rowbase = (long long)g.nx * (long long)A.nky * (k - 1);
+  const int nl = g.nx + 1 - i0;   /* lines of this tile inside the field */
   const V * S = (const V *)A.S;
+  const V * row = S + (long long)g.nx * (long long)A.nky * (k - 1) + (i0 - 1);
   const V * twN = (const V *)A.twN;
-  /* load X_1..X_{M-1}; Z'_0 needs X_0 and X_M only and is formed here.  FFT_GZ elements are
-   * loaded together (with X_M for a kk = 0 element); out-of-field elements read element 0 and
-   * are put as 0 */
-  const int nel = ti * M;
-  for(int e0 = threadIdx.x; e0 < nel; e0 += FFT_GZ * A.P.nt){
-    V v[FFT_GZ], xm[FFT_GZ];
+  /* Z'_k and Z'_{M-k} from X_k and X_{M-k}, k = 1..M/2, put in LDS as they are formed: EPT / 2
+   * pairs per thread, whose loads are issued together; and Z'_0 from X_0 and X_M by the first
+   * ti threads */
+  constexpr int GP = EPT / 2;
+  const int npair = (M / 2) * ti;
+  const bool ok0 = (int)threadIdx.x < ti && (int)threadIdx.x < nl;
+  V x0 = tck_ld(ok0 ? &row[threadIdx.x] : S), xm = tck_ld(ok0 ? &row[threadIdx.x + (long long)g.nx * M] : S);
+  for(int e0 = threadIdx.x; e0 < npair; e0 += GP * A.P.nt){
+    V xa[GP], xb[GP];
     #pragma unroll
-    for(int u = 0; u < FFT_GZ; u++){
+    for(int u = 0; u < GP; u++){
       const int e = e0 + u * A.P.nt;
-      const int t = (e & (ti - 1)), kk = (e >> fft_lg(ti)), i = i0 + t;
-      const bool ok = e < nel && i <= g.nx;
-      const long long o = (long long)(i - 1) + rowbase;
-      v[u] = tck_ld(ok ? &S[o + (long long)g.nx * kk] : S);
-      xm[u] = tck_ld((ok && kk == 0) ? &S[o + (long long)g.nx * M] : S);
+      const int t = e & (ti - 1), k1 = 1 + (e >> lg);
+      const bool ok = e < npair && t < nl;
+      xa[u] = tck_ld(ok ? &row[t + (long long)g.nx * k1] : S);
+      xb[u] = tck_ld(ok ? &row[t + (long long)g.nx * (M - k1)] : S);
     }
     #pragma unroll
-    for(int u = 0; u < FFT_GZ; u++){
+    for(int u = 0; u < GP; u++){
       const int e = e0 + u * A.P.nt;
-      if(e >= nel) break;
-      const int t = (e & (ti - 1)), kk = (e >> fft_lg(ti)), i = i0 + t;
-      V w = mk2<T>(T(0.), T(0.));
-      if(i <= g.nx){
-        w = v[u];
-        if(kk == 0){
-          V x0 = v[u], xmm = xm[u];
-          x0.y = T(0.);
-          xmm.y = T(0.);
-          w = c2r_pre(x0, xmm, twN[0]);
-        }
-      }
-      sm[t * A.ld + fpad(kk)] = w;
+      if(e >= npair) break;
+      const int t = e & (ti - 1), k1 = 1 + (e >> lg), k2 = M - k1;
+      const V z1 = c2r_pre(xa[u], xb[u], twN[k1]);
+      if(k2 != k1) sm[t * A.ld + fpad(k2)] = c2r_pre(xb[u], xa[u], twN[k2]);
+      sm[t * A.ld + fpad(k1)] = z1;
     }
   }
-  __syncthreads();
-  /* pairs (k, M-k), k = 1..M/2, in place */
-  const int half = M / 2;
-  for(int e = threadIdx.x; e < ti * half; e += A.P.nt){
-    const int t = (e & (ti - 1));
-    const int k1 = 1 + (e >> fft_lg(ti));
-    const int k2 = M - k1;
-    const V xa = sm[t * A.ld + fpad(k1)];
-    const V xb = sm[t * A.ld + fpad(k2)];
-    const V z1 = c2r_pre(xa, xb, twN[k1]);
-    if(k2 != k1){
-      const V z2 = c2r_pre(xb, xa, twN[k2]);
-      sm[t * A.ld + fpad(k2)] = z2;
+  if((int)threadIdx.x < ti){
+    x0.y = T(0.);
+    xm.y = T(0.);
+    sm[threadIdx.x * A.ld + fpad(0)] = c2r_pre(x0, xm, twN[0]);
+  }
+  fft_lds_barrier();
+  /* element n of a line is psi at rows 2 n + 1 and 2 n + 2.  A thread's line is the same for all
+   * its butterflies (the block size is a multiple of the tile width), so its wall copy is one
+   * offset, and the z image of the first and last planes a uniform one; the y images are those
+   * of elements 0 and M - 1 */
+  const int i = i0 + ((int)threadIdx.x & (ti - 1));
+  T * col = (T *)A.psi + tck_idx(g, i, 0, k);
+  const int wall = i == 1 ? -1 : (i == g.nx ? 1 : 0);
+  const long long dk = k == 1 ? g.plane * g.nz : (k == g.nz ? - g.plane * g.nz : 0);
+  const auto put = [&](int j, T v){
+    T * p = col + (long long)g.px * j;
+    tck_st(p, v);
+    if(wall) p[wall] = v;
+    if(dk){
+      p[dk] = v;
+      if(wall) p[dk + wall] = v;
     }
-    sm[t * A.ld + fpad(k1)] = z1;
-  }
-  __syncthreads();
-  lds_fft<T, FFT_EPT, W>(sm, A.ld, ti, A.P, (const V *)A.twM, T(1.));
-  T * psi = (T *)A.psi;
-  for(int e = threadIdx.x; e < ti * g.ny; e += A.P.nt){
-    const int t = (e & (ti - 1));
-    const int jj = (e >> fft_lg(ti));
-    const int i = i0 + t;
-    if(i > g.nx) continue;
-    const T v = ((const T *)(sm + t * A.ld))[2 * fpad(jj >> 1) + (jj & 1)];
-    tck_store_halo(psi, g, i, jj + 1, k, v, true);
-  }
+  };
+  const auto store = [&](int t, int n, V v, bool ok){
+    if(ok && t < nl){
+      put(2 * n + 1, v.x);
+      put(2 * n + 2, v.y);
+      if(n == 0) put(g.ny + 1, v.x);
+      if(n == M - 1) put(0, v.y);
+    }
+  };
+  fft_mid<T, EPT, W>(sm, A.ld, ti, A.P, (const V *)A.twM, T(1.), 0, A.P.nst - 1);
+  fft_last<T, EPT, W>(sm, A.ld, lg, A.P, (const V *)A.twM, T(1.), store);
 }
 
 /* Persistent form of tck_yifft_psi (compiled for EPTK elements per thread per pass): each
@@ -1169,7 +1332,7 @@ static int fft_ncu(void){
 /* share: tiles sized to leave room for `share` blocks per CU in the LDS (while at least 4
  * transforms, 64 B of contiguous FP64 complex values, remain per row access).  lines: the
  * transforms of the launch; small launches take narrower tiles, so that there are at least
- * two blocks per CU */
+ * two blocks per CU, while a tile keeps 16 butterflies of 8 (a thread takes whole ones) */
 /* LDS pitch of one padded line of M elements, odd so that the rows of a tile start in
  * different banks */
 static int fft_ld(int M){
@@ -1185,16 +1348,17 @@ static int fft_tile(int M, int cap, size_t csize, int * threads, int share, long
   while(b > 1 && ((size_t)b * lb > lds_limit() || b * M > FFT_EPT * FFT_MAXTHREADS)) b /= 2;
   while(share > 1 && b > 4 && (size_t)b * lb * share > lds_limit()) b /= 2;
   while(b * 2 <= cap && b * 2 * M <= FFT_EPT * 64) b *= 2;   /* short transforms: wider tiles */
-  while(b > 1 && lines / b < 2LL * fft_ncu()) b /= 2;
+  while(b > 1 && b * M > 128 && lines / b < 2LL * fft_ncu()) b /= 2;
   if(b > cap) b = cap < 1 ? 1 : cap;
   /* elements per thread: FFT_EPT, or half that where the LDS holds so few blocks per CU that
    * FFT_EPT would leave fewer than 16 waves on it (FP64 tiles of long transforms: one block
-   * per CU).  The device passes loop over their butterflies, so any count up to FFT_EPT
+   * per CU), and for every FP64 tile, whose 16 elements do not fit in a thread's registers
+   * beside a pass that loads or stores them.  The device passes loop over their butterflies, so any count up to FFT_EPT
    * computes the same bits. */
   int ept = FFT_EPT;
   const long long per = (long long)(lds_limit() / ((size_t)b * lb));
   const int w16 = ((b * M + FFT_EPT - 1) / FFT_EPT + 63) / 64;
-  if(TCK_FFT_HALFEPT && per * w16 < 16 && (b * M + FFT_EPT / 2 - 1) / (FFT_EPT / 2) <= FFT_MAXTHREADS) ept = FFT_EPT / 2;
+  if(TCK_FFT_HALFEPT && (csize == sizeof(double2) || per * w16 < 16) && (b * M + FFT_EPT / 2 - 1) / (FFT_EPT / 2) <= FFT_MAXTHREADS) ept = FFT_EPT / 2;
   int t = (b * M + ept - 1) / ept;
   t = (t + 63) / 64 * 64;
   if(t < 64) t = 64;
@@ -1269,13 +1433,13 @@ static int launch_persistent(void (*kern)(const Args), const Args & A, int nt, s
 
 extern "C" {
 
-/* the one-tile form of kernel K for the transform type (float when mixed) and radix set;
- * nonzero when the LDS limit could not be raised */
-#define FFT_ONE(K, mixed, wide) ( \
-  (mixed) ? ((wide) ? fft_one((const void *)K<float, true>, [&]{ hipLaunchKernelGGL((K<float, true>), grd, dim3(nt), lds, stream, A); }, lds) \
-                    : fft_one((const void *)K<float, false>, [&]{ hipLaunchKernelGGL((K<float, false>), grd, dim3(nt), lds, stream, A); }, lds)) \
-          : ((wide) ? fft_one((const void *)K<double, true>, [&]{ hipLaunchKernelGGL((K<double, true>), grd, dim3(nt), lds, stream, A); }, lds) \
-                    : fft_one((const void *)K<double, false>, [&]{ hipLaunchKernelGGL((K<double, false>), grd, dim3(nt), lds, stream, A); }, lds)))
+/* the one-tile form of kernel K, compiled for E elements per thread per pass, for the transform
+ * type (float when mixed) and radix set; nonzero when the LDS limit could not be raised */
+#define FFT_ONE_E(K, E, mixed, wide) ( \
+  (mixed) ? ((wide) ? fft_one((const void *)K<float, E, true>, [&]{ hipLaunchKernelGGL((K<float, E, true>), grd, dim3(nt), lds, stream, A); }, lds) \
+                    : fft_one((const void *)K<float, E, false>, [&]{ hipLaunchKernelGGL((K<float, E, false>), grd, dim3(nt), lds, stream, A); }, lds)) \
+          : ((wide) ? fft_one((const void *)K<double, E, true>, [&]{ hipLaunchKernelGGL((K<double, E, true>), grd, dim3(nt), lds, stream, A); }, lds) \
+                    : fft_one((const void *)K<double, E, false>, [&]{ hipLaunchKernelGGL((K<double, E, false>), grd, dim3(nt), lds, stream, A); }, lds)))
 
 /* mixed: spectrum, transforms and psi in FP32 (twiddles twM, twN, tw as float2) */
 int tck_launch_div_yfft(const tc_geom_t * g, const tc_coef_t * c, const double * ux,
@@ -1315,7 +1479,20 @@ int tck_launch_div_yfft(const tc_geom_t * g, const tc_coef_t * c, const double *
   }
 #endif
   const dim3 grd((unsigned)ntiles);
-  if(FFT_ONE(tck_div_yfft, mixed, plan_wide(&A.P))) return (int)hipErrorInvalidValue;
+  const long long el = (long long)A.ti * A.P.M;
+  const bool wide = plan_wide(&A.P);
+  if(mixed && (el + FFT_EPT / 2 - 1) / (FFT_EPT / 2) <= FFT_MAXTHREADS){
+    nt = (int)(((el + FFT_EPT / 2 - 1) / (FFT_EPT / 2) + 63) / 64 * 64);
+    A.P.nt = nt;
+  }
+  const bool half = (long long)nt * (FFT_EPT / 2) >= el;
+  /* at most two waves per SIMD */
+  const bool few = nt <= 256 && ntiles * (nt / 64) <= 8LL * fft_ncu();
+  #define DIV_ONE(T, E, W, N) fft_one((const void *)tck_div_yfft<T, E, W, N>, [&]{ hipLaunchKernelGGL((tck_div_yfft<T, E, W, N>), grd, dim3(nt), lds, stream, A); }, lds)
+  #define DIV_N(T, W) (half ? (few ? DIV_ONE(T, FFT_EPT / 2, W, 256) : nt <= 512 ? DIV_ONE(T, FFT_EPT / 2, W, 512) : DIV_ONE(T, FFT_EPT / 2, W, FFT_MAXTHREADS)) : DIV_ONE(T, FFT_EPT, W, FFT_MAXTHREADS))
+  if(mixed ? (wide ? DIV_N(float, true) : DIV_N(float, false)) : (wide ? DIV_N(double, true) : DIV_N(double, false))) return (int)hipErrorInvalidValue;
+  #undef DIV_N
+  #undef DIV_ONE
   TCK_CHECK_LAUNCH();
   return 0;
 }
@@ -1352,7 +1529,8 @@ int tck_launch_zfft(int nx, int nky, int nz, void * S, const void * tw, int sign
   }
 #endif
   const dim3 grd((unsigned)ntiles);
-  if(FFT_ONE(tck_zfft, mixed, plan_wide(&A.P))) return (int)hipErrorInvalidValue;
+  const bool half = (long long)nt * (FFT_EPT / 2) >= (long long)A.tz * nz;
+  if(half ? FFT_ONE_E(tck_zfft, FFT_EPT / 2, mixed, plan_wide(&A.P)) : FFT_ONE_E(tck_zfft, FFT_EPT, mixed, plan_wide(&A.P))) return (int)hipErrorInvalidValue;
   TCK_CHECK_LAUNCH();
   return 0;
 }
@@ -1396,7 +1574,8 @@ int tck_launch_yifft_psi(const tc_geom_t * g, const void * S, void * psi, const 
   }
 #endif
   const dim3 grd((unsigned)ntiles);
-  if(FFT_ONE(tck_yifft_psi, mixed, plan_wide(&A.P))) return (int)hipErrorInvalidValue;
+  const bool half = (long long)nt * (FFT_EPT / 2) >= (long long)A.ti * A.P.M;
+  if(half ? FFT_ONE_E(tck_yifft_psi, FFT_EPT / 2, mixed, plan_wide(&A.P)) : FFT_ONE_E(tck_yifft_psi, FFT_EPT, mixed, plan_wide(&A.P))) return (int)hipErrorInvalidValue;
   TCK_CHECK_LAUNCH();
   return 0;
 }
