@@ -90,7 +90,7 @@ struct tc_solver_s {
   tc_prof_t prof[TC_NSTAGE];
   int tune[TC_NTUNE][2];
   int predict_window;     /* 1: the predictor variant with the fields' planes staged in LDS */
-  int fft_exact;          /* forms of the persistent transforms where they apply: 1 axial exact, 2 divergence twiddles in LDS, 4 inverse theta exact */
+  int fft_exact;          /* persistent transforms where they apply: 1 axial, 4 inverse theta (2 has no effect) */
   int psolve_lean;        /* periodic line solves: 1 interior waves skip the row tests, 2 batched LDS folds */
   /* bumped by every host-side change that work recorded earlier (an ensemble's graphs)
    * cannot see: fields replaced, a closure coupled, uncoupled or destroyed, launch shapes,

@@ -888,7 +888,7 @@ static int potential(tc_solver_t * s, int rkstep){
   const int mx = s->mixed;
   void * psi = mx ? (void *)s->d_psi32 : (void *)s->d_psi;
   PROF(TC_S_DIVY, tck_launch_div_yfft(g, &s->coef, tc_field_ptr(s, TC_FUX), tc_field_ptr(s, TC_FUY),
-      tc_field_ptr(s, TC_FUZ), s->d_dt, rkstep, s->d_spec, s->d_twy, s->d_twyn, mx, s->fft_exact & 2, s->stream));
+      tc_field_ptr(s, TC_FUZ), s->d_dt, rkstep, s->d_spec, s->d_twy, s->d_twyn, mx, s->stream));
   PROF(TC_S_ZFFT, tck_launch_zfft(g->nx, s->nky, g->nz, s->d_spec, s->d_twz, -1, mx, s->fft_exact & 1, s->stream));
   PROF(TC_S_PXSOLVE, tck_launch_pxsolve(g->nx, s->nky * g->nz, s->d_spec, s->d_pr, s->d_pl, s->d_pu, mx, s->stream));
   PROF(TC_S_ZFFT, tck_launch_zfft(g->nx, s->nky, g->nz, s->d_spec, s->d_twz, +1, mx, s->fft_exact & 1, s->stream));
@@ -1159,11 +1159,11 @@ int tc_dissipation(tc_solver_t * s, double out[2]){
 
 /* launch shapes of the cell kernels ("predict", "correct"): planes per block and j rows per
  * block; results do not depend on them.  "predict_window" (kb 0 or 1) switches between forms
- * of the predictor, "fft_exact" (kb a mask: 1 the axial transforms, 2 the divergence + theta
- * transform's twiddles in LDS, 4 the inverse theta transform) between forms of the persistent
- * transforms, "psolve_lean" (kb a mask: 1 the periodic line solves' interior waves skip the row
- * tests, 2 their folds read LDS four segments at a time; default 3) between forms of the
- * periodic line solves; each pair computes the same bits */
+ * of the predictor, "fft_exact" (kb a mask: 1 the axial transforms, 4 the inverse theta
+ * transform; 2 is accepted and has no effect: the divergence + theta transform has one form)
+ * between the persistent and the one-tile transforms, "psolve_lean" (kb a mask: 1 the periodic
+ * line solves' interior waves skip the row tests, 2 their folds read LDS four segments at a
+ * time; default 3) between forms of the periodic line solves; each pair computes the same bits */
 int tc_tune_set(tc_solver_t * s, const char * kernel, int kb, int ty){
   if(kernel && strcmp(kernel, "predict_window") == 0){
     s->predict_window = kb ? 1 : 0;

@@ -13,10 +13,13 @@
  *  tck_zfft       complex axial transforms, forward or backward, in place.
  *  tck_yifft_psi  complex-to-real theta transform fused with extract_output (:427-443): psi
  *                 with its periodic halos and Neumann wall copies (boundary/psi.c:13-45).
- * Each has a persistent form (suffix _p) for FP64 tiles of long transforms: a block loops
- * over tiles and issues part of the next tile's loads before the current tile's LDS passes.
- * Tiles whose LDS leaves few blocks per CU run with half the elements per thread (twice the
- * threads), so that a CU still holds 16 waves.  Every form computes the same bits.
+ * The first pass of a tile takes its butterflies from memory and the last pass stores from
+ * registers, so a tile crosses LDS only between passes (tck_div_yfft's split and
+ * tck_yifft_psi's pairing each add one crossing).  tck_zfft and tck_yifft_psi have a persistent
+ * form (suffix _p) for launches whose tiles cover the data exactly: a block loops over tiles and
+ * issues the next tile's loads before the current tile's passes.  Tiles whose LDS leaves few
+ * blocks per CU run with half the elements per thread (twice the threads), so that a CU still
+ * holds 16 waves.  Every form computes the same bits.
  * Transforms are unnormalised, as FFTW's; the imaginary parts of the DC and Nyquist bins are
  * ignored by the complex-to-real transform, as FFTW's c2r does with a Hermitian input.
  *
@@ -258,27 +261,6 @@ __device__ __forceinline__ void fft_stage(typename cvec<T>::type * buf, int M, i
   fft_pass_barrier();
 }
 
-/* nb transforms of length P.M stored at buf + b * ld; tw[t] = exp(-2 pi i t / M); each pass
- * keeps at most EPT elements per thread in registers, so blockDim.x * EPT >= nb * P.M.  W:
- * the plan may hold radix 5 and 7 passes (compiled only into the kernels of such lengths, so
- * that the 2^a 3^b kernels keep their register budget) */
-template <typename T, int EPT = FFT_EPT, bool W = false>
-__device__ void lds_fft(typename cvec<T>::type * buf, int ld, int nb, const FftPlan & P,
-    const typename cvec<T>::type * __restrict__ tw, T s){
-  int Ns = 1;
-  for(int st = 0; st < P.nst; st++){
-    const int R = P.rad[st];
-    const unsigned mp = P.mper[st], mn = P.mns[st];
-    if(R == 8) fft_stage<8, T, EPT>(buf, P.M, ld, nb, Ns, tw, s, mp, mn, P.nt);
-    else if(R == 4) fft_stage<4, T, EPT>(buf, P.M, ld, nb, Ns, tw, s, mp, mn, P.nt);
-    else if(R == 3) fft_stage<3, T, EPT>(buf, P.M, ld, nb, Ns, tw, s, mp, mn, P.nt);
-    else if(W && R == 5) fft_stage<5, T, EPT>(buf, P.M, ld, nb, Ns, tw, s, mp, mn, P.nt);
-    else if(W && R == 7) fft_stage<7, T, EPT>(buf, P.M, ld, nb, Ns, tw, s, mp, mn, P.nt);
-    else if(R == 2) fft_stage<2, T, EPT>(buf, P.M, ld, nb, Ns, tw, s, mp, mn, P.nt);
-    Ns *= R;
-  }
-}
-
 /* The first and last passes with the tile's memory accesses in them.  The inputs of a first
  * pass's butterfly jj are the elements jj + r M / R, and the outputs of a last pass's the same,
  * so a thread loads its butterflies' inputs straight into registers and stores the last
@@ -331,6 +313,10 @@ __device__ __forceinline__ void fft_first(typename cvec<T>::type * buf, int ld, 
 }
 
 /* passes st0 .. st1 - 1 in LDS */
+/* passes st0..st1 - 1 of nb transforms of length P.M stored at buf + b * ld; tw[t] =
+ * exp(-2 pi i t / M); each pass keeps at most EPT elements per thread in registers, so
+ * P.nt * EPT >= nb * P.M.  W: the plan may hold radix 5 and 7 passes (compiled only into the
+ * kernels of such lengths, so that the 2^a 3^b kernels keep their register budget) */
 template <typename T, int EPT, bool W>
 __device__ __forceinline__ void fft_mid(typename cvec<T>::type * buf, int ld, int nb, const FftPlan & P,
     const typename cvec<T>::type * __restrict__ tw, T s, int st0, int st1){
@@ -566,194 +552,6 @@ __global__ void __launch_bounds__(NTMAX) tck_div_yfft(const YFwdArgs A){
   }
 }
 
-/* Persistent form (compiled for EPTK elements per thread per pass): each block loops over
- * tiles and loads the velocities of the first PF of its divergence elements of the next tile
- * before the current tile's passes. */
-#ifndef TCK_DIVY_PF
-#define TCK_DIVY_PF 1
-#endif
-#ifndef TCK_DIVY_KRUN
-#define TCK_DIVY_KRUN 1
-#endif
-
-template <typename T, int PF, int EPTK, bool W, bool TL>
-__global__ void __launch_bounds__(FFT_MAXTHREADS) tck_div_yfft_p(const YFwdArgs A){
-  typedef typename cvec<T>::type V;
-  extern __shared__ __align__(16) unsigned char fft_smem[];
-  V * sm = (V *)fft_smem;
-  const tc_geom_t & g = A.g;
-  const tc_coef_t & c = A.c;
-  const int ti = A.ti;
-  const int M = A.P.M;
-  const int nt = A.P.nt;
-  const int ntx = (g.nx + ti - 1) / ti;
-  const int ntiles = ntx * g.nz;
-  const double dt = *A.dt;
-  const double gamma = c_fft_rka[A.rkstep] + c_fft_rkb[A.rkstep];
-  const double norm = 1. * g.ny * g.nz;
-  const double prefactor = 1. / (gamma * dt) / norm;
-  const long long sy = g.px;
-  const long long sz = g.plane;
-  const V * twM = (const V *)A.twM;
-  const V * twN = (const V *)A.twN;
-  if constexpr (TL){
-    /* TL: both twiddle tables copied to LDS after the tile's lines, so that neither the passes
-     * nor the split below wait for a global load (a wait for a load also waits for the stores
-     * issued before it: in the split, each element's stores would wait for the last's) */
-    V * twl = sm + ti * A.ld;
-    for(int t = threadIdx.x; t < M; t += nt) twl[t] = twM[t];
-    for(int t = threadIdx.x; t <= M; t += nt) twl[M + t] = twN[t];
-    twM = twl;
-    twN = twl + M;
-  }
-  V * S = (V *)A.S;
-  /* element q of this thread in a tile: line t0, row j = r0 + q dr (the block size is a
-   * multiple of the tile width, a power of two no larger than 64) */
-  const int t0i = (threadIdx.x & (ti - 1)), r0i = (threadIdx.x >> fft_lg(ti)), dr = (nt >> fft_lg(ti));
-  int t0 = t0i, r0 = r0i;
-  double pre[PF][6];
-  bool pok[PF];
-  /* the six velocities of element q of tile tl: ok when inside the field; otherwise the loads
-   * read an in-bounds stand-in (cell i = 1, j = 1 of the tile's plane) and the element is put
-   * as 0, so that no load is conditional */
-  #define DV_LOAD(tl, q, P, ok) { \
-    const int j_ = r0 + (q) * dr; \
-    const int i_ = 1 + ((tl) % ntx) * ti + t0; \
-    ok = j_ < g.ny && i_ <= g.nx; \
-    const long long o_ = tck_idx(g, ok ? i_ : 1, ok ? j_ + 1 : 1, 1 + (tl) / ntx); \
-    P[0] = A.ux[o_]; P[1] = A.ux[o_ + 1]; P[2] = A.uy[o_]; P[3] = A.uy[o_ + sy]; \
-    P[4] = A.uz[o_]; P[5] = A.uz[o_ + sz]; }
-  /* elements per thread of a tile (the launch guarantees that they cover it), and how many
-   * are loaded together */
-  constexpr int EPT2 = 2 * EPTK;
-  constexpr int G = 2;
-#if TCK_DIVY_KRUN
-  /* The same with uz's lower face taken from uzc when cz: in a block's run of planes the next
-   * tile is the same column one plane up, whose lower faces are this tile's upper faces, held
-   * in registers (the same values, so the same bits) instead of read again */
-  double uzc[EPT2];
-  #define DV_LOADC(tl, q, P, ok, cz) { \
-    const int j_ = r0 + (q) * dr; \
-    const int i_ = 1 + ((tl) % ntx) * ti + t0; \
-    ok = j_ < g.ny && i_ <= g.nx; \
-    const long long o_ = tck_idx(g, ok ? i_ : 1, ok ? j_ + 1 : 1, 1 + (tl) / ntx); \
-    P[0] = A.ux[o_]; P[1] = A.ux[o_ + 1]; P[2] = A.uy[o_]; P[3] = A.uy[o_ + sy]; \
-    if(cz) P[4] = uzc[q]; else P[4] = A.uz[o_]; \
-    P[5] = A.uz[o_ + sz]; }
-  /* each block walks a contiguous run of planes of one column of tiles, so that the uz
-   * plane a tile reads as its upper face is read again as the next tile's lower face soon
-   * after, from cache; tile index tile = tx + ntx (k - 1) as in the plain order */
-  const int per = (ntiles + (int)gridDim.x - 1) / (int)gridDim.x;
-  const int c0 = blockIdx.x * per, c1 = min(c0 + per, ntiles);
-  #define DV_TILE(c) (((c) / g.nz) + ntx * ((c) % g.nz))
-  int cc = c0;
-  if(cc < c1){
-    #pragma unroll
-    for(int q = 0; q < PF; q++){ DV_LOAD(DV_TILE(cc), q, pre[q], pok[q]); }
-  }
-  for(; cc < c1; cc++){
-    const int tile = DV_TILE(cc);
-    const int tnext = cc + 1 < c1 ? DV_TILE(cc + 1) : ntiles;
-    /* this tile's lower faces in uzc (the previous tile was the plane below), and the next
-     * tile's (it is the plane above); not with radix 5 and 7 plans, whose passes need the
-     * registers */
-    const bool cz = !W && cc > c0 && tile == DV_TILE(cc - 1) + ntx;
-    const bool czn = !W && tnext == tile + ntx;
-#else
-  int tile = blockIdx.x;
-  if(tile < ntiles){
-    #pragma unroll
-    for(int q = 0; q < PF; q++){ DV_LOAD(tile, q, pre[q], pok[q]); }
-  }
-  for(; tile < ntiles; tile += gridDim.x){
-    const int tnext = tile + (int)gridDim.x;
-#endif
-    /* the element offsets are recomputed in every tile rather than held across the passes */
-    t0 = t0i; r0 = r0i;
-    asm volatile("" : "+v"(t0), "+v"(r0));
-    const int i0 = 1 + (tile % ntx) * ti;
-    const int k = 1 + tile / ntx;
-    /* divergence (assign_input :404-423, same operand order as tck_div_yfft) packed as
-     * z_m = x_2m + i x_2m+1 */
-    const int i = i0 + t0;
-    auto put = [&](const int q, const double * P, const bool ok){
-      const int j0 = r0 + q * dr;
-      if(j0 >= g.ny) return;
-      double val = 0.;
-      if(ok){
-        const double div = c.ijdxc[i] * (
-            - c.jhxf[i] * P[0] + c.jhxf[i + 1] * P[1]
-            - c.jhyc[i] * P[2] + c.jhyc[i] * P[3]
-            - c.jhzc[i] * P[4] + c.jhzc[i] * P[5]);
-        val = prefactor * div;
-      }
-      ((T *)(sm + t0 * A.ld))[2 * fpad(j0 >> 1) + (j0 & 1)] = T(val);
-    };
-    /* the rest of the tile, G elements (6 G loads) issued before the first is waited for */
-    #pragma unroll
-    for(int q0 = PF; q0 < EPT2; q0 += G){
-      double P[G][6];
-      bool ok[G];
-#if TCK_DIVY_KRUN
-      #pragma unroll
-      for(int u = 0; u < G; u++) if(q0 + u < EPT2){ DV_LOADC(tile, q0 + u, P[u], ok[u], cz); }
-#else
-      #pragma unroll
-      for(int u = 0; u < G; u++) if(q0 + u < EPT2){ DV_LOAD(tile, q0 + u, P[u], ok[u]); }
-#endif
-      if(q0 == PF){
-        #pragma unroll
-        for(int q = 0; q < PF; q++){
-          put(q, pre[q], pok[q]);
-#if TCK_DIVY_KRUN
-          uzc[q] = pre[q][5];
-#endif
-        }
-      }
-      #pragma unroll
-      for(int u = 0; u < G; u++) if(q0 + u < EPT2){
-        put(q0 + u, P[u], ok[u]);
-#if TCK_DIVY_KRUN
-        uzc[q0 + u] = P[u][5];
-#endif
-      }
-    }
-    fft_lds_barrier();
-    if(tnext < ntiles){
-#if TCK_DIVY_KRUN
-      #pragma unroll
-      for(int q = 0; q < PF; q++){ DV_LOADC(tnext, q, pre[q], pok[q], czn); }
-#else
-      #pragma unroll
-      for(int q = 0; q < PF; q++){ DV_LOAD(tnext, q, pre[q], pok[q]); }
-#endif
-    }
-    lds_fft<T, EPTK, W>(sm, A.ld, ti, A.P, twM, T(-1.));
-    for(int e = threadIdx.x; e < ti * (M + 1); e += nt){
-      const int t = (e & (ti - 1));
-      const int kk = (e >> fft_lg(ti));
-      const int ii = i0 + t;
-      if(ii > g.nx) continue;
-      const V zk = sm[t * A.ld + fpad(kk == M ? 0 : kk)];
-      const V zc = cconj(sm[t * A.ld + fpad(kk == 0 ? 0 : M - kk)]);
-      const V w = twN[kk];
-      const V ev = mk2<T>(T(0.5) * (zk.x + zc.x), T(0.5) * (zk.y + zc.y));
-      const V od = mk2<T>(T(0.5) * (zk.x - zc.x), T(0.5) * (zk.y - zc.y));
-      const V wo = cmul(w, od);
-      const V Xk = mk2<T>(ev.x + wo.y, ev.y - wo.x);
-      tck_st(&S[(long long)(ii - 1) + (long long)g.nx * ((long long)kk + (long long)A.nky * (k - 1))], Xk);
-    }
-    fft_lds_barrier();
-  }
-  #undef DV_LOAD
-#if TCK_DIVY_KRUN
-  #undef DV_LOADC
-#endif
-#if TCK_DIVY_KRUN
-  #undef DV_TILE
-#endif
-}
-
 /* ------------------------------------------------------------------------------------- */
 struct ZArgs {
   int nx, nky, nz, tz, ld;
@@ -782,147 +580,111 @@ __global__ void __launch_bounds__(FFT_MAXTHREADS) tck_zfft(const ZArgs A){
       [&](int t, int kz, V v, bool ok){ if(ok && t < nl) tck_st(&base[t + kstride * kz], v); });
 }
 
-/* Persistent form: each block loops over tiles and issues the loads of the first PF of its
- * elements of the next tile before the current tile's transform, so that part of the HBM
- * traffic overlaps the LDS passes; the remaining elements are loaded when the tile starts, all
- * issued before the first is waited for.  Compiled for EPTK elements per thread per pass: the
- * launch guarantees that blockDim.x EPTK covers the tile and that blockDim.x is a multiple of
- * the tile width. */
-#ifndef TCK_ZFFT_PF
-#define TCK_ZFFT_PF 2            /* elements per thread loaded one tile ahead */
-#endif
-
-template <typename T, int PF, int EPTK, bool W, bool X>
+/* Persistent exact form: the tiles cover the spectrum exactly (nx a multiple of tz, blockDim.x EPTK
+ * = tz nz), so no access is conditional; the first radix is 8 and the last one RL (2, 3, 4 or 8).
+ * The twiddle factors are read from LDS (after the tile's lines), so that the passes issue no
+ * global loads.  The inputs of the next tile's first pass are loaded into registers before the
+ * current tile's middle passes, and the last pass stores its results from registers, so a tile
+ * crosses LDS once between passes.  Outstanding global loads and stores complete in issue order
+ * as far as the wait counter is concerned, so a wait for a load issued after a store also waits
+ * for the store: here the loads of tile n+1 are issued before the stores of tile n, and the
+ * first pass of tile n+1 waits only for its loads.  The stores into a zero-size buffer before the
+ * loop (they write nothing) give the loop's entry the same outstanding loads-then-stores
+ * sequence as the end of an iteration, so that the compiler's wait there is the same counted
+ * wait on both paths into it.  Bound by HBM (the spectrum read and written once).  Against a
+ * persistent form that went through LDS for the first loads and the last stores, ms per step
+ * (six launches): FP64 512x1024x512 6.02 -> 5.17, 256x512x512 1.60 -> 1.38; FP32 256x512x512
+ * 0.82 -> 0.74 */
+template <typename T, int EPTK, int RL>
 __global__ void __launch_bounds__(FFT_MAXTHREADS) tck_zfft_p(const ZArgs A){
   typedef typename cvec<T>::type V;
   extern __shared__ __align__(16) unsigned char fft_smem[];
   V * sm = (V *)fft_smem;
-  const int tz = A.tz, nz = A.nz, nt = A.P.nt;
-  const int ntx = (A.nx + tz - 1) / tz;
+  constexpr int NB = EPTK / 8, NL = (EPTK + RL - 1) / RL;     /* butterflies per thread: first, last pass */
+  constexpr bool ALL = NL * RL == EPTK;             /* every thread has NL in the last pass */
+  const int tz = A.tz, nz = A.nz, nt = A.P.nt, lg = fft_lg(tz);
+  const int ntx = A.nx / tz;
   const int ntiles = ntx * A.nky;
   const long long kstride = (long long)A.nx * A.nky;
-  /* element q of this thread in a tile: line t0, row kz = r0 + q dr (the block size is a
-   * multiple of the tile width, a power of two no larger than 64) */
-  const int t0i = (threadIdx.x & (tz - 1)), r0i = (threadIdx.x >> fft_lg(tz)), dr = (nt >> fft_lg(tz));
-  if constexpr (X){
-    /* Exact form: the tiles cover the spectrum exactly (nx a multiple of tz, blockDim.x EPTK =
-     * tz nz), so no access is conditional; the twiddle factors are read from LDS (after the
-     * tile's lines), so that the passes issue no global loads; and every element of the next
-     * tile is loaded before the current tile's passes and stores.  Outstanding global loads and
-     * stores complete in issue order as far as the wait counter is concerned, so a wait for a
-     * load issued after a store also waits for the store: here the loads of tile n+1 are
-     * issued before the stores of tile n, and the put of tile n+1 waits only for its loads.
-     * The stores into a zero-size buffer before the loop (they write nothing) give the loop's
-     * entry the same outstanding loads-then-stores sequence as the end of an iteration, so that
-     * the compiler's wait at the put is the same counted wait on both paths into it. */
-    V * twl = sm + tz * A.ld;
-    for(int t = threadIdx.x; t < A.P.M; t += nt) twl[t] = ((const V *)A.tw)[t];
-    int tile = blockIdx.x;             /* the launch has at least four tiles per block */
-    V pre[EPTK];
-    #define ZX_OFF(tl, q) ((long long)A.nx * ((tl) / ntx) + (long long)(((tl) % ntx) * tz + t0i) + kstride * (long long)(r0i + (q) * dr))
-    /* FP32: the spectrum spans under 4 GB (checked on the host), so a tile's accesses are a
-     * buffer resource at the tile's first column plus 32-bit offsets: one register of address
-     * per thread instead of one 64-bit address per element */
-    const unsigned vz = (unsigned)sizeof(V) * (unsigned)(t0i + kstride * r0i);
-    const unsigned sq = (unsigned)sizeof(V) * (unsigned)(kstride * dr);
-    #define ZX_RS(tl) tck_rsrc_u((const V *)A.S + (long long)A.nx * ((tl) / ntx) + (long long)(((tl) % ntx) * tz), \
-      (unsigned)sizeof(V) * (unsigned)(kstride * nz))
-    if constexpr (sizeof(T) == 4){
-      const __amdgpu_buffer_rsrc_t rs = ZX_RS(tile);
-      #pragma unroll
-      for(int q = 0; q < EPTK; q++) pre[q] = tck_bldf2(rs, vz, sq * q);
-    }else{
-      #pragma unroll
-      for(int q = 0; q < EPTK; q++) pre[q] = tck_ld((const V *)A.S + ZX_OFF(tile, q));
+  V * twl = sm + tz * A.ld;
+  for(int t = threadIdx.x; t < nz; t += nt) twl[t] = ((const V *)A.tw)[t];
+  /* butterfly q of this thread: line t0, index j0 + q dr */
+  const int t0 = threadIdx.x & (tz - 1), j0 = (int)threadIdx.x >> lg, dr = nt >> lg;
+  const int perf = nz / 8, perl = nz / RL;
+  /* FP32: the spectrum spans under 4 GB (checked on the host), so a tile's accesses are a buffer
+   * resource at the tile's first column plus 32-bit offsets */
+  const unsigned vz = (unsigned)sizeof(V) * (unsigned)(t0 + kstride * j0);
+  const unsigned ks = (unsigned)sizeof(V) * (unsigned)kstride;
+  #define ZX_COL(tl) ((V *)A.S + (long long)A.nx * ((tl) / ntx) + (long long)(((tl) % ntx) * tz))
+  #define ZX_RS(tl) tck_rsrc_u(ZX_COL(tl), ks * (unsigned)nz)
+  #define ZX_LOAD(tl) \
+    if constexpr (sizeof(T) == 4){ \
+      const __amdgpu_buffer_rsrc_t rs = ZX_RS(tl); \
+      _Pragma("unroll") for(int q = 0; q < NB; q++) \
+        _Pragma("unroll") for(int r = 0; r < 8; r++) pre[q][r] = tck_bldf2(rs, vz, ks * (unsigned)(q * dr + r * perf)); \
+    }else{ \
+      const V * col = ZX_COL(tl) + (t0 + kstride * j0); \
+      _Pragma("unroll") for(int q = 0; q < NB; q++) \
+        _Pragma("unroll") for(int r = 0; r < 8; r++) pre[q][r] = tck_ld(col + kstride * (q * dr + r * perf)); \
     }
+  int tile = blockIdx.x;             /* the launch has at least four tiles per block */
+  const T s = T(A.sign);
+  V pre[NB][8];
+  ZX_LOAD(tile)
+  {
+    const __amdgpu_buffer_rsrc_t nul = tck_rsrc(A.S, 0u);
+    #pragma unroll
+    for(int q = 0; q < EPTK; q++) tck_bst0(nul, 16u * q);
+  }
+  for(;;){
+    /* the LDS offsets are recomputed in every tile rather than held across the passes */
+    int tt = t0, jj0 = j0;
+    asm volatile("" : "+v"(tt), "+v"(jj0));
+    #pragma unroll
+    for(int q = 0; q < NB; q++){
+      dftr<8, T>::run(pre[q], s);
+      V * dst = sm + tt * A.ld;
+      #pragma unroll
+      for(int r = 0; r < 8; r++) dst[fpad(8 * (jj0 + q * dr) + r)] = pre[q][r];
+    }
+    fft_pass_barrier();
+    const int nxt = tile + (int)gridDim.x < ntiles ? tile + (int)gridDim.x : tile;
+    ZX_LOAD(nxt)
+    fft_mid<T, EPTK, false>(sm, A.ld, tz, A.P, twl, s, 1, A.P.nst - 1);
     {
-      const __amdgpu_buffer_rsrc_t nul = tck_rsrc(A.S, 0u);
+      const __amdgpu_buffer_rsrc_t rs = ZX_RS(tile);
+      V * col = ZX_COL(tile) + (tt + kstride * jj0);
+      const V * src = sm + tt * A.ld;
       #pragma unroll
-      for(int q = 0; q < EPTK; q++) tck_bst0(nul, 16u * q);
-    }
-    for(;;){
-      #pragma unroll
-      for(int q = 0; q < EPTK; q++) sm[t0i * A.ld + fpad(r0i + q * dr)] = pre[q];
-      fft_lds_barrier();
-      const int nxt = tile + (int)gridDim.x < ntiles ? tile + (int)gridDim.x : tile;
-      if constexpr (sizeof(T) == 4){
-        const __amdgpu_buffer_rsrc_t rs = ZX_RS(nxt);
+      for(int q = 0; q < NL; q++){
+        const int jj = jj0 + q * dr;
+        if(!ALL && jj >= perl) break;
+        V v[RL];
         #pragma unroll
-        for(int q = 0; q < EPTK; q++) pre[q] = tck_bldf2(rs, vz, sq * q);
-      }else{
+        for(int r = 0; r < RL; r++){
+          V x = src[fpad(jj + r * perl)];
+          if(r > 0){
+            V w = twl[jj * r];
+            if(s > T(0.)) w.y = - w.y;
+            x = cmul(x, w);
+          }
+          v[r] = x;
+        }
+        dftr<RL, T>::run(v, s);
         #pragma unroll
-        for(int q = 0; q < EPTK; q++) pre[q] = tck_ld((const V *)A.S + ZX_OFF(nxt, q));
-      }
-      lds_fft<T, EPTK, W>(sm, A.ld, tz, A.P, twl, T(A.sign));
-      if constexpr (sizeof(T) == 4){
-        const __amdgpu_buffer_rsrc_t rs = ZX_RS(tile);
-        #pragma unroll
-        for(int q = 0; q < EPTK; q++) tck_bstf2(rs, vz, sq * q, sm[t0i * A.ld + fpad(r0i + q * dr)]);
-      }else{
-        V * base = (V *)A.S + (long long)A.nx * (tile / ntx) + (long long)((tile % ntx) * tz + t0i);
-        #pragma unroll
-        for(int q = 0; q < EPTK; q++){
-          const int kz = r0i + q * dr;
-          tck_st(&base[kstride * kz], sm[t0i * A.ld + fpad(kz)]);
+        for(int r = 0; r < RL; r++){
+          if constexpr (sizeof(T) == 4) tck_bstf2(rs, vz, ks * (unsigned)(q * dr + r * perl), v[r]);
+          else tck_st(col + kstride * (q * dr + r * perl), v[r]);
         }
       }
-      fft_lds_barrier();
-      tile += (int)gridDim.x;
-      if(tile >= ntiles) break;
     }
-    #undef ZX_OFF
-    #undef ZX_RS
-    return;
-  }
-  int t0 = t0i, r0 = r0i;
-  V pre[PF];
-  bool pok[PF];
-  int tile = blockIdx.x;
-  /* element q of tile tl: ok when inside the spectrum; otherwise the load reads element 0
-   * (in bounds) and the value is replaced by 0 when put, so that no load is conditional */
-  #define ZF_ELEM(tl, q, out, ok) { \
-    const int kz_ = r0 + (q) * dr; \
-    const int tx_ = (tl) % ntx; \
-    const int ii_ = tx_ * tz + t0; \
-    ok = kz_ < nz && ii_ < A.nx; \
-    const V * b_ = (const V *)A.S + (long long)A.nx * ((tl) / ntx); \
-    out = tck_ld(ok ? &b_[ii_ + kstride * kz_] : (const V *)A.S); }
-  #define ZF_PUT(q, v, ok) { const int kz_ = r0 + (q) * dr; \
-    if(kz_ < nz) sm[t0 * A.ld + fpad(kz_)] = (ok) ? (v) : mk2<T>(T(0.), T(0.)); }
-  if(tile < ntiles){
-    #pragma unroll
-    for(int q = 0; q < PF; q++){ ZF_ELEM(tile, q, pre[q], pok[q]); }
-  }
-  for(; tile < ntiles; tile += gridDim.x){
-    /* the element offsets are recomputed in every tile rather than held across the passes */
-    t0 = t0i; r0 = r0i;
-    asm volatile("" : "+v"(t0), "+v"(r0));
-    /* the rest of the tile: all loads issued before the first is waited for */
-    V cur[EPTK - PF > 0 ? EPTK - PF : 1];
-    bool cok[EPTK - PF > 0 ? EPTK - PF : 1];
-    #pragma unroll
-    for(int q = PF; q < EPTK; q++){ ZF_ELEM(tile, q, cur[q - PF], cok[q - PF]); }
-    #pragma unroll
-    for(int q = 0; q < PF; q++){ ZF_PUT(q, pre[q], pok[q]); }
-    #pragma unroll
-    for(int q = PF; q < EPTK; q++){ ZF_PUT(q, cur[q - PF], cok[q - PF]); }
-    fft_lds_barrier();
-    if(tile + (int)gridDim.x < ntiles){
-      #pragma unroll
-      for(int q = 0; q < PF; q++){ ZF_ELEM(tile + (int)gridDim.x, q, pre[q], pok[q]); }
-    }
-    lds_fft<T, EPTK, W>(sm, A.ld, tz, A.P, (const V *)A.tw, T(A.sign));
-    const int ii = (tile % ntx) * tz + t0;
-    V * base = (V *)A.S + (long long)A.nx * (tile / ntx);
-    #pragma unroll
-    for(int q = 0; q < EPTK; q++){
-      const int kz = r0 + q * dr;
-      if(kz < nz && ii < A.nx) tck_st(&base[ii + kstride * kz], sm[t0 * A.ld + fpad(kz)]);
-    }
+    tile += (int)gridDim.x;
+    if(tile >= ntiles) break;
     fft_lds_barrier();
   }
-  #undef ZF_ELEM
-  #undef ZF_PUT
+  #undef ZX_COL
+  #undef ZX_RS
+  #undef ZX_LOAD
 }
 
 /* ------------------------------------------------------------------------------------- */
@@ -1010,7 +772,7 @@ __global__ void __launch_bounds__(FFT_MAXTHREADS) tck_yifft_psi(const YInvArgs A
   const auto put = [&](int j, T v){
     T * p = col + (long long)g.px * j;
     tck_st(p, v);
-    if(wall) p[wall] = v;
+    if(wall) tck_st(&p[wall], v);
     if(dk){
       p[dk] = v;
       if(wall) p[dk + wall] = v;
@@ -1028,221 +790,142 @@ __global__ void __launch_bounds__(FFT_MAXTHREADS) tck_yifft_psi(const YInvArgs A
   fft_last<T, EPT, W>(sm, A.ld, lg, A.P, (const V *)A.twM, T(1.), store);
 }
 
-/* Persistent form of tck_yifft_psi (compiled for EPTK elements per thread per pass): each
- * block loops over tiles and issues the spectrum loads of the first PF of its elements of the
- * next tile before the current tile's passes. */
-#ifndef TCK_YIFFT_PF
-#define TCK_YIFFT_PF 2
-#endif
-
-template <typename T, int PF, int EPTK, bool W, bool X>
+/* Persistent exact form: the tiles cover the field exactly (nx a multiple of ti,
+ * blockDim.x EPTK = ti M), so no load is conditional and the loops have fixed counts; the last
+ * radix is RL.  The twiddle factors are read from LDS (after the
+ * tile's lines); the pairs (X_k, X_{M-k}) of the next tile are loaded into registers before the
+ * current tile's passes and stores, and forming Z' from them waits only for those loads (the
+ * zero-size stores before the loop give its entry the outstanding loads-then-stores sequence of
+ * an iteration's end, as in tck_zfft_p).  Bound by HBM (a read of the spectrum and a write of
+ * psi).  One-tile form against this one, ms per step (three launches): FP64 512x1024x512
+ * 4.07 -> 3.06, 256x512x512 0.82 -> 0.77, 128x1024x256 0.574 -> 0.448; FP32 512x1024x512
+ * 2.26 -> 1.72, 128x1024x256 0.363 -> 0.297 */
+template <typename T, int EPTK, int RL>
 __global__ void __launch_bounds__(FFT_MAXTHREADS) tck_yifft_psi_p(const YInvArgs A){
   typedef typename cvec<T>::type V;
   extern __shared__ __align__(16) unsigned char fft_smem[];
   V * sm = (V *)fft_smem;
+  constexpr int NP = EPTK / 2, NL = (EPTK + RL - 1) / RL;   /* pairs, last-pass butterflies per thread */
+  constexpr bool ALL = NL * RL == EPTK;
   const tc_geom_t & g = A.g;
-  const int ti = A.ti;
+  const int ti = A.ti, lg = fft_lg(ti);
   const int M = A.P.M;
   const int nt = A.P.nt;
-  const int ntx = (g.nx + ti - 1) / ti;
+  const int ntx = g.nx / ti;
   const int ntiles = ntx * g.nz;
   const V * S = (const V *)A.S;
-  const V * twN = (const V *)A.twN;
   T * psi = (T *)A.psi;
-  /* element q of this thread in a tile: line t0, wavenumber kk = r0 + q dr (the block size is
-   * a multiple of the tile width, a power of two no larger than 64); only q = 0 can hold
-   * kk = 0 */
-  const int t0i = (threadIdx.x & (ti - 1)), r0i = (threadIdx.x >> fft_lg(ti)), dr = (nt >> fft_lg(ti));
-  if constexpr (X){
-    /* Exact form: the tiles cover the field exactly (nx a multiple of ti, blockDim.x EPTK =
-     * ti M), so no load is conditional and the loops have fixed counts; the twiddle factors
-     * are read from LDS (after the tile's lines); every spectrum value of the next tile is
-     * loaded before the current tile's passes and stores, and the put waits only for those
-     * loads (the zero-size stores before the loop give its entry the outstanding
-     * loads-then-stores sequence of an iteration's end, as in tck_zfft_p). */
-    V * twl = sm + ti * A.ld;
-    V * twnl = twl + M;
-    const V * twM = (const V *)A.twM;
-    for(int t = threadIdx.x; t < M; t += nt){ twl[t] = twM[t]; twnl[t] = twN[t]; }
-    constexpr int NST = 2 * EPTK;        /* psi values stored per thread: ti ny = 2 blockDim.x EPTK */
-    int tile = blockIdx.x;               /* the launch has at least four tiles per block */
-    /* buffer addressing: a tile's spectrum values lie in one plane of S (nky nx complex values)
-     * and its psi values in one plane of the field, so each access is a per-thread byte offset
-     * that does not change between tiles plus a uniform one */
-    constexpr unsigned CB = sizeof(V), RB = sizeof(T);                 /* complex, real bytes */
-    const unsigned vs = CB * (unsigned)(t0i + g.nx * r0i);             /* X_kk, kk = r0 + q dr */
-    const unsigned ss = CB * (unsigned)(g.nx * dr);                    /* per q */
-    const unsigned vxm = CB * (unsigned)(t0i + g.nx * M);              /* X_M */
-    const unsigned sbytes = CB * (unsigned)(g.nx * A.nky);
-    const unsigned vp = RB * (unsigned)(t0i + g.px * r0i);             /* psi row r0 + 1 + q dr */
-    const unsigned sp = RB * (unsigned)(g.px * dr);
-    const unsigned pbytes = RB * (unsigned)(g.px * g.ny);
-    #define YX_RS(tl) tck_rsrc(S + (long long)((tl) % ntx * ti) + (long long)g.nx * A.nky * ((tl) / ntx), sbytes)
-    V pre[EPTK], prexm;
-    {
-      const __amdgpu_buffer_rsrc_t rs = YX_RS(tile);
-      #pragma unroll
-      for(int q = 0; q < EPTK; q++) pre[q] = tck_bldc<V>(rs, vs, ss * q);
-      prexm = tck_bldc<V>(rs, vxm, 0u);
-      const __amdgpu_buffer_rsrc_t nul = tck_rsrc(A.S, 0u);
-      #pragma unroll
-      for(int q = 0; q < NST; q++) tck_bst0(nul, 16u * q);
-    }
-    for(;;){
-      /* the LDS offsets are recomputed in every tile rather than held across the passes */
-      int t0 = t0i, r0 = r0i;
-      asm volatile("" : "+v"(t0), "+v"(r0));
-      const int i0 = 1 + (tile % ntx) * ti;
-      const int k = 1 + tile / ntx;
-      /* X_1..X_{M-1} as loaded; Z'_0 from X_0 and X_M (element 0 of the threads with r0 = 0) */
-      #pragma unroll
-      for(int q = 0; q < EPTK; q++){
-        V v = pre[q];
-        if(q == 0 && r0 == 0){
-          V xm = prexm;
-          v.y = T(0.);
-          xm.y = T(0.);
-          v = c2r_pre(v, xm, twnl[0]);
-        }
-        sm[t0 * A.ld + fpad(r0 + q * dr)] = v;
-      }
-      fft_lds_barrier();
-      {
-        const int nxt = tile + (int)gridDim.x < ntiles ? tile + (int)gridDim.x : tile;
-        const __amdgpu_buffer_rsrc_t rs = YX_RS(nxt);
-        #pragma unroll
-        for(int q = 0; q < EPTK; q++) pre[q] = tck_bldc<V>(rs, vs, ss * q);
-        prexm = tck_bldc<V>(rs, vxm, 0u);
-      }
-      /* Z'_k1, Z'_k2 for k1 = 1..M/2 (ti M / 2 = blockDim.x EPTK / 2 pairs) */
-      #pragma unroll
-      for(int q = 0; q < EPTK / 2; q++){
-        const int e = threadIdx.x + q * nt;
-        const int t = (e & (ti - 1));
-        const int k1 = 1 + (e >> fft_lg(ti));
-        const int k2 = M - k1;
-        const V xa = sm[t * A.ld + fpad(k1)];
-        const V xb = sm[t * A.ld + fpad(k2)];
-        const V z1 = c2r_pre(xa, xb, twnl[k1]);
-        if(k2 != k1){
-          const V z2 = c2r_pre(xb, xa, twnl[k2]);
-          sm[t * A.ld + fpad(k2)] = z2;
-        }
-        sm[t * A.ld + fpad(k1)] = z1;
-      }
-      fft_lds_barrier();
-      lds_fft<T, EPTK, W>(sm, A.ld, ti, A.P, twl, T(1.));
-      /* element q of this thread: line t0, row jj = r0 + q dr; the interior values first, all
-       * unconditional, then the halo images and wall copies of the threads that have any */
-      const int i = i0 + t0;
-      const T * ln = (const T *)(sm + t0 * A.ld);
-      {
-        const __amdgpu_buffer_rsrc_t rp = tck_rsrc(psi + tck_idx(g, i0, 1, k), pbytes);
-        #pragma unroll
-        for(int q = 0; q < NST; q++){
-          const int jj = r0 + q * dr;
-          tck_bstn<T>(rp, vp, sp * q, ln[2 * fpad(jj >> 1) + (jj & 1)]);
-        }
-      }
-      if(i == 1 || i == g.nx || k == 1 || k == g.nz || r0 == 0 || r0 == dr - 1){
-        for(int q = 0; q < NST; q++){
-          const int jj = r0 + q * dr;
-          tck_store_halo<T, false>(psi, g, i, jj + 1, k, ln[2 * fpad(jj >> 1) + (jj & 1)], true);
-        }
-      }
-      fft_lds_barrier();
-      tile += (int)gridDim.x;
-      if(tile >= ntiles) break;
-    }
-    #undef YX_RS
-    return;
-  }
-  int t0 = t0i, r0 = r0i;
-  V pre[PF];
-  bool pok[PF];
-  int tile = blockIdx.x;
-  /* raw spectrum value X_kk of element q of tile tl: ok when inside the field; otherwise the
-   * load reads element 0 (in bounds) and the value is replaced by 0 when put, so that no load
-   * is conditional */
-  #define YI_ELEM(tl, q, out, ok) { \
-    const int kk_ = r0 + (q) * dr; \
-    const int i_ = 1 + ((tl) % ntx) * ti + t0; \
-    ok = kk_ < M && i_ <= g.nx; \
-    const long long o_ = (long long)(i_ - 1) + (long long)g.nx * ((long long)A.nky * ((tl) / ntx) + kk_); \
-    out = tck_ld(ok ? &S[o_] : S); }
-  /* X_M of the line of element 0 (used when that element is kk = 0) */
-  #define YI_XM(tl, out) { \
-    const int i_ = 1 + ((tl) % ntx) * ti + t0; \
-    const bool ok_ = r0 == 0 && i_ <= g.nx; \
-    const long long o_ = (long long)(i_ - 1) + (long long)g.nx * ((long long)A.nky * ((tl) / ntx) + M); \
-    out = tck_ld(ok_ ? &S[o_] : S); }
-  V prexm = mk2<T>(T(0.), T(0.));
-  if(tile < ntiles){
+  V * twl = sm + ti * A.ld;
+  V * twnl = twl + M;
+  for(int t = threadIdx.x; t < M; t += nt){ twl[t] = ((const V *)A.twM)[t]; twnl[t] = ((const V *)A.twN)[t]; }
+  fft_lds_barrier();   /* twnl is read for the first tile before any of the barriers of the loop */
+  /* pair u of this thread: line t0, k1 = 1 + r0 + u dr; last-pass butterfly q: index r0 + q dr */
+  const int t0i = (int)threadIdx.x & (ti - 1), r0i = (int)threadIdx.x >> lg, dr = nt >> lg;
+  const int perl = M / RL;
+  int tile = blockIdx.x;               /* the launch has at least four tiles per block */
+  /* buffer addressing: a tile's spectrum values lie in one plane of S (nky nx complex values) and
+   * its psi values in one plane of the field, so each access is a per-thread byte offset that does
+   * not change between tiles plus a uniform one */
+  constexpr unsigned CB = sizeof(V), RB = sizeof(T);                 /* complex, real bytes */
+  const unsigned ss = CB * (unsigned)(g.nx * dr);                    /* per u */
+  const unsigned va = CB * (unsigned)(t0i + g.nx * (1 + r0i));       /* X_k1, u = 0 */
+  const unsigned vb = CB * (unsigned)(t0i + g.nx * (M - 1 - r0i - (NP - 1) * dr));   /* X_{M-k1}, u = NP - 1 */
+  const unsigned v0 = CB * (unsigned)t0i, vm = CB * (unsigned)(t0i + g.nx * M);
+  const unsigned sbytes = CB * (unsigned)(g.nx * A.nky);
+  const unsigned vp = RB * (unsigned)(t0i + 2 * g.px * r0i);         /* psi row 2 r0 + 1 */
+  const unsigned sp = RB * (unsigned)g.px;
+  const unsigned pbytes = RB * (unsigned)(g.px * g.ny);
+  V xa[NP], xb[NP], x0, xm;
+  #define YX_LOAD(tl) { \
+    const __amdgpu_buffer_rsrc_t rs = tck_rsrc(S + (long long)((tl) % ntx * ti) + (long long)g.nx * A.nky * ((tl) / ntx), sbytes); \
+    _Pragma("unroll") for(int u = 0; u < NP; u++){ xa[u] = tck_bldc<V>(rs, va, ss * u); xb[u] = tck_bldc<V>(rs, vb, ss * (NP - 1 - u)); } \
+    x0 = tck_bldc<V>(rs, v0, 0u); \
+    xm = tck_bldc<V>(rs, vm, 0u); }
+  YX_LOAD(tile)
+  {
+    const __amdgpu_buffer_rsrc_t nul = tck_rsrc(A.S, 0u);
     #pragma unroll
-    for(int q = 0; q < PF; q++){ YI_ELEM(tile, q, pre[q], pok[q]); }
-    YI_XM(tile, prexm);
+    for(int q = 0; q < 2 * EPTK; q++) tck_bst0(nul, 16u * q);
   }
-  for(; tile < ntiles; tile += gridDim.x){
-    /* the element offsets are recomputed in every tile rather than held across the passes */
-    t0 = t0i; r0 = r0i;
+  for(;;){
+    /* the LDS offsets are recomputed in every tile rather than held across the passes */
+    int t0 = t0i, r0 = r0i;
     asm volatile("" : "+v"(t0), "+v"(r0));
-    const int i0 = 1 + (tile % ntx) * ti;
     const int k = 1 + tile / ntx;
-    /* X_1..X_{M-1} as loaded; Z'_0 from X_0 and X_M */
-    auto put = [&](const int q, V v, const bool ok, V xm){
-      const int kk = r0 + q * dr;
-      if(kk >= M) return;
-      if(!ok) v = mk2<T>(T(0.), T(0.));
-      else if(kk == 0){
-        v.y = T(0.);
-        xm.y = T(0.);
-        v = c2r_pre(v, xm, twN[0]);
-      }
-      sm[t0 * A.ld + fpad(kk)] = v;
-    };
-    /* the rest of the tile: all loads issued before the first is waited for */
-    V cur[EPTK - PF > 0 ? EPTK - PF : 1];
-    bool cok[EPTK - PF > 0 ? EPTK - PF : 1];
+    const int i = 1 + (tile % ntx) * ti + t0;
+    V * ln = sm + t0 * A.ld;
     #pragma unroll
-    for(int q = PF; q < EPTK; q++){ YI_ELEM(tile, q, cur[q - PF], cok[q - PF]); }
-    #pragma unroll
-    for(int q = 0; q < PF; q++) put(q, pre[q], pok[q], prexm);
-    #pragma unroll
-    for(int q = PF; q < EPTK; q++) put(q, cur[q - PF], cok[q - PF], prexm);
+    for(int u = 0; u < NP; u++){
+      const int k1 = 1 + r0 + u * dr, k2 = M - k1;
+      const V z1 = c2r_pre(xa[u], xb[u], twnl[k1]);
+      if(k2 != k1) ln[fpad(k2)] = c2r_pre(xb[u], xa[u], twnl[k2]);
+      ln[fpad(k1)] = z1;
+    }
+    if(r0 == 0){
+      x0.y = T(0.);
+      xm.y = T(0.);
+      ln[fpad(0)] = c2r_pre(x0, xm, twnl[0]);
+    }
     fft_lds_barrier();
-    if(tile + (int)gridDim.x < ntiles){
+    const int nxt = tile + (int)gridDim.x < ntiles ? tile + (int)gridDim.x : tile;
+    YX_LOAD(nxt)
+    fft_mid<T, EPTK, false>(sm, A.ld, ti, A.P, twl, T(1.), 0, A.P.nst - 1);
+    V v[NL][RL];
+    const __amdgpu_buffer_rsrc_t rp = tck_rsrc(psi + tck_idx(g, 1 + (tile % ntx) * ti, 1, k), pbytes);
+    #pragma unroll
+    for(int q = 0; q < NL; q++){
+      const int jj = r0 + q * dr;
+      if(!ALL && jj >= perl) break;
       #pragma unroll
-      for(int q = 0; q < PF; q++){ YI_ELEM(tile + (int)gridDim.x, q, pre[q], pok[q]); }
-      YI_XM(tile + (int)gridDim.x, prexm);
-    }
-    const int half = M / 2;
-    for(int e = threadIdx.x; e < ti * half; e += nt){
-      const int t = (e & (ti - 1));
-      const int k1 = 1 + (e >> fft_lg(ti));
-      const int k2 = M - k1;
-      const V xa = sm[t * A.ld + fpad(k1)];
-      const V xb = sm[t * A.ld + fpad(k2)];
-      const V z1 = c2r_pre(xa, xb, twN[k1]);
-      if(k2 != k1){
-        const V z2 = c2r_pre(xb, xa, twN[k2]);
-        sm[t * A.ld + fpad(k2)] = z2;
+      for(int r = 0; r < RL; r++){
+        V x = ln[fpad(jj + r * perl)];
+        if(r > 0){
+          V w = twl[jj * r];
+          w.y = - w.y;
+          x = cmul(x, w);
+        }
+        v[q][r] = x;
       }
-      sm[t * A.ld + fpad(k1)] = z1;
+      dftr<RL, T>::run(v[q], T(1.));
+      #pragma unroll
+      for(int r = 0; r < RL; r++){
+        tck_bstn<T>(rp, vp, sp * (unsigned)(2 * (q * dr + r * perl)), v[q][r].x);
+        tck_bstn<T>(rp, vp, sp * (unsigned)(2 * (q * dr + r * perl) + 1), v[q][r].y);
+      }
     }
-    fft_lds_barrier();
-    lds_fft<T, EPTK, W>(sm, A.ld, ti, A.P, (const V *)A.twM, T(1.));
-    for(int e = threadIdx.x; e < ti * g.ny; e += nt){
-      const int t = (e & (ti - 1));
-      const int jj = (e >> fft_lg(ti));
-      const int i = i0 + t;
-      if(i > g.nx) continue;
-      const T v = ((const T *)(sm + t * A.ld))[2 * fpad(jj >> 1) + (jj & 1)];
-      tck_store_halo(psi, g, i, jj + 1, k, v, true);
+    /* the halo images and wall copies of the threads that have any */
+    if(i == 1 || i == g.nx || k == 1 || k == g.nz || r0 == 0 || r0 == dr - 1){
+      T * col = psi + tck_idx(g, i, 0, k);
+      const int wall = i == 1 ? -1 : (i == g.nx ? 1 : 0);
+      const long long dk = k == 1 ? g.plane * g.nz : (k == g.nz ? - g.plane * g.nz : 0);
+      const auto img = [&](int j, T x, bool self){
+        T * p = col + (long long)g.px * j;
+        if(self) *p = x;
+        if(wall) tck_st(&p[wall], x);
+        if(dk){
+          p[dk] = x;
+          if(wall) p[dk + wall] = x;
+        }
+      };
+      #pragma unroll
+      for(int q = 0; q < NL; q++){
+        const int jj = r0 + q * dr;
+        if(!ALL && jj >= perl) break;
+        #pragma unroll
+        for(int r = 0; r < RL; r++){
+          const int n = jj + r * perl;
+          img(2 * n + 1, v[q][r].x, false);
+          img(2 * n + 2, v[q][r].y, false);
+          if(r == 0 && n == 0) img(g.ny + 1, v[q][r].x, true);
+          if(r == RL - 1 && n == M - 1) img(0, v[q][r].y, true);
+        }
+      }
     }
+    tile += (int)gridDim.x;
+    if(tile >= ntiles) break;
     fft_lds_barrier();
   }
-  #undef YI_ELEM
-  #undef YI_XM
+  #undef YX_LOAD
 }
 
 /* ------------------------------------------------------------------------------------- */
@@ -1385,15 +1068,14 @@ static int set_lds(const void * fn, size_t bytes){
   return 0;
 }
 
-/* Persistent launches, FP64 only (the FP32 forms, at 16 elements per thread, spill with the
- * prefetch registers).  The persistent kernels are compiled for FFT_EPT / 2 elements per
- * thread per pass, the count the LDS-bound FP64 tiles take; a launch qualifies when its
- * threads cover the tile at that count and it has at least four tiles per resident block.
+/* Persistent launches.  The kernels are compiled for ept elements per thread per pass
+ * (FFT_EPT / 2, or FFT_EPT for the FP32 axial transforms); a launch qualifies when its threads
+ * cover the tile at that count and it has at least four tiles per resident block.
  * Returns 1 when launched (the caller checks the launch), 0 when the caller should launch the
  * one-tile form, < 0 when the LDS limit could not be raised.  Resident blocks per CU are
  * queried once per (kernel, threads, LDS), so launches recorded into a graph make no query. */
 #define PERSIST_EPT (FFT_EPT / 2)
-#define PERSIST_CACHE 16
+#define PERSIST_CACHE 32
 static const void * g_pc_fn[PERSIST_CACHE];
 static int g_pc_nt[PERSIST_CACHE], g_pc_per[PERSIST_CACHE];
 static size_t g_pc_lds[PERSIST_CACHE];
@@ -1444,7 +1126,7 @@ extern "C" {
 /* mixed: spectrum, transforms and psi in FP32 (twiddles twM, twN, tw as float2) */
 int tck_launch_div_yfft(const tc_geom_t * g, const tc_coef_t * c, const double * ux,
     const double * uy, const double * uz, const double * dt, int rkstep, void * S,
-    const void * twM, const void * twN, int mixed, int twl, hipStream_t stream){
+    const void * twM, const void * twN, int mixed, hipStream_t stream){
   YFwdArgs A;
   A.g = *g; A.c = *c; A.ux = ux; A.uy = uy; A.uz = uz; A.dt = dt; A.rkstep = rkstep;
   A.S = S; A.nky = g->ny / 2 + 1;
@@ -1457,27 +1139,6 @@ int tck_launch_div_yfft(const tc_geom_t * g, const tc_coef_t * c, const double *
   A.ld = fft_ld(A.P.M);
   const size_t lds = cs * (size_t)A.ti * A.ld;
   const long long ntiles = (long long)((g->nx + A.ti - 1) / A.ti) * g->nz;
-#if TCK_DIVY_PF > 0
-  {
-    const long long el = (long long)A.ti * A.P.M;
-    /* the twiddle tables in LDS where they fit beside the tile (radix 2, 3, 4, 8 plans) */
-    const size_t ldsx = lds + cs * (size_t)(2 * A.P.M + 1);
-    const bool tl = twl && !plan_wide(&A.P) && ldsx <= lds_limit();
-    /* FP32 tiles: persistent only in this form, with FFT_EPT / 2 elements per thread (twice
-     * the threads of the one-tile form), which keeps the carried faces and the prefetch in
-     * registers */
-    const int ntf = (int)(el / PERSIST_EPT);
-    YFwdArgs AF = A;
-    AF.P.nt = ntf;
-    const bool tlf = tl && ntf <= FFT_MAXTHREADS && ntf % 64 == 0 && ntf % A.ti == 0 && (long long)ntf * PERSIST_EPT == el;
-    const int r = mixed ? (tlf ? launch_persistent(tck_div_yfft_p<float, TCK_DIVY_PF, PERSIST_EPT, false, true>, AF, ntf, ldsx, el, ntiles, stream) : 0)
-                : tl ? launch_persistent(tck_div_yfft_p<double, TCK_DIVY_PF, PERSIST_EPT, false, true>, A, nt, ldsx, el, ntiles, stream)
-                    : (plan_wide(&A.P) ? launch_persistent(tck_div_yfft_p<double, TCK_DIVY_PF, PERSIST_EPT, true, false>, A, nt, lds, el, ntiles, stream)
-                                       : launch_persistent(tck_div_yfft_p<double, TCK_DIVY_PF, PERSIST_EPT, false, false>, A, nt, lds, el, ntiles, stream));
-    if(r < 0) return (int)hipErrorInvalidValue;
-    if(r > 0){ TCK_CHECK_LAUNCH(); return 0; }
-  }
-#endif
   const dim3 grd((unsigned)ntiles);
   const long long el = (long long)A.ti * A.P.M;
   const bool wide = plan_wide(&A.P);
@@ -1509,25 +1170,25 @@ int tck_launch_zfft(int nx, int nky, int nz, void * S, const void * tw, int sign
   A.ld = fft_ld(nz);
   const size_t lds = cs * (size_t)A.tz * A.ld;
   const long long ntiles = (long long)((nx + A.tz - 1) / A.tz) * nky;
-#if TCK_ZFFT_PF > 0
   {
     const long long el = (long long)A.tz * nz;
-    /* the exact form when the tiles cover the spectrum exactly, the plan has no radix 5 or 7
-     * passes and its twiddle factors fit in the LDS beside the tile */
+    /* the exact form when the tiles cover the spectrum exactly, the plan starts with radix 8, has
+     * two passes at least and no radix 5 or 7, and its twiddle factors fit in the LDS beside the
+     * tile.  Where it does not hold (300x512x512), the one-tile form took 2.35 ms per step against
+     * 2.79 ms of a persistent one with conditional accesses */
     const size_t ldsx = lds + cs * (size_t)nz;
-    const bool x = exact && !plan_wide(&A.P) && nx % A.tz == 0 && (long long)nt * PERSIST_EPT == el && ldsx <= lds_limit();
-    /* FP32 tiles (twice as wide, FFT_EPT elements per thread): only the exact form is
-     * persistent, its registers holding the next tile in place of the prefetch */
-    const bool xf = exact && !plan_wide(&A.P) && nx % A.tz == 0 && (long long)nt * FFT_EPT == el && ldsx <= lds_limit()
-        && (long long)sizeof(float2) * nx * nky * nz < (1LL << 32);
-    const int r = mixed ? (xf ? launch_persistent(tck_zfft_p<float, TCK_ZFFT_PF, FFT_EPT, false, true>, A, nt, ldsx, el, ntiles, stream, FFT_EPT) : 0)
-                : x ? launch_persistent(tck_zfft_p<double, TCK_ZFFT_PF, PERSIST_EPT, false, true>, A, nt, ldsx, el, ntiles, stream)
-                    : (plan_wide(&A.P) ? launch_persistent(tck_zfft_p<double, TCK_ZFFT_PF, PERSIST_EPT, true, false>, A, nt, lds, el, ntiles, stream)
-                                       : launch_persistent(tck_zfft_p<double, TCK_ZFFT_PF, PERSIST_EPT, false, false>, A, nt, lds, el, ntiles, stream));
+    const int rl = A.P.rad[A.P.nst - 1];
+    const bool x = exact && !plan_wide(&A.P) && A.P.nst >= 2 && A.P.rad[0] == 8 && nx % A.tz == 0 && ldsx <= lds_limit() && (long long)nt * (mixed ? FFT_EPT : PERSIST_EPT) == el
+        && (!mixed || (long long)sizeof(float2) * nx * nky * nz < (1LL << 32));
+    #define ZX(T, E) (rl == 8 ? launch_persistent(tck_zfft_p<T, E, 8>, A, nt, ldsx, el, ntiles, stream, E) \
+        : rl == 4 ? launch_persistent(tck_zfft_p<T, E, 4>, A, nt, ldsx, el, ntiles, stream, E) \
+        : rl == 3 ? launch_persistent(tck_zfft_p<T, E, 3>, A, nt, ldsx, el, ntiles, stream, E) \
+                  : launch_persistent(tck_zfft_p<T, E, 2>, A, nt, ldsx, el, ntiles, stream, E))
+    const int r = !x ? 0 : mixed ? ZX(float, FFT_EPT) : ZX(double, PERSIST_EPT);
+    #undef ZX
     if(r < 0) return (int)hipErrorInvalidValue;
     if(r > 0){ TCK_CHECK_LAUNCH(); return 0; }
   }
-#endif
   const dim3 grd((unsigned)ntiles);
   const bool half = (long long)nt * (FFT_EPT / 2) >= (long long)A.tz * nz;
   if(half ? FFT_ONE_E(tck_zfft, FFT_EPT / 2, mixed, plan_wide(&A.P)) : FFT_ONE_E(tck_zfft, FFT_EPT, mixed, plan_wide(&A.P))) return (int)hipErrorInvalidValue;
@@ -1548,31 +1209,31 @@ int tck_launch_yifft_psi(const tc_geom_t * g, const void * S, void * psi, const 
   A.ld = fft_ld(A.P.M);
   const size_t lds = cs * (size_t)A.ti * A.ld;
   const long long ntiles = (long long)((g->nx + A.ti - 1) / A.ti) * g->nz;
-#if TCK_YIFFT_PF > 0
   {
     const long long el = (long long)A.ti * A.P.M;
-    /* the exact form when the tiles cover the field exactly, the plan has no radix 5 or 7
-     * passes, both twiddle tables fit in the LDS beside the tile and a plane's byte offsets fit
-     * in 31 bits */
+    /* the persistent form when the tiles cover the field exactly, the plan has two passes at least
+     * and no radix 5 or 7, both twiddle tables fit in the LDS beside the tile and a plane's byte
+     * offsets fit in 31 bits.  It is the faster one at every such FP64 size measured (128 to 1024
+     * rows, one to four blocks per CU: by 1 to 25 %), and in FP32 with a last radix other than 3
+     * (1 to 24 %); with radix 3, whose three butterflies per thread do not divide its 8 elements,
+     * FP32 256x384x768 takes 0.654 ms against 0.596 ms per step (FP64: 0.93 against 1.005) */
     const size_t ldsx = lds + cs * (size_t)(2 * A.P.M);
-    const bool x = exact && !plan_wide(&A.P) && g->nx % A.ti == 0 && (long long)nt * PERSIST_EPT == el && ldsx <= lds_limit()
+    const int rl = A.P.rad[A.P.nst - 1];
+    const int ntx = (int)(el / PERSIST_EPT);
+    const bool x = exact && !plan_wide(&A.P) && A.P.nst >= 2 && A.P.M % 2 == 0 && g->nx % A.ti == 0
+        && (!mixed || rl != 3) && ntx <= FFT_MAXTHREADS && ntx % 64 == 0 && (long long)ntx * PERSIST_EPT == el && ldsx <= lds_limit()
         && 16LL * g->plane < (1LL << 31) && 16LL * g->nx * A.nky < (1LL << 31);
-    /* FP32 tiles: only the exact form is persistent, with FFT_EPT / 2 elements per thread
-     * (twice the threads of the one-tile form), which keeps its registers below 128 */
-    const int ntf = (int)(el / PERSIST_EPT);
-    YInvArgs AF = A;
-    AF.P.nt = ntf;
-    const bool xf = exact && !plan_wide(&A.P) && g->nx % A.ti == 0 && ntf <= FFT_MAXTHREADS && ntf % 64 == 0
-        && ntf % A.ti == 0 && (long long)ntf * PERSIST_EPT == el && ldsx <= lds_limit()
-        && 16LL * g->plane < (1LL << 31) && 16LL * g->nx * A.nky < (1LL << 31);
-    const int r = mixed ? (xf ? launch_persistent(tck_yifft_psi_p<float, TCK_YIFFT_PF, PERSIST_EPT, false, true>, AF, ntf, ldsx, el, ntiles, stream) : 0)
-                : x ? launch_persistent(tck_yifft_psi_p<double, TCK_YIFFT_PF, PERSIST_EPT, false, true>, A, nt, ldsx, el, ntiles, stream)
-                    : (plan_wide(&A.P) ? launch_persistent(tck_yifft_psi_p<double, TCK_YIFFT_PF, PERSIST_EPT, true, false>, A, nt, lds, el, ntiles, stream)
-                                       : launch_persistent(tck_yifft_psi_p<double, TCK_YIFFT_PF, PERSIST_EPT, false, false>, A, nt, lds, el, ntiles, stream));
+    YInvArgs X = A;
+    X.P.nt = ntx;
+    #define YX(T) (rl == 8 ? launch_persistent(tck_yifft_psi_p<T, PERSIST_EPT, 8>, X, ntx, ldsx, el, ntiles, stream) \
+        : rl == 4 ? launch_persistent(tck_yifft_psi_p<T, PERSIST_EPT, 4>, X, ntx, ldsx, el, ntiles, stream) \
+                  : launch_persistent(tck_yifft_psi_p<T, PERSIST_EPT, 2>, X, ntx, ldsx, el, ntiles, stream))
+    const int r = !x ? 0 : mixed ? YX(float)
+        : rl == 3 ? launch_persistent(tck_yifft_psi_p<double, PERSIST_EPT, 3>, X, ntx, ldsx, el, ntiles, stream) : YX(double);
+    #undef YX
     if(r < 0) return (int)hipErrorInvalidValue;
     if(r > 0){ TCK_CHECK_LAUNCH(); return 0; }
   }
-#endif
   const dim3 grd((unsigned)ntiles);
   const bool half = (long long)nt * (FFT_EPT / 2) >= (long long)A.ti * A.P.M;
   if(half ? FFT_ONE_E(tck_yifft_psi, FFT_EPT / 2, mixed, plan_wide(&A.P)) : FFT_ONE_E(tck_yifft_psi, FFT_EPT, mixed, plan_wide(&A.P))) return (int)hipErrorInvalidValue;

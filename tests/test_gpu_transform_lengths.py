@@ -39,3 +39,28 @@ def test_potential_matches_oracle(need_gpu, nx, ny, nz):
         assert np.array_equal(full[..., 0], full[..., 1]) and np.array_equal(full[..., -1], full[..., -2])
         s.close()
     o.close()
+
+
+@pytest.mark.parametrize("nx,ny,nz", [(64, 128, 2048), (128, 192, 1024), (96, 1024, 192), (128, 512, 256), (128, 256, 512)])
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_persistent_forms_compute_the_same_bits(need_gpu, nx, ny, nz, precision):
+    """launches of enough tiles for the persistent axial (last radix 4, 2, 3, 4, 8) and inverse
+    theta (8, 3, 8, 4, 2) transforms: the same potential as the one-tile forms, bit for bit, each
+    repeated, with halo images and wall copies"""
+    small = make_case(nx=nx, ny=ny, nz=4, Re=100.0, amp=0.0, uy_walls=(0.0, 0.0))
+    rng = np.random.default_rng(5)
+    f = {"ux": rng.random((nz, ny, nx + 1)), "uy": rng.random((nz, ny, nx + 2)), "uz": rng.random((nz, ny, nx + 2))}
+    f["ux"][:, :, 0] = 0.0
+    f["ux"][:, :, -1] = 0.0
+    s = Solver(nx, ny, nz, small["xf"], small["xc"], precision=precision, **small["kw"])
+    s.load_fields(f)
+    want = None
+    for mask in (0, 1, 4, 5, 5):
+        s.tune("fft_exact", mask, 0)
+        s.potential(1, 0.13)
+        got = s.get_field_ref("psi")
+        if want is None:
+            want = got
+            assert np.abs(want).max() > 0.0
+        assert np.array_equal(got, want), mask
+    s.close()
