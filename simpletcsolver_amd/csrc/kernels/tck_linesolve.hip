@@ -1193,9 +1193,13 @@ struct PXSolveArgs {
   const double * pr; const double * pl; const double * pu;
 };
 
-/* one (ky, kz) line per wave per iteration, WPB waves per block looping over groups of WPB
- * lines; the spectrum row and its factor row are staged through LDS so that every global
- * access is contiguous across the wave (WPB keeps the staging area within 64 KB) */
+/* one (ky, kz) line per wave per iteration; the spectrum row and its factor row are staged
+ * through the wave's own part of LDS so that every global access is contiguous across the wave,
+ * and the next line's are loaded before the current one is solved; the waves of a block do not
+ * wait for each other.  Bound by HBM (40 B per value in FP64).  Against a form whose block loaded
+ * one line per wave at a time between barriers, ms per step (three launches): FP64 512x512x512
+ * 1.89 -> 1.52, 1000x256x256 1.62 -> 0.82, 128x192x256 0.116 -> 0.104; mixed 512x512x512
+ * 1.62 -> 0.95, 256x512x512 0.646 -> 0.543 */
 template <int SEG, int WPB, typename C2>
 __global__ void __launch_bounds__(WPB * TCK_WAVE) tck_pxsolve(const PXSolveArgs A){
   __shared__ double2 smq_all[WPB][TCK_WAVE * (SEG + 1)];
@@ -1212,24 +1216,36 @@ __global__ void __launch_bounds__(WPB * TCK_WAVE) tck_pxsolve(const PXSolveArgs 
     ll[e] = A.pl[row0 + e < n ? row0 + e : n - 1];
     uu[e] = A.pu[row0 + e < n ? row0 + e : n - 1];
   }
-  for(long long g0 = (long long)blockIdx.x * WPB; g0 < A.nlines; g0 += (long long)gridDim.x * WPB){
-    const long long line = g0 + w;
-    const bool live = line < A.nlines;
-    C2 * row = (C2 *)A.s + (live ? line : 0) * n;
-    const double * r = A.pr + (live ? line : 0) * n;
-    if(live){
-      #pragma unroll
-      for(int e = 0; e < SEG; e++){
-        const int idx = lane + e * TCK_WAVE;
-        if(idx < n){
-          const int p = stage_pos<SEG>(idx);
-          const C2 x = row[idx];
-          smq[p] = make_double2(double(x.x), double(x.y));
-          smr[p] = r[idx];
-        }
+  const long long step = (long long)gridDim.x * WPB;
+  long long line = (long long)blockIdx.x * WPB + w;
+  if(line >= A.nlines) return;
+  C2 nq[SEG];
+  double nr[SEG];
+  const auto fetch = [&](long long l){
+    const C2 * row = (const C2 *)A.s + l * n;
+    const double * r = A.pr + l * n;
+    #pragma unroll
+    for(int e = 0; e < SEG; e++){
+      const int idx = lane + e * TCK_WAVE;
+      nq[e] = row[idx < n ? idx : n - 1];
+      nr[e] = r[idx < n ? idx : n - 1];
+    }
+  };
+  fetch(line);
+  for(;;){
+    C2 * row = (C2 *)A.s + line * n;
+    #pragma unroll
+    for(int e = 0; e < SEG; e++){
+      const int idx = lane + e * TCK_WAVE;
+      if(idx < n){
+        const int p = stage_pos<SEG>(idx);
+        smq[p] = make_double2(double(nq[e].x), double(nq[e].y));
+        smr[p] = nr[e];
       }
     }
-    __syncthreads();
+    wave_sync();
+    const long long nxt = line + step;
+    fetch(nxt < A.nlines ? nxt : line);
     double q[SEG][2], rr[SEG], vv[SEG];
     #pragma unroll
     for(int e = 0; e < SEG; e++){
@@ -1239,24 +1255,26 @@ __global__ void __launch_bounds__(WPB * TCK_WAVE) tck_pxsolve(const PXSolveArgs 
       rr[e] = smr[lane * (SEG + 1) + e];
       /* v as the factor kernel forms it: u_0 / c_0 (r_0 holds c_0), r_i u_i, 0 at the end */
       const int row = row0 + e;
-      vv[e] = row == 0 ? uu[e] / rr[e] : (row == n - 1 ? 0. : rr[e] * uu[e]);
+      vv[e] = e == 0 && row == 0 ? uu[e] / rr[e] : (row == n - 1 ? 0. : rr[e] * uu[e]);
     }
     wave_tdm<SEG, 2>(q, rr, ll, vv, n);
     #pragma unroll
     for(int e = 0; e < SEG; e++) smq[lane * (SEG + 1) + e] = make_double2(q[e][0], q[e][1]);
-    __syncthreads();
-    if(live){
-      #pragma unroll
-      for(int e = 0; e < SEG; e++){
-        const int idx = lane + e * TCK_WAVE;
-        if(idx < n){
-          const double2 x = smq[stage_pos<SEG>(idx)];
-          row[idx].x = x.x;
-          row[idx].y = x.y;
-        }
+    wave_sync();
+    #pragma unroll
+    for(int e = 0; e < SEG; e++){
+      const int idx = lane + e * TCK_WAVE;
+      if(idx < n){
+        const double2 x = smq[stage_pos<SEG>(idx)];
+        C2 y;
+        y.x = x.x;
+        y.y = x.y;
+        row[idx] = y;
       }
     }
-    __syncthreads();
+    if(nxt >= A.nlines) return;
+    line = nxt;
+    wave_sync();
   }
 }
 
@@ -1292,7 +1310,10 @@ template <int SEG>
 static int launch_pxsolve_t(const PXSolveArgs & A, int mixed, hipStream_t stream){
   constexpr int WPB = SEG >= 16 ? 1 : 2;
   long long nblocks = ((long long)A.nlines + WPB - 1) / WPB;
-  const long long cap = (long long)num_cus() * 16 / WPB;
+  /* 24 waves per CU, more than are resident at most lengths, against 8, 12 and 16: 512x512x512
+   * mixed 0.953, 0.951, 1.039, 0.960 ms per step; 256x512x512 mixed 0.543, 0.622, 0.604, 0.561;
+   * 128x192x256 0.104, 0.120, 0.114, 0.110 */
+  const long long cap = (long long)num_cus() * 24 / WPB;
   if(nblocks > cap) nblocks = cap;
   if(mixed) hipLaunchKernelGGL((tck_pxsolve<SEG, WPB, float2>), dim3((unsigned)nblocks), dim3(WPB * TCK_WAVE), 0, stream, A);
   else hipLaunchKernelGGL((tck_pxsolve<SEG, WPB, double2>), dim3((unsigned)nblocks), dim3(WPB * TCK_WAVE), 0, stream, A);
