@@ -1289,12 +1289,23 @@ template <int SEG>
 static int launch_xsolve_t(const XSolveArgs & A, int nf, int mixed, hipStream_t stream){
   const long long nlines = (long long)A.g.ny * A.g.nz;
   const int wpb = TCK_BLOCK / TCK_WAVE;
-  long long nblocks = (nlines + wpb - 1) / wpb;
-  const long long cap = (long long)num_cus() * 8;
-  if(nblocks > cap) nblocks = cap;
-  const dim3 grd((unsigned)nblocks, (unsigned)nf);
   /* the final pass (the new fields written from the old ones) is a form of its own */
   const bool u = A.ucur[0] != NULL;
+  /* blocks per CU and field: 2 to 16, doubled while a wave keeps 4 lines and the rows per lane
+   * (lines times SEG) that repay what a block does before its lines.  The final pass, with more
+   * memory traffic per line, repays it with 16 rows, the others with 64; more than 8 blocks
+   * gained nothing there in FP32.  Against 8 blocks at every size, ms per step: 32x64x64 0.048 ->
+   * 0.043, 97x150x105 0.131 -> 0.113, mixed 150x140x180 0.220 -> 0.194, 1000x128x128 1.09 ->
+   * 0.99, 256x512x512 (final pass) 3.69 -> 3.58, 512x512x512 4.93 -> 4.87; 2 blocks at every size:
+   * 3.98 and 5.12 for the last two */
+  const long long lw = nlines / ((long long)wpb * num_cus());
+  const int rows = u ? 16 : 64, top = mixed && !u ? 8 : 16;
+  int bpc = 2;
+  while(bpc < top && lw / (2 * bpc) >= 4 && lw / (2 * bpc) * SEG >= rows) bpc *= 2;
+  long long nblocks = (nlines + wpb - 1) / wpb;
+  const long long cap = (long long)num_cus() * bpc;
+  if(nblocks > cap) nblocks = cap;
+  const dim3 grd((unsigned)nblocks, (unsigned)nf);
   if(mixed){
     if(u) hipLaunchKernelGGL((tck_xsolve<SEG, float, true>), grd, dim3(TCK_BLOCK), 0, stream, A);
     else hipLaunchKernelGGL((tck_xsolve<SEG, float, false>), grd, dim3(TCK_BLOCK), 0, stream, A);

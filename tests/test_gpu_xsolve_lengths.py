@@ -22,3 +22,18 @@ def test_x_solves_match_oracle(need_gpu, nx, implicit):
         assert rel_l2(sf[n], of[n]) <= 1e-14, n
     s.close()
     o.close()
+
+
+@pytest.mark.parametrize("implicit", [(1, 0, 0), (1, 1, 0)])
+@pytest.mark.parametrize("nx,ny,nz", [(3, 512, 512), (65, 128, 96), (150, 256, 70), (300, 128, 35)])
+def test_x_solves_of_many_lines_match_oracle(need_gpu, nx, ny, nz, implicit):
+    """several lines per wave, at launches of 2 to 16 blocks per CU; the same bound"""
+    case = make_case(nx=nx, ny=ny, nz=nz, implicit=implicit, t_amp=1e-2, Re=1e3)
+    o, s = oracle_for(case), gpu_for(case)
+    o.predict(0, 1e-3)
+    s.predict(0, 1e-3)
+    of, sf = o.npy_fields(), s.fields()
+    for n in ("ux", "uy", "uz", "t"):
+        assert rel_l2(sf[n], of[n]) <= 1e-14, n
+    s.close()
+    o.close()
