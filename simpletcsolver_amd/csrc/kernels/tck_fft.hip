@@ -822,6 +822,9 @@ __global__ void __launch_bounds__(FFT_MAXTHREADS) tck_yifft_psi_p(const YInvArgs
   /* pair u of this thread: line t0, k1 = 1 + r0 + u dr; last-pass butterfly q: index r0 + q dr */
   const int t0i = (int)threadIdx.x & (ti - 1), r0i = (int)threadIdx.x >> lg, dr = nt >> lg;
   const int perl = M / RL;
+  /* the thread row whose last-pass butterflies include the last one, perl - 1, whose last output
+   * is element M - 1 and with it row ny (dr - 1 only where RL divides EPTK) */
+  const int rlast = (perl - 1) % dr;
   int tile = blockIdx.x;               /* the launch has at least four tiles per block */
   /* buffer addressing: a tile's spectrum values lie in one plane of S (nky nx complex values) and
    * its psi values in one plane of the field, so each access is a per-thread byte offset that does
@@ -894,7 +897,7 @@ __global__ void __launch_bounds__(FFT_MAXTHREADS) tck_yifft_psi_p(const YInvArgs
       }
     }
     /* the halo images and wall copies of the threads that have any */
-    if(i == 1 || i == g.nx || k == 1 || k == g.nz || r0 == 0 || r0 == dr - 1){
+    if(i == 1 || i == g.nx || k == 1 || k == g.nz || r0 == 0 || r0 == rlast){
       T * col = psi + tck_idx(g, i, 0, k);
       const int wall = i == 1 ? -1 : (i == g.nx ? 1 : 0);
       const long long dk = k == 1 ? g.plane * g.nz : (k == g.nz ? - g.plane * g.nz : 0);
@@ -1214,9 +1217,11 @@ int tck_launch_yifft_psi(const tc_geom_t * g, const void * S, void * psi, const 
     /* the persistent form when the tiles cover the field exactly, the plan has two passes at least
      * and no radix 5 or 7, both twiddle tables fit in the LDS beside the tile and a plane's byte
      * offsets fit in 31 bits.  It is the faster one at every such FP64 size measured (128 to 1024
-     * rows, one to four blocks per CU: by 1 to 25 %), and in FP32 with a last radix other than 3
-     * (1 to 24 %); with radix 3, whose three butterflies per thread do not divide its 8 elements,
-     * FP32 256x384x768 takes 0.654 ms against 0.596 ms per step (FP64: 0.93 against 1.005) */
+     * rows, one to four blocks per CU: by 1 to 25 %; with a last radix of 3, one-tile against
+     * persistent, ms per step: 128x192x1024 0.333 and 0.332, 256x384x768 0.981 and 0.922,
+     * 512x768x768 4.98 and 4.19), and in FP32 with a last radix other than 3 (1 to 24 %); with radix
+     * 3, whose three butterflies per thread do not divide its 8 elements, FP32 256x384x768 takes
+     * 0.654 ms against 0.596 ms per step */
     const size_t ldsx = lds + cs * (size_t)(2 * A.P.M);
     const int rl = A.P.rad[A.P.nst - 1];
     const int ntx = (int)(el / PERSIST_EPT);
