@@ -154,11 +154,12 @@ __global__ void __launch_bounds__(CNN_TZ * TCK_WAVE) tck_cnn_conv(const ConvArgs
   };
   if(t0 < t1) fetch(t0);
   {
+    /* loaded without a condition: an element written only under one stays in scratch memory */
     uint4 wp[NW];
     #pragma unroll
     for(int q = 0; q < NW; q++){
       const int e = threadIdx.x + q * NTH;
-      if(e < 27 * CO * PC) wp[q] = *(const uint4 *)(A.w + 8LL * e);
+      wp[q] = *(const uint4 *)(A.w + 8LL * (e < 27 * CO * PC ? e : 0));
     }
     #pragma unroll
     for(int q = 0; q < NW; q++){
