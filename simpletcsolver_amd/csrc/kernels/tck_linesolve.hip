@@ -710,7 +710,11 @@ __device__ __forceinline__ int ps_seg(int m, int S){
  * past a segment's end) is decided for the wave, so that most groups run the lean form's
  * instructions; its rows are reached the same way, through a resource based at the group's
  * first row and bounded by the array's end (a lane's rows past its segment may lie past it:
- * they read as 0 and are not used).  The arithmetic of a row is the same in both. */
+ * they read as 0 and are not used).  The arithmetic of a row is the same in both.
+ * Registers bound the FP64 form (32 rows are 64 of its 128): what is needed only at the end (den)
+ * or can be formed again (row 0's quotient) is not held across the passes, so nothing is
+ * spilled; with 14 registers spilled it took, ms per step, y solves of 512x1024x1024 22.6 against
+ * 20.9, of 256x100x1000 1.13 against 1.00, z solves 31.9 against 30.5 and 1.67 against 1.56. */
 template <typename D, int MAXM, bool LEAN>
 __device__ __forceinline__ void psolve_body(const PSolveArgs & A, D * __restrict__ d, double * uout,
     const double * __restrict__ ucur, const double * __restrict__ rt, const double * __restrict__ vt,
@@ -742,7 +746,6 @@ __device__ __forceinline__ void psolve_body(const PSolveArgs & A, D * __restrict
   const double * r = rt + col;
   const double * v = vt + col;
   typedef D Q;   /* arithmetic type: the increment's own */
-  const Q den = Q(meta[col]);
   const Q tl = Q(meta[ts + col]);
   const Q tu = Q(meta[2 * ts + col]);
   const int jc = (int)meta[3 * ts + col];
@@ -798,7 +801,7 @@ __device__ __forceinline__ void psolve_body(const PSolveArgs & A, D * __restrict
   if(valid && sg == S - 1) smX[2 * TI + ti] = Q(d[base + step * m]);
   Q t[PS_PRE];
   /* forward: q0 = q0 / c0, q_i = r_i (q_i - l q_{i-1}) */
-  Q a = Q(1.), b = Q(0.), q0d = Q(0.);   /* q0d: row 0's result */
+  Q a = Q(1.), b = Q(0.);
   if constexpr(LEAN){
     /* rows from jc on: the factors are the constants */
     #pragma unroll
@@ -813,7 +816,7 @@ __device__ __forceinline__ void psolve_body(const PSolveArgs & A, D * __restrict
     for(int e0 = 0; e0 < MAXM; e0 += PS_PRE){
       if(e0 < cu){
         PS_ROWS(t, r, e0, rc, rlast);
-        if(e0 == 0 && row0 == 0) q0d = q[0] / t[0];
+        const Q q0d = e0 == 0 && row0 == 0 ? q[0] / t[0] : Q(0.);   /* row 0's result */
         #define PS_STEP(e) { \
           const Q ai = - t[e] * tl; \
           b = ai * b + t[e] * q[e0 + e]; \
@@ -859,6 +862,7 @@ __device__ __forceinline__ void psolve_body(const PSolveArgs & A, D * __restrict
     for(int e0 = 0; e0 < MAXM; e0 += PS_PRE){
       if(e0 < cu){
         PS_ROWS(t, r, e0, rc, rlast);
+        const Q q0d = e0 == 0 && row0 == 0 ? q[0] / t[0] : Q(0.);
         #define PS_STEP(e) { \
           q[e0 + e] = t[e] * (q[e0 + e] - tl * in); \
           if(e0 + e == 0 && row0 == 0) q[0] = q0d; \
@@ -949,6 +953,7 @@ __device__ __forceinline__ void psolve_body(const PSolveArgs & A, D * __restrict
       }
     }
   }
+  const Q den = Q(meta[col]);   /* read here: held from the start it would be spilled */
   if(cnt > 0 && row0 == 0) smX[ti] = q[0];
   __syncthreads();
   /* x_{n-1} (tdm.c:92-94) and x_i += x_{n-1} q1_i (:96-98) */
@@ -1074,7 +1079,6 @@ __device__ __forceinline__ void psolve_body(const PSolveArgs & A, D * __restrict
           const Q x = q[e0 + e] + xl * qq[e];
           q[e0 + e] = ucur ? Q(uu[e] + double(x)) : x;
         }
-        if(e0 == 0) img0 = double(q[0]);
       }else{
         double y[PS_PRE];
         #pragma unroll
@@ -1092,6 +1096,7 @@ __device__ __forceinline__ void psolve_body(const PSolveArgs & A, D * __restrict
     for(int e0 = 0; e0 < MAXM; e0 += PS_PRE) if(e0 < cu) PS_OUT(e0, double(q[e0 + e]))
   }
   if(ucur && row0 == 0 && cnt > 0){
+    if constexpr(sizeof(Q) == 8) img0 = double(q[0]);
     uout[base + step * n] = img0;
     if(dimg != 0) uout[base + step * n + dimg] = img0;
   }
