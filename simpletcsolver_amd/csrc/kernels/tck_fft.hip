@@ -1027,11 +1027,17 @@ static int fft_ld(int M){
 }
 
 /* the tile width b is a power of two (16 halved or doubled, capped at a power of two): the
- * kernels divide by it with shifts */
-static int fft_tile(int M, int cap, size_t csize, int * threads, int share, long long lines){
+ * kernels divide by it with shifts.  most: elements of a tile at most.  FFT_MOST is what a block
+ * takes at all; the FP64 axial transforms keep to half of it, eight elements per thread: with
+ * 16, which only tiles of 513 to 568, 1025 to 1137 and 2049 to 2275 rows would have, their first and
+ * last passes spill, and narrower tiles are the quicker ones, ms per step of both directions (16
+ * elements, 8): 128x256x540 0.948 / 0.690, 64x1120x560 1.83 / 1.29, 128x256x1080 2.01 / 1.78.
+ * The theta transforms are not: 128x1080x256 divergence + theta 1.27 / 1.37, inverse 0.83 / 0.89 */
+#define FFT_MOST (FFT_EPT * FFT_MAXTHREADS)
+static int fft_tile(int M, int cap, size_t csize, int * threads, int share, long long lines, int most){
   int b = 16;
   const size_t lb = (size_t)fft_ld(M) * csize;
-  while(b > 1 && ((size_t)b * lb > lds_limit() || b * M > FFT_EPT * FFT_MAXTHREADS)) b /= 2;
+  while(b > 1 && ((size_t)b * lb > lds_limit() || b * M > most)) b /= 2;
   while(share > 1 && b > 4 && (size_t)b * lb * share > lds_limit()) b /= 2;
   while(b * 2 <= cap && b * 2 * M <= FFT_EPT * 64) b *= 2;   /* short transforms: wider tiles */
   while(b > 1 && b * M > 128 && lines / b < 2LL * fft_ncu()) b /= 2;
@@ -1119,12 +1125,12 @@ static int launch_persistent(void (*kern)(const Args), const Args & A, int nt, s
 extern "C" {
 
 /* the one-tile form of kernel K, compiled for E elements per thread per pass, for the transform
- * type (float when mixed) and radix set; nonzero when the LDS limit could not be raised */
-#define FFT_ONE_E(K, E, mixed, wide) ( \
-  (mixed) ? ((wide) ? fft_one((const void *)K<float, E, true>, [&]{ hipLaunchKernelGGL((K<float, E, true>), grd, dim3(nt), lds, stream, A); }, lds) \
-                    : fft_one((const void *)K<float, E, false>, [&]{ hipLaunchKernelGGL((K<float, E, false>), grd, dim3(nt), lds, stream, A); }, lds)) \
-          : ((wide) ? fft_one((const void *)K<double, E, true>, [&]{ hipLaunchKernelGGL((K<double, E, true>), grd, dim3(nt), lds, stream, A); }, lds) \
-                    : fft_one((const void *)K<double, E, false>, [&]{ hipLaunchKernelGGL((K<double, E, false>), grd, dim3(nt), lds, stream, A); }, lds)))
+ * type T (E: float when mixed, else double) and radix set; nonzero when the LDS limit could not be
+ * raised */
+#define FFT_ONE_T(K, T, E, wide) ( \
+  (wide) ? fft_one((const void *)K<T, E, true>, [&]{ hipLaunchKernelGGL((K<T, E, true>), grd, dim3(nt), lds, stream, A); }, lds) \
+         : fft_one((const void *)K<T, E, false>, [&]{ hipLaunchKernelGGL((K<T, E, false>), grd, dim3(nt), lds, stream, A); }, lds))
+#define FFT_ONE_E(K, E, mixed, wide) ((mixed) ? FFT_ONE_T(K, float, E, wide) : FFT_ONE_T(K, double, E, wide))
 
 /* mixed: spectrum, transforms and psi in FP32 (twiddles twM, twN, tw as float2) */
 int tck_launch_div_yfft(const tc_geom_t * g, const tc_coef_t * c, const double * ux,
@@ -1136,7 +1142,7 @@ int tck_launch_div_yfft(const tc_geom_t * g, const tc_coef_t * c, const double *
   if(make_plan(g->ny / 2, &A.P) != 0) return (int)hipErrorInvalidValue;
   const size_t cs = mixed ? sizeof(float2) : sizeof(double2);
   int nt;
-  A.ti = fft_tile(A.P.M, 64, cs, &nt, TCK_FFT_YSHARE, (long long)g->nx * g->nz);
+  A.ti = fft_tile(A.P.M, 64, cs, &nt, TCK_FFT_YSHARE, (long long)g->nx * g->nz, FFT_MOST);
   A.P.nt = nt;
   A.twM = twM; A.twN = twN;
   A.ld = fft_ld(A.P.M);
@@ -1168,7 +1174,7 @@ int tck_launch_zfft(int nx, int nky, int nz, void * S, const void * tw, int sign
   if(make_plan(nz, &A.P) != 0) return (int)hipErrorInvalidValue;
   const size_t cs = mixed ? sizeof(float2) : sizeof(double2);
   int nt;
-  A.tz = fft_tile(nz, 64, cs, &nt, TCK_FFT_ZSHARE, (long long)nx * nky);
+  A.tz = fft_tile(nz, 64, cs, &nt, TCK_FFT_ZSHARE, (long long)nx * nky, mixed ? FFT_MOST : FFT_MOST / 2);
   A.P.nt = nt;
   A.ld = fft_ld(nz);
   const size_t lds = cs * (size_t)A.tz * A.ld;
@@ -1193,8 +1199,11 @@ int tck_launch_zfft(int nx, int nky, int nz, void * S, const void * tw, int sign
     if(r > 0){ TCK_CHECK_LAUNCH(); return 0; }
   }
   const dim3 grd((unsigned)ntiles);
-  const bool half = (long long)nt * (FFT_EPT / 2) >= (long long)A.tz * nz;
-  if(half ? FFT_ONE_E(tck_zfft, FFT_EPT / 2, mixed, plan_wide(&A.P)) : FFT_ONE_E(tck_zfft, FFT_EPT, mixed, plan_wide(&A.P))) return (int)hipErrorInvalidValue;
+  const bool wide = plan_wide(&A.P);
+  /* FP64 tiles always have FFT_EPT / 2 elements per thread (fft_tile) */
+  const bool half = !mixed || (long long)nt * (FFT_EPT / 2) >= (long long)A.tz * nz;
+  if((long long)nt * (half ? FFT_EPT / 2 : FFT_EPT) < (long long)A.tz * nz) return (int)hipErrorInvalidValue;
+  if(half ? FFT_ONE_E(tck_zfft, FFT_EPT / 2, mixed, wide) : FFT_ONE_T(tck_zfft, float, FFT_EPT, wide)) return (int)hipErrorInvalidValue;
   TCK_CHECK_LAUNCH();
   return 0;
 }
@@ -1206,7 +1215,7 @@ int tck_launch_yifft_psi(const tc_geom_t * g, const void * S, void * psi, const 
   if(make_plan(g->ny / 2, &A.P) != 0) return (int)hipErrorInvalidValue;
   const size_t cs = mixed ? sizeof(float2) : sizeof(double2);
   int nt;
-  A.ti = fft_tile(A.P.M, 64, cs, &nt, TCK_FFT_YSHARE, (long long)g->nx * g->nz);
+  A.ti = fft_tile(A.P.M, 64, cs, &nt, TCK_FFT_YSHARE, (long long)g->nx * g->nz, FFT_MOST);
   A.P.nt = nt;
   A.twM = twM; A.twN = twN;
   A.ld = fft_ld(A.P.M);
