@@ -124,9 +124,9 @@ int tc_stat_get(tc_solver_t * s, const char * name, double * host, size_t * num)
  * read LDS four segments at a time; 3, the default: both) the forms of the periodic solves.
  * Results are identical for every shape and form; only the speed changes */
 int tc_tune_set(tc_solver_t * s, const char * kernel, int kb, int ty);
-/* no reference counterpart: times the predictor for every candidate shape (kb in 2..32,
- * ty in 1, 2, 4) on the solver's own buffers, reps launches each, and keeps the fastest for
- * the predictor and the correction.  Only the next-field and RK buffers are written, which
+/* no reference counterpart: times the predictor for its shape in force and every candidate (kb in
+ * 2..32, ty in 1, 2, 4) on the solver's own buffers, reps launches each, and keeps the fastest;
+ * the correction keeps its shape.  Only the next-field and RK buffers are written, which
  * the next step overwrites, so the flow itself is unchanged. */
 int tc_autotune(tc_solver_t * s, int reps, int * kb, int * ty, double * best_ms);
 
