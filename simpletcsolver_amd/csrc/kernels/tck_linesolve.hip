@@ -1430,9 +1430,12 @@ int tck_launch_psolve(const tc_geom_t * g, int dir, int nf, void * const * d, do
   const long long seg = mixed ? (m + S - 1) / S : maxm;
   const long long wspan = ((long long)(64 / TI + 2) * seg + maxm) * step + 64;
   const long long tspan = ((long long)(tcol ? tstride : 1) * (m + 1) + g->px) * 8;
-  /* the other form's: from the first lane's row of a group to the last lane's (grids past this
-   * would not fit in memory) */
-  if(((63 / TI) * seg + PS_PRE) * step * 8 >= (1LL << 32) || tspan >= (1LL << 32)) return (int)hipErrorInvalidValue;
+  /* the other form's: from the first lane's row of a group to the last lane's.  Waves start at lanes
+   * 64 w, whose columns 64 w mod TI are at most TI - gcd(64, TI), so that the last lane is that many
+   * and 63 columns on (grids past this would not fit in memory) */
+  const int gcd = TI & -TI & 63 ? TI & -TI : 64;
+  const long long gspan = (TI - gcd + 63) / TI;
+  if((gspan * seg + PS_PRE) * step * 8 >= (1LL << 32) || tspan >= (1LL << 32)) return (int)hipErrorInvalidValue;
   A.lean = (lean & 2) | ((lean & 1) && wspan * 8 < (1LL << 31) && tspan < (1LL << 31) ? 1 : 0);
   if(mixed) hipLaunchKernelGGL((tck_psolve<float, 2 * PS_MAXM>), grd, dim3(TI, S), lds, stream, A);
   else hipLaunchKernelGGL((tck_psolve<double, PS_MAXM>), grd, dim3(TI, S), lds, stream, A);
