@@ -116,10 +116,9 @@ int tc_stat_get(tc_solver_t * s, const char * name, double * host, size_t * num)
  * marched per block (1..nz) and ty j rows per block of 64 x ty threads (1, 2 or 4).  Kernel
  * "predict_window" with kb 1 or 0 switches the predictor's form that stages the fields'
  * planes in LDS (32 x 8 tiles, taken when ty is 4; the default) on or off; "fft_exact" with
- * kb a mask (1: the axial transforms, 4: the inverse theta transform: their exact-tiling
- * forms where the tiles cover the spectrum exactly; 2: the divergence + theta transform's
- * twiddle tables in LDS; 7, the default: all three) the forms of the persistent FP64
- * transforms; "psolve_lean" with kb a mask (1: the periodic y and z solves' waves of interior
+ * kb a mask (1: the axial transforms, 4: the inverse theta transform; 5, the default: both; 2
+ * is accepted and has no effect, the divergence + theta transform has one form) their
+ * persistent forms, where they apply, or the one-tile ones; "psolve_lean" with kb a mask (1: the periodic y and z solves' waves of interior
  * full-length segments past the factors' convergence row skip the row tests; 2: their folds
  * read LDS four segments at a time; 3, the default: both) the forms of the periodic solves.
  * Results are identical for every shape and form; only the speed changes */

@@ -384,7 +384,7 @@ static void default_shapes(tc_solver_t * s){
     s->tune[TC_TUNE_CORRECT][1] = 4;
   }
   s->predict_window = 1;
-  s->fft_exact = 7;
+  s->fft_exact = 5;
   s->psolve_lean = 3;
 }
 

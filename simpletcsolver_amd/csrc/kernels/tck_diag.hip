@@ -78,8 +78,8 @@ struct DiagArgs {
   int scalar;
 };
 
-/* planes a block of 64 x 4 columns marches: 16, fewer while the grid has under eight blocks per
- * CU */
+/* planes a block of 64 x 4 columns marches: 16, fewer while the grid has under 2048 blocks,
+ * eight for each of the 256 CUs */
 static int diag_kb(const tc_geom_t * g){
   const long long cols = (long long)((g->nx + 1 + 63) / 64) * ((g->ny + 3) / 4);
   int kb = 16;

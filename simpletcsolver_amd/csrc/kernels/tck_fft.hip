@@ -24,8 +24,8 @@
  * ignored by the complex-to-real transform, as FFTW's c2r does with a Hermitian input.
  *
  * The in-LDS transform is a Stockham autosort FFT (Govindaraju et al., "High performance
- * discrete Fourier transforms on graphics processors", SC 2008) with radix 8, 4, 3 and 2
- * passes; each pass reads all its butterfly inputs into registers, synchronises, and
+ * discrete Fourier transforms on graphics processors", SC 2008) with radix 8, 7, 5, 4, 3
+ * and 2 passes; each pass reads all its butterfly inputs into registers, synchronises, and
  * writes in place.
  */
 #include "tck_common.h"
@@ -312,8 +312,7 @@ __device__ __forceinline__ void fft_first(typename cvec<T>::type * buf, int ld, 
   fft_pass_barrier();
 }
 
-/* passes st0 .. st1 - 1 in LDS */
-/* passes st0..st1 - 1 of nb transforms of length P.M stored at buf + b * ld; tw[t] =
+/* passes st0..st1 - 1, in LDS, of nb transforms of length P.M stored at buf + b * ld; tw[t] =
  * exp(-2 pi i t / M); each pass keeps at most EPT elements per thread in registers, so
  * P.nt * EPT >= nb * P.M.  W: the plan may hold radix 5 and 7 passes (compiled only into the
  * kernels of such lengths, so that the 2^a 3^b kernels keep their register budget) */
@@ -1044,9 +1043,9 @@ static int fft_tile(int M, int cap, size_t csize, int * threads, int share, long
   if(b > cap) b = cap < 1 ? 1 : cap;
   /* elements per thread: FFT_EPT, or half that where the LDS holds so few blocks per CU that
    * FFT_EPT would leave fewer than 16 waves on it (FP64 tiles of long transforms: one block
-   * per CU), and for every FP64 tile, whose 16 elements do not fit in a thread's registers
-   * beside a pass that loads or stores them.  The device passes loop over their butterflies, so any count up to FFT_EPT
-   * computes the same bits. */
+   * per CU), and for every FP64 tile that 1024 threads cover so, because 16 elements do not fit in
+   * a thread's registers beside a pass that loads or stores them.  The device passes loop over their
+   * butterflies, so any count up to FFT_EPT computes the same bits. */
   int ept = FFT_EPT;
   const long long per = (long long)(lds_limit() / ((size_t)b * lb));
   const int w16 = ((b * M + FFT_EPT - 1) / FFT_EPT + 63) / 64;
