@@ -59,11 +59,11 @@ struct CnnGrid { int nx, ny, nz, nb; long long nv; };
  * read 36 pieces from LDS instead of 72.  The taps are added in the order of their index
  * whatever the tile, so the result does not depend on the tiling.
  *
- * Measured on a million cells (64 x 128 x 128): 88 us for 32 -> 32 channels (660 TFLOP/s), 56
+ * Measured on a million cells (64 x 128 x 128): 86 us for 32 -> 32 channels (675 TFLOP/s), 58
  * us for 32 -> 16 and 63 us for 16 -> 32; reading each tap's operands from LDS again for every
  * row, with the halo images found by runtime division, took 149, 111 and 73 us.  LDS reads
- * and, on small grids, the staging bound it: 18, 11 and 14 us at 32 x 64 x 64, where each CU
- * has one tile (23, 18 and 14 us before).
+ * and, on small grids, the staging bound it: 16, 11 and 13 us at 32 x 64 x 64, where each CU
+ * has one tile (23, 18 and 14 us before; 18.5, 11.3 and 13.7 with the kernel's pieces in scratch).
  * ------------------------------------------------------------------------------------- */
 struct ConvArgs {
   CnnGrid G;
